@@ -149,6 +149,45 @@ int acquire_workspace(const credit_cfg* cfg, size_t bytes, char** base) {
   return workspace_cache().get(dev, cfg_stream(cfg), need, base);
 }
 
+// A query that fails (the null stream while another stream captures) counts
+// as capturing.
+bool stream_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) == hipSuccess)
+    return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+int acquire_workspace_with(const credit_cfg* cfg, size_t own, size_t extra, char** base,
+                           char** spare, size_t* spare_bytes) {
+  const size_t at = align_up(own, 256);
+  *spare = nullptr;
+  *spare_bytes = 0;
+  if (extra == 0) return acquire_workspace(cfg, own, base);
+  if (cfg != nullptr && cfg->workspace != nullptr) {
+    CREDIT_TRY(acquire_workspace(cfg, own, base));
+    if (cfg->workspace_bytes > kScratchOffset + at) {
+      *spare = ws_scratch(*base) + at;
+      *spare_bytes = cfg->workspace_bytes - (kScratchOffset + at);
+    }
+    return CREDIT_OK;
+  }
+  int dev = 0;
+  CREDIT_HIP(hipGetDevice(&dev));
+  hipStream_t stream = cfg_stream(cfg);
+  const size_t all = kScratchOffset + at + extra;
+  if (workspace_cache().capacity(dev, stream) < all && stream_capturing(stream))
+    return acquire_workspace(cfg, own, base);
+  if (workspace_cache().get(dev, stream, all, base) != CREDIT_OK) {
+    (void)hipGetLastError();
+    return acquire_workspace(cfg, own, base);
+  }
+  *spare = ws_scratch(*base) + at;
+  *spare_bytes = extra;
+  return CREDIT_OK;
+}
+
 __global__ void fill_f32_kernel(float* __restrict__ p, float v, int64_t n) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -386,7 +425,7 @@ size_t credit_workspace_bytes(int32_t op, int64_t rows, int64_t cols,
       body = layernorm_bwd_workspace(rows, cols, variant, split, 2, cus);
       break;
     case CREDIT_OP_FFN:  // cols = the FFN hidden width f
-      body = ffn_workspace(rows, cols);
+      body = ffn_workspace_advised(rows, cols);
       break;
     case CREDIT_OP_SOFTMAX_FWD:
     case CREDIT_OP_SOFTMAX_BWD:

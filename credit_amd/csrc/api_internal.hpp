@@ -128,6 +128,14 @@ inline size_t split_slot_bytes(int64_t groups, int members, int k_values, int ri
   return static_cast<size_t>(groups) * ring * k_values * members * sizeof(uint64_t);
 }
 int acquire_workspace(const credit_cfg* cfg, size_t bytes, char** base);
+// Whether `stream` is being captured into a graph (nothing can be allocated).
+bool stream_capturing(hipStream_t stream);
+// A workspace of `own` scratch bytes and, where they can be had, `extra` more
+// behind them (*spare, *spare_bytes) that the call can do without: the rest of
+// a caller's workspace, or the library's buffer unless it would have to grow
+// while the stream is being captured or does not fit the device.
+int acquire_workspace_with(const credit_cfg* cfg, size_t own, size_t extra, char** base,
+                           char** spare, size_t* spare_bytes);
 
 // Workspace of a ticketed split launch: the counter area, the partial slots
 // of `groups` groups (in the slot area), then `extra_bytes` of scratch for
@@ -211,6 +219,7 @@ int check_launch(const char* kernel);
 size_t row_sum_max_workspace(int64_t rows, int64_t cols, int variant, int split,
                              int cu_count);
 size_t ffn_workspace(int64_t rows, int64_t ffn_dim);
+size_t ffn_workspace_advised(int64_t rows, int64_t ffn_dim);
 size_t ffn_bwd_workspace(int64_t rows, int64_t d, int64_t ffn_dim);
 size_t layernorm_bwd_workspace(int64_t rows, int64_t cols, int variant, int split,
                                int elem_bytes, int cu_count);

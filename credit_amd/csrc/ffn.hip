@@ -1,14 +1,14 @@
 // C5: norm-fused FFN on MFMA, bf16 with fp32 accumulation.
 //
 //   rstd = 1/sqrt(mean_j x^2 + eps)                          (unit RMSNorm weight)
-//   h    = bf16(GELU_tanh(rstd * (x @ W1^T)))   256-tile kernel (the C5 path)
-//   h    = bf16(GELU_tanh(bf16(x * rstd) @ W1^T))   128-tile kernel
+//   h    = bf16(GELU_tanh(rstd * (x @ W1^T)))   shapes of 256-multiples (C5)
+//   h    = bf16(GELU_tanh(bf16(x * rstd) @ W1^T))   other shapes (big_shape)
 //   out  = bf16(x + h @ W2^T)
 //
-// The 256-tile kernel multiplies the fp32 accumulator of x @ W1^T by the
-// row's rstd in its epilogue (the row scale commutes with the GEMM), so the
-// normalised input is never rounded; the 128-tile kernel scales and rounds
-// the A tile to bf16 as it stages it.  Both are the same function up to that
+// On the first the fp32 accumulator of x @ W1^T is multiplied by the row's rstd
+// in the epilogue (the row scale commutes with the GEMM), so the normalised
+// input is never rounded; on the others the product reads a copy of x scaled
+// and rounded to bf16.  Both are the same function up to that
 // rounding (the oracle's round_a switch selects either).
 //
 // No FFN exists in the reference; this is the consumer of the row-norm
@@ -24,18 +24,21 @@
 //     RMSNorm commutes with the GEMM and is applied as a row scale.
 //  3. GEMM2 with epilogue kEpiResidual: out = bf16(acc + x).
 // Each GEMM runs on ffn_gemm256_kernel (256 x 256 x 64 tiles, four waves,
-// LDS-direct operand loads; the C5 path) when the shape allows, else on
-// ffn_gemm_kernel (128 x 128 x 64 tiles, operands prefetched through
-// registers one K-step ahead, the A tile scaled by rstd and rounded to bf16
-// while it is staged into LDS).  The backward (credit_ffn_rmsnorm_gelu_bwd_bf16)
-// runs five GEMMs on the same two kernels with its own epilogues.
+// LDS-direct operand loads; the C5 path) or on ffn_gemm_tile_kernel (128 or 256
+// x 128 x 64 tiles, K split over workgroups where the tiles leave CUs idle),
+// whichever gemm_plan's count says is done sooner.  The backward
+// (credit_ffn_rmsnorm_gelu_bwd_bf16) runs five GEMMs on the same two kernels
+// with its own epilogues.
+#include <algorithm>
 #include <atomic>
 #include <initializer_list>
+#include <mutex>
 #include <type_traits>
 #include <utility>
 
 #include "api_internal.hpp"
 #include "common.hpp"
+#include "workspace_cache.hpp"
 
 namespace credit {
 namespace {
@@ -43,11 +46,7 @@ namespace {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kBM = 128;
-constexpr int kBN = 128;
-constexpr int kBK = 64;
-constexpr int kThreads = 256;
-constexpr int kLdsStride = kBK + 8;  // bf16 per LDS row: 16-byte pad against bank conflicts
+constexpr int kFfnMultiple = 128;  // rows, d and f
 
 // GEMM epilogues.  Forward: kEpiGelu (h = GELU(acc * rstd[m])),
 // kEpiResidual (out = acc + x); the training forward's kEpiGeluSave (h =
@@ -64,6 +63,7 @@ constexpr int kEpiStore = 4;
 constexpr int kEpiStoreF32 = 5;
 constexpr int kEpiGeluSave = 6;
 constexpr int kEpiStoreT = 7;  // C^T [N, M] = bf16(acc): the output stored transposed
+constexpr int kEpiPartial = 8;  // Cf[slice] = acc as fp32: a K slice's partial sums
 
 // GELU with the tanh approximation, z = sqrt(2/pi) (v + 0.044715 v^3):
 // 0.5 (1 + tanh z) = sigmoid(2z), so GELU(v) = v / (1 + e') with
@@ -108,56 +108,53 @@ __device__ __forceinline__ float gelu_tanh_grad(float v) {
                         g.s);
 }
 
-// One output element of every epilogue.  s is the row scale still to apply
-// (rstd[m] for the 256-tile kernel, 1 where the A tile was scaled on load);
-// rv is R[m, n] widened to fp32 for kEpiResidual and kEpiGeluBwd (unused
-// otherwise).
+// The output values of one element of every epilogue: c goes to C (kEpiStoreF32:
+// Cf) and c2 to C2, row-major or transposed as the epilogue says.  s is the
+// row scale rstd[m], rv is R[m, n] widened to fp32.
+struct EpiValue {
+  float c, c2;
+};
 template <int EPI>
-__device__ __forceinline__ void epilogue(float acc, float s, float rv, int m, int n, int M, int N,
-                                         uint16_t* __restrict__ C, uint16_t* __restrict__ C2,
-                                         float* __restrict__ Cf) {
-  const size_t idx = static_cast<size_t>(m) * N + n;
-  const size_t tdx = static_cast<size_t>(n) * M + m;
-  if (EPI == kEpiGelu) {
-    C[idx] = f32_to_bf16(gelu_tanh(acc * s));
-  } else if (EPI == kEpiGeluSave) {
+__device__ __forceinline__ EpiValue epilogue_value(float acc, float s, float rv) {
+  if constexpr (EPI == kEpiGelu) {
+    return {gelu_tanh(acc * s), 0.0f};
+  } else if constexpr (EPI == kEpiGeluSave) {
     // The same h as kEpiGelu, and the u the backward's kEpiUH recomputes.
     const float u = acc * s;
-    C[idx] = f32_to_bf16(gelu_tanh(u));
-    C2[idx] = f32_to_bf16(u);
-  } else if (EPI == kEpiResidual) {
-    C[idx] = f32_to_bf16(acc + rv);
-  } else if (EPI == kEpiUH) {
+    return {gelu_tanh(u), u};
+  } else if constexpr (EPI == kEpiResidual) {
+    return {acc + rv, 0.0f};
+  } else if constexpr (EPI == kEpiUH) {
     const float u = acc * s;
-    C[idx] = f32_to_bf16(u);
-    C2[tdx] = f32_to_bf16(gelu_tanh(u));
-  } else if (EPI == kEpiGeluBwd) {
-    const uint16_t v = f32_to_bf16(acc * gelu_tanh_grad(rv));
-    C[idx] = v;
-    if (C2 != nullptr) C2[tdx] = v;
-  } else if (EPI == kEpiStoreT) {
-    C[tdx] = f32_to_bf16(acc);
-  } else if (EPI == kEpiStore) {
-    C[idx] = f32_to_bf16(acc);
+    return {u, gelu_tanh(u)};
+  } else if constexpr (EPI == kEpiGeluBwd) {
+    const float v = acc * gelu_tanh_grad(rv);
+    return {v, v};
   } else {
-    Cf[idx] = acc;
+    return {acc, 0.0f};
   }
 }
 
 // Epilogues that read a second [M, N] operand.
 template <int EPI>
 constexpr bool kEpiReadsR = EPI == kEpiResidual || EPI == kEpiGeluBwd;
+// Epilogues that scale row m by scale[m].
+template <int EPI>
+constexpr bool kEpiScaled = EPI == kEpiGelu || EPI == kEpiGeluSave || EPI == kEpiUH;
 
-__device__ __forceinline__ u32x4 scale_bf16x8(u32x4 v, float s) {
-  return u32x4{pack_bf16x2(bf16_lo(v.x) * s, bf16_hi(v.x) * s),
-               pack_bf16x2(bf16_lo(v.y) * s, bf16_hi(v.y) * s),
-               pack_bf16x2(bf16_lo(v.z) * s, bf16_hi(v.z) * s),
-               pack_bf16x2(bf16_lo(v.w) * s, bf16_hi(v.w) * s)};
+__device__ __forceinline__ bf16x8_t scale_bf16x8(bf16x8_t x, float s) {
+  const u32x4 v = __builtin_bit_cast(u32x4, x);
+  return __builtin_bit_cast(bf16x8_t, u32x4{pack_bf16x2(bf16_lo(v.x) * s, bf16_hi(v.x) * s),
+                                            pack_bf16x2(bf16_lo(v.y) * s, bf16_hi(v.y) * s),
+                                            pack_bf16x2(bf16_lo(v.z) * s, bf16_hi(v.z) * s),
+                                            pack_bf16x2(bf16_lo(v.w) * s, bf16_hi(v.w) * s)});
 }
 
 // rstd[m] = 1/sqrt(mean(x[m]^2) + eps); cols % 8 == 0, rows 16-byte aligned.
+// With a != nullptr also a = bf16(x * rstd), the row re-read from L2.
 __global__ __launch_bounds__(256) void ffn_rstd_kernel(const uint16_t* __restrict__ x,
-                                                       float* __restrict__ rstd, int cols,
+                                                       float* __restrict__ rstd,
+                                                       uint16_t* __restrict__ a, int cols,
                                                        float eps) {
   __shared__ double red[4];
   const u32x4* xr = reinterpret_cast<const u32x4*>(x + static_cast<size_t>(blockIdx.x) * cols);
@@ -172,134 +169,12 @@ __global__ __launch_bounds__(256) void ffn_rstd_kernel(const uint16_t* __restric
     }
   }
   const double t = block_reduce_sum_f64<4>(static_cast<double>(s), red);
-  if (threadIdx.x == 0) rstd[blockIdx.x] = static_cast<float>(1.0 / __builtin_sqrt(t / cols + eps));
-}
-
-// C[m, n] = epi(sum_k A[m, k] * B[n, k]).  A [M, K] and B [N, K] row-major
-// bf16 (KN: B [K, N], element (n, k) at B[k * N + n]); M % 128 == 0,
-// N % 128 == 0, K % 64 == 0 (checked on the host).
-//  kEpiGelu:     A rows scaled by a_scale[m] on load; C = bf16(gelu(acc)).
-//  kEpiGeluSave: likewise, and C2 = bf16(acc) (u).
-//  kEpiResidual: C = bf16(acc + R[m, n]).
-// KN: thread t stages 16-byte chunk t % 16 (8 columns) of K-rows t / 16 +
-// 16 i of the 64 x 128 B tile and scatters its 8 values into the [n][k]
-// LDS tile (2-byte stores; this kernel only serves shapes the 256-tile
-// kernel does not take).
-template <int EPI, bool KN>
-__global__ __launch_bounds__(kThreads) void ffn_gemm_kernel(
-    const uint16_t* __restrict__ A, const float* __restrict__ a_scale,
-    const uint16_t* __restrict__ B, const uint16_t* __restrict__ R, uint16_t* __restrict__ C,
-    uint16_t* __restrict__ C2, float* __restrict__ Cf, int M, int N, int K) {
-  constexpr bool kScaleA = EPI == kEpiGelu || EPI == kEpiUH || EPI == kEpiGeluSave;
-  __shared__ __attribute__((aligned(16))) uint16_t As[kBM * kLdsStride];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[kBN * kLdsStride];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  // Tile order: consecutive workgroups walk down M for a fixed N strip, so
-  // the B strip (the weight tile) is reused from L2 by neighbours.
-  const int tiles_m = M / kBM;
-  const int tm = blockIdx.x % tiles_m;
-  const int tn = blockIdx.x / tiles_m;
-  const int m0 = tm * kBM, n0 = tn * kBN;
-
-  // Global -> register staging: thread t moves rows t/8 + 32*i, 16-byte
-  // chunk t%8 of the 128-byte K-row, for i = 0..3 (A and B alike).
-  const int ld_row = tid >> 3;
-  const int ld_chunk = tid & 7;
-  const u32x4* a_src[4];
-  const u32x4* b_src[4];
-  float scale[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = ld_row + 32 * i;
-    a_src[i] = reinterpret_cast<const u32x4*>(A + static_cast<size_t>(m0 + r) * K) + ld_chunk;
-    b_src[i] = KN ? reinterpret_cast<const u32x4*>(B + static_cast<size_t>((tid >> 4) + 16 * i) * N +
-                                                   n0) + (tid & 15)
-                  : reinterpret_cast<const u32x4*>(B + static_cast<size_t>(n0 + r) * K) + ld_chunk;
-    scale[i] = kScaleA ? a_scale[m0 + r] : 1.0f;
-  }
-  const size_t b_step = KN ? static_cast<size_t>(kBK) * N / 8 : kBK / 8;  // u32x4 per K-step
-  u32x4 ra[4], rb[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    ra[i] = a_src[i][0];
-    rb[i] = b_src[i][0];
-  }
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-  const int ksteps = K / kBK;
-  for (int ks = 0; ks < ksteps; ++ks) {
-    __syncthreads();  // previous step's fragment reads are done
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = ld_row + 32 * i;
-      const u32x4 av = kScaleA ? scale_bf16x8(ra[i], scale[i]) : ra[i];
-      *reinterpret_cast<u32x4*>(&As[r * kLdsStride + ld_chunk * 8]) = av;
-      if constexpr (KN) {
-        const int kr = (tid >> 4) + 16 * i, n8 = (tid & 15) * 8;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          Bs[(n8 + 2 * e) * kLdsStride + kr] = static_cast<uint16_t>(rb[i][e] & 0xffffu);
-          Bs[(n8 + 2 * e + 1) * kLdsStride + kr] = static_cast<uint16_t>(rb[i][e] >> 16);
-        }
-      } else {
-        *reinterpret_cast<u32x4*>(&Bs[r * kLdsStride + ld_chunk * 8]) = rb[i];
-      }
-    }
-    __syncthreads();
-    if (ks + 1 < ksteps) {  // prefetch the next K-step into registers
-      const int off = (ks + 1) * (kBK / 8);
-      const size_t boff = (ks + 1) * b_step;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        ra[i] = a_src[i][off];
-        rb[i] = b_src[i][boff];
-      }
-    }
-#pragma unroll
-    for (int kk = 0; kk < kBK / 16; ++kk) {
-      const int kcol = kk * 16 + (lane >> 5) * 8;
-      bf16x8_t af[2], bfr[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int r = wm * 64 + i * 32 + (lane & 31);
-        af[i] = *reinterpret_cast<const bf16x8_t*>(&As[r * kLdsStride + kcol]);
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int c = wn * 64 + j * 32 + (lane & 31);
-        bfr[j] = *reinterpret_cast<const bf16x8_t*>(&Bs[c * kLdsStride + kcol]);
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-    }
-  }
-
-  // Epilogue.  Accumulator register r of lane l holds row
-  // 8*(r/4) + 4*(l/32) + r%4 and column l%32 of the 32 x 32 tile.
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int n = n0 + wn * 64 + j * 32 + (lane & 31);
-        const float rv = kEpiReadsR<EPI> ? bf16_to_f32(R[static_cast<size_t>(m) * N + n]) : 0.0f;
-        epilogue<EPI>(acc[i][j][r], 1.0f, rv, m, n, M, N, C, C2, Cf);
-      }
+  const float rs = static_cast<float>(1.0 / __builtin_sqrt(t / cols + eps));
+  if (threadIdx.x == 0) rstd[blockIdx.x] = rs;
+  if (a == nullptr) return;
+  u32x4* ar = reinterpret_cast<u32x4*>(a + static_cast<size_t>(blockIdx.x) * cols);
+  for (int i = threadIdx.x; i < nvec; i += 256)
+    ar[i] = __builtin_bit_cast(u32x4, scale_bf16x8(__builtin_bit_cast(bf16x8_t, xr[i]), rs));
 }
 
 // ----------------------------------------------------- 256 x 256 tiles ---
@@ -393,6 +268,18 @@ __device__ __forceinline__ void load_to_lds(buffer_rsrc_t rsrc, uint32_t voff, u
       "s_add_u32 m0, %2, %3\n\t"
       "s_nop 0\n\t"
       "buffer_load_dwordx4 %0, %1, %4 offen lds"
+      :
+      : "v"(voff), "s"(rsrc), "s"(m0base), "i"(QOFF), "s"(soff)
+      : "memory", "m0", "scc");
+}
+// The same with the nontemporal hint.
+template <uint32_t QOFF>
+__device__ __forceinline__ void load_to_lds_nt(buffer_rsrc_t rsrc, uint32_t voff, uint32_t m0base,
+                                               uint32_t soff) {
+  asm volatile(
+      "s_add_u32 m0, %2, %3\n\t"
+      "s_nop 0\n\t"
+      "buffer_load_dwordx4 %0, %1, %4 offen nt lds"
       :
       : "v"(voff), "s"(rsrc), "s"(m0base), "i"(QOFF), "s"(soff)
       : "memory", "m0", "scc");
@@ -761,6 +648,351 @@ __global__ __launch_bounds__(kBigThreads) void ffn_gemm256_kernel(
   clock_probe_add(probe, false);
 }
 
+// ------------------------------------------------- BM x 128 tiles, split K --
+// The GEMM of every shape the 256-tile kernel does not fill the chip with:
+// BM x 128 x 64 tiles (BM 128 or 256) of four waves in a 2 x 2 grid, wave
+// (wm, wn) owning a BM/2 x 64 block as BM/64 x 2 v_mfma_f32_32x32x16_bf16
+// tiles, and K cut into `slices` pieces whose fp32 sums are added in slice
+// order.
+//  - One operand ring for A and B: ST stages of (BM + 128) rows x 64 K, filled by the LDS-direct loads of the 256-tile kernel (the same row
+//    swizzle; KN: the stage's B part is 64 K-rows of 256 bytes, chunk c of
+//    K-row r at position c ^ 4 (r & 3)).
+//  - K-step k reads stage k % ST.  Iteration it runs four sub-steps of k = 16,
+//    each reading the next one's fragments while its MFMAs issue.  Before the
+//    last sub-step: own loads of step it+1 landed (vmcnt leaves the ST - 2
+//    steps behind it in flight), then an LDS-only barrier, after which stage
+//    it % ST is free: step it+ST's loads go there, a quarter of them in each
+//    of that sub-step and the next iteration's first three (two stages: all in
+//    that sub-step).  Tail steps
+//    re-load the last K-step into stages nobody reads again.
+//  - With few tiles a CU would sit idle or run one long K chain (128 rows x
+//    8192 x 28672: 64 tiles on 256 CUs), so gemm_plan cuts K until the units
+//    (tiles x slices) fill the chip.  kEpiPartial launches one workgroup per
+//    unit, which stores its sums to Cf[slice] for ffn_reduce_kernel; every
+//    other EPI covers all slices of its tile in order with the same additions,
+//    so both forms give the same bits.
+//  - B loads carry the nontemporal hint, which leaves the L2 to the A rows
+//    that every workgroup of an XCD reads (128 rows x 8192 x 28672: 206 ->
+//    196 us; no shape measured slower).
+//  - skew: tile column t starts each slice at its (skew t)-th step and wraps
+//    around.  A K pitch of a power of two puts the same K-step of every weight
+//    row on one channel, and tiles of one wave march in step; apart by one
+//    128-byte step each they spread over all channels (230 -> 206 us there).
+//    Only where one M-tile covers all rows (weights read once): a product's
+//    order of additions must not depend on which side is called M.
+//  - RA: the A rows are scaled by scale[m] and rounded to bf16 as their
+//    fragments are used.  Twice as slow as reading an A that
+//    ffn_rstd_kernel scaled (176 against 87 us for 128 x 28672 x 8192), so it
+//    serves calls with no room for that copy.
+constexpr int kTileN = 128;
+template <int BM>
+constexpr int kTileStageBytes = (BM + kTileN) * kBigK * 2;
+
+template <int EPI, bool KN, int BM, int ST, bool RA>
+__global__ __launch_bounds__(256) void ffn_gemm_tile_kernel(
+    const uint16_t* __restrict__ A, const float* __restrict__ scale,
+    const uint16_t* __restrict__ B, const uint16_t* __restrict__ R, uint16_t* __restrict__ C,
+    uint16_t* __restrict__ C2, float* __restrict__ Cf, int M, int N, int K, int slices,
+    int skew) {
+  constexpr int kStage = kTileStageBytes<BM>;
+  constexpr int kBOff = BM * kBigK * 2;    // B after A in a stage
+  constexpr int MI = BM / 64;              // 32-row tiles per wave
+  constexpr int AL = BM / 32, L = AL + 4;  // loads per wave and step: A, all
+  // Loads per sub-step: L3 right behind the barrier, LQ in each of the next
+  // three.  With two stages all go behind the barrier: the next wait is three
+  // sub-steps away.
+  constexpr int L3 = ST == 2 ? L : L / 4, LQ = (L - L3) / 3;
+  constexpr int NF = MI + 2;               // fragments per sub-step
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+
+  // XCD x runs blocks x, x + 8, ...: a contiguous run of the unit sequence
+  // (slice-major), walked in blocks of kGroupM M-tiles as the 256-tile kernel.
+  const int tiles_m = M / BM, tiles_n = N / kTileN;
+  const int units = static_cast<int>(gridDim.x);
+  const int xcd = static_cast<int>(blockIdx.x) % 8, rem = units % 8;
+  const int unit = xcd * (units / 8) + (xcd < rem ? xcd : rem) + static_cast<int>(blockIdx.x) / 8;
+  const int slice = unit / (tiles_m * tiles_n);
+  const int t = unit - slice * tiles_m * tiles_n;
+  const int group = t / (kGroupM * tiles_n);
+  const int gm = tiles_m - group * kGroupM < kGroupM ? tiles_m - group * kGroupM : kGroupM;
+  const int within = t - group * kGroupM * tiles_n;
+  const int m0 = (group * kGroupM + within % gm) * BM;
+  const int n0 = within / gm * kTileN;
+  const int steps = K / kBigK;
+  auto slice_begin = [&](int s) { return s * steps / slices; };
+  const int s0 = EPI == kEpiPartial ? slice : 0;
+  const int s1 = EPI == kEpiPartial ? slice + 1 : slices;
+  int first = 0, steps_here = 0, turn = 0;  // the slice being summed: its steps and first load
+
+  const buffer_rsrc_t rsrc_a =
+      make_rsrc(A + static_cast<size_t>(m0) * K, static_cast<uint32_t>(BM) * K * 2u);
+  const buffer_rsrc_t rsrc_b =
+      KN ? make_rsrc(B + n0,
+                     static_cast<uint32_t>((static_cast<size_t>(K - 1) * N + kTileN) * 2))
+         : make_rsrc(B + static_cast<size_t>(n0) * K, static_cast<uint32_t>(kTileN) * K * 2u);
+  const int chunk = (lane & 7) ^ (((wave & 1) << 2) + (lane >> 4));
+  const uint32_t voff = (static_cast<uint32_t>(wave * 8 + (lane >> 3)) * K + chunk * 8) * 2u;
+  const uint32_t voff_kn = (static_cast<uint32_t>(wave * 4 + (lane >> 4)) * N +
+                            ((lane & 15) ^ ((lane >> 4) << 2)) * 8) * 2u;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
+  const uint32_t m0_wave = static_cast<uint32_t>(
+      __builtin_amdgcn_readfirstlane(static_cast<int>(lds0 + wave * 1024)));
+  // Load q of the slice's k-th K-step into `stage`: A rows 8 (4 q + w) .. + 7 (q < AL), else B
+  // rows likewise (KN: K-rows 16 (q - AL) + 4 w .. + 3).
+  auto load = [&](int k, int stage, auto qc) {
+    constexpr int q = decltype(qc)::value;
+    constexpr int qb = q < AL ? q : q - AL;
+    constexpr uint32_t qoff = static_cast<uint32_t>(qb * 4096 + (q < AL ? 0 : kBOff));
+    int kk = (k < steps_here ? k : steps_here - 1) + turn;  // tail: a re-load
+    if (kk >= steps_here) kk -= steps_here;
+    const uint32_t kc = static_cast<uint32_t>(first + kk);
+    const uint32_t soff =
+        KN && q >= AL ? (kc * kBigK + qb * 16) * static_cast<uint32_t>(N) * 2u
+                      : kc * (kBigK * 2) + static_cast<uint32_t>(qb * 64) * static_cast<uint32_t>(K);
+    const uint32_t base = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+        static_cast<int>(m0_wave + static_cast<uint32_t>(stage * kStage))));
+    const uint32_t so =
+        static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(soff)));
+    if constexpr (q < AL)
+      load_to_lds<qoff>(rsrc_a, voff, base, so);
+    else
+      load_to_lds_nt<qoff>(rsrc_b, KN ? voff_kn : voff, base, so);
+  };
+
+  const int fsw = ((lane & 31) >> 1) & 7;
+  const int a_frag = (wm * (BM / 2) + (lane & 31)) * 128;
+  const int b_frag = kBOff + (wn * 64 + (lane & 31)) * 128;
+  // KN fragment j of sub-step kk: as in the 256-tile kernel, with 256-byte
+  // K-rows; the row's swizzle acts on bits 2 and 3 of the chunk, 2 wn + j.
+  const int kn_g = (lane >> 4) & 3, kn_s = (lane & 15) >> 2;
+  const int kn_lane = kBOff + (8 * (kn_g >> 1) + kn_s) * 256 +
+                      (2 * (kn_g & 1) + ((lane >> 1) & 1)) * 16 + 8 * (lane & 1);
+  struct Frags { bf16x8_t v[NF]; };  // A fragments, then B
+  float a_scale[MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+    a_scale[i] = RA ? scale[m0 + wm * (BM / 2) + i * 32 + (lane & 31)] : 1.0f;
+  auto frag = [&](int stage, int kk, int idx) {
+    const char* base = smem + __builtin_amdgcn_readfirstlane(stage * kStage);
+    if (KN && idx >= MI) {
+      const char* p = base + kn_lane + (((2 * wn + idx - MI) ^ kn_s) << 6) + kk * 4096;
+      return __builtin_shufflevector(ds_read_tr16(p), ds_read_tr16(p + 1024), 0, 1, 2, 3, 4, 5,
+                                     6, 7);
+    }
+    const int c = ((2 * kk + (lane >> 5)) ^ fsw) << 4;
+    return *reinterpret_cast<const bf16x8_t*>(
+        base + c + (idx < MI ? a_frag + idx * 4096 : b_frag + (idx - MI) * 4096));
+  };
+  f32x16 acc[MI][2], total[MI][2];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+  // One sub-step: 2 MI MFMAs in MI regions of two, region r with fragment
+  // reads 2 r and 2 r + 1 of the next sub-step and its share of loads Q0 ..
+  // Q0 + NQ - 1 of step lk, each region pinned as in the 256-tile kernel.
+  auto sub_step = [&]<int Q0, int NQ>(const Frags& cur, Frags& nxt, int ns, int nkk, int lk, int ls) {
+    [&]<int... Rs>(std::integer_sequence<int, Rs...>) {
+      (
+          [&] {
+            constexpr int r = Rs;
+            const bf16x8_t a = RA ? scale_bf16x8(cur.v[r], a_scale[r]) : cur.v[r];
+            [&]<int... Js>(std::integer_sequence<int, Js...>) {
+              (
+                  [&] {
+                    constexpr int Mi = 2 * r + Js;
+                    if constexpr (Mi < NF) nxt.v[Mi] = frag(ns, nkk, Mi);
+                    acc[r][Js] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, cur.v[MI + Js],
+                                                                         acc[r][Js], 0, 0, 0);
+                  }(),
+                  ...);
+            }(std::make_integer_sequence<int, 2>{});
+            [&]<int... Qs>(std::integer_sequence<int, Qs...>) {
+              (load(lk, ls, std::integral_constant<int, Q0 + r * NQ / MI + Qs>{}), ...);
+            }(std::make_integer_sequence<int, (r + 1) * NQ / MI - r * NQ / MI>{});
+            [&]<int... Js>(std::integer_sequence<int, Js...>) {
+              (
+                  [&] {
+                    constexpr int Mi = 2 * r + Js;
+                    if constexpr (Mi < NF)
+                      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, KN && Mi >= MI ? 2 : 1,
+                                                           0);
+                    __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+                  }(),
+                  ...);
+            }(std::make_integer_sequence<int, 2>{});
+            __builtin_amdgcn_sched_barrier(0);
+          }(),
+          ...);
+    }(std::make_integer_sequence<int, MI>{});
+  };
+  static_assert(NF <= 2 * MI, "a sub-step's reads fit its regions");
+
+  for (int s = s0; s < s1; ++s) {
+    first = slice_begin(s);
+    steps_here = slice_begin(s + 1) - first;
+    turn = static_cast<int>(static_cast<uint32_t>(skew * (n0 / kTileN)) %
+                            static_cast<uint32_t>(steps_here));
+    // Prologue: the first ST - 1 steps whole and the next one's L3 loads; the
+    // first step landed before its fragments are read.
+#pragma unroll
+    for (int k = 0; k < ST - 1; ++k)
+      [&]<int... Qs>(std::integer_sequence<int, Qs...>) {
+        (load(k, k, std::integral_constant<int, Qs>{}), ...);
+      }(std::make_integer_sequence<int, L>{});
+    [&]<int... Qs>(std::integer_sequence<int, Qs...>) {
+      (load(ST - 1, ST - 1, std::integral_constant<int, Qs>{}), ...);
+    }(std::make_integer_sequence<int, L3>{});
+    wait_vmcnt<(ST - 2) * L + L3>();
+    lds_barrier();
+    Frags f0, f1;
+#pragma unroll
+    for (int m = 0; m < NF; ++m) f0.v[m] = frag(0, 0, m);
+    int cur = 0, prev = ST - 1;  // cur = stage of step it, prev of it - 1 and it + ST - 1
+    for (int it = 0; it < steps_here; ++it) {
+      const int next = cur + 1 == ST ? 0 : cur + 1;
+      sub_step.template operator()<L3, LQ>(f0, f1, cur, 1, it + ST - 1, prev);
+      sub_step.template operator()<L3 + LQ, LQ>(f1, f0, cur, 2, it + ST - 1, prev);
+      sub_step.template operator()<L3 + 2 * LQ, LQ>(f0, f1, cur, 3, it + ST - 1, prev);
+      wait_vmcnt<(ST - 2) * L>();  // own loads of step it+1 landed
+      lds_barrier();
+      sub_step.template operator()<0, L3>(f1, f0, next, 0, it + ST, cur);
+      prev = cur;
+      cur = next;
+    }
+    wait_vmcnt<0>();  // the tail re-loads
+    if constexpr (EPI != kEpiPartial) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            total[i][j][r] = s == s0 ? acc[i][j][r] : total[i][j][r] + acc[i][j][r];
+            acc[i][j][r] = 0.0f;
+          }
+      if (s + 1 < s1) lds_barrier();  // every wave has read its last fragments
+    }
+  }
+
+  // Epilogue.  Registers 4q .. 4q + 3 of tile (i, j) are rows mb .. mb + 3 of
+  // column n.
+  float* part = Cf + static_cast<size_t>(slice) * M * N;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int mb = m0 + wm * (BM / 2) + i * 32 + 8 * q + 4 * (lane >> 5);
+      float sc[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sc[e] = kEpiScaled<EPI> && !RA && scale != nullptr ? scale[mb + e] : 1.0f;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int n = n0 + wn * 64 + j * 32 + (lane & 31);
+        const size_t idx = static_cast<size_t>(mb) * N + n;
+        EpiValue v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (EPI == kEpiPartial) {
+            part[idx + static_cast<size_t>(e) * N] = acc[i][j][4 * q + e];
+          } else {
+            const float rv =
+                kEpiReadsR<EPI> ? bf16_to_f32(R[idx + static_cast<size_t>(e) * N]) : 0.0f;
+            v[e] = epilogue_value<EPI>(total[i][j][4 * q + e], sc[e], rv);
+          }
+        }
+        if constexpr (EPI == kEpiPartial) continue;
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+          const size_t at = idx + static_cast<size_t>(e) * N;
+          if constexpr (EPI == kEpiStoreF32) {
+            Cf[at] = v[e].c;
+            Cf[at + N] = v[e + 1].c;
+          } else if constexpr (EPI != kEpiStoreT) {
+            const uint32_t p = pack_bf16x2(v[e].c, v[e + 1].c);
+            C[at] = static_cast<uint16_t>(p);
+            C[at + N] = static_cast<uint16_t>(p >> 16);
+          }
+          if constexpr (EPI == kEpiGeluSave) {
+            const uint32_t p = pack_bf16x2(v[e].c2, v[e + 1].c2);
+            C2[at] = static_cast<uint16_t>(p);
+            C2[at + N] = static_cast<uint16_t>(p >> 16);
+          }
+        }
+        const size_t tdx = static_cast<size_t>(n) * M + mb;
+        if constexpr (EPI == kEpiStoreT) {
+          *reinterpret_cast<uint2*>(C + tdx) =
+              uint2{pack_bf16x2(v[0].c, v[1].c), pack_bf16x2(v[2].c, v[3].c)};
+        } else if constexpr (EPI == kEpiUH || EPI == kEpiGeluBwd) {
+          if (EPI == kEpiUH || C2 != nullptr)
+            *reinterpret_cast<uint2*>(C2 + tdx) =
+                uint2{pack_bf16x2(v[0].c2, v[1].c2), pack_bf16x2(v[2].c2, v[3].c2)};
+        }
+      }
+    }
+}
+
+// The epilogue of a split GEMM: acc[m, n] = sum over slices, in slice order,
+// of part[slice][m][n].  A 64 x 64 block per workgroup, 4 x 4 elements per
+// lane (16-byte partial reads, 8-byte stores either way round).
+template <int EPI>
+__global__ __launch_bounds__(256) void ffn_reduce_kernel(
+    const float* __restrict__ part, int slices, const float* __restrict__ scale,
+    const uint16_t* __restrict__ R, uint16_t* __restrict__ C, uint16_t* __restrict__ C2,
+    float* __restrict__ Cf, int M, int N) {
+  const int n = blockIdx.x * 64 + (threadIdx.x & 15) * 4;
+  const int m = blockIdx.y * 64 + (threadIdx.x >> 4) * 4;
+  const size_t mn = static_cast<size_t>(M) * N;
+  f32x4 acc[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    acc[e] = *reinterpret_cast<const f32x4*>(part + static_cast<size_t>(m + e) * N + n);
+  for (int s = 1; s < slices; ++s)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      acc[e] += *reinterpret_cast<const f32x4*>(part + s * mn + static_cast<size_t>(m + e) * N + n);
+  float c2[4][4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const size_t idx = static_cast<size_t>(m + e) * N + n;
+    const float sc = kEpiScaled<EPI> && scale != nullptr ? scale[m + e] : 1.0f;
+    uint2 rw{0, 0};
+    if constexpr (kEpiReadsR<EPI>) rw = *reinterpret_cast<const uint2*>(R + idx);
+    const float rv[4] = {bf16_lo(rw.x), bf16_hi(rw.x), bf16_lo(rw.y), bf16_hi(rw.y)};
+    float c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const EpiValue v = epilogue_value<EPI>(acc[e][k], sc, rv[k]);
+      c[k] = v.c;
+      c2[e][k] = EPI == kEpiStoreT ? v.c : v.c2;
+    }
+    if constexpr (EPI == kEpiStoreF32)
+      *reinterpret_cast<f32x4*>(Cf + idx) = f32x4{c[0], c[1], c[2], c[3]};
+    else if constexpr (EPI != kEpiStoreT)
+      *reinterpret_cast<uint2*>(C + idx) =
+          uint2{pack_bf16x2(c[0], c[1]), pack_bf16x2(c[2], c[3])};
+    if constexpr (EPI == kEpiGeluSave)
+      *reinterpret_cast<uint2*>(C2 + idx) =
+          uint2{pack_bf16x2(c2[e][0], c2[e][1]), pack_bf16x2(c2[e][2], c2[e][3])};
+  }
+  if constexpr (EPI == kEpiUH || EPI == kEpiGeluBwd || EPI == kEpiStoreT) {
+    uint16_t* dst = EPI == kEpiStoreT ? C : C2;
+    if (EPI == kEpiGeluBwd && C2 == nullptr) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      *reinterpret_cast<uint2*>(dst + static_cast<size_t>(n + k) * M + m) =
+          uint2{pack_bf16x2(c2[0][k], c2[1][k]), pack_bf16x2(c2[2][k], c2[3][k])};
+    }
+  }
+}
+
 // dst[c, r] = bf16(src[r, c] * scale[r]) (scale == nullptr: a plain copy
 // of the bits) for a rows x cols bf16 matrix, through a 64 x 64 LDS tile.
 // Full tiles (rows and cols multiples of 64, 16-byte aligned rows) move 16
@@ -865,51 +1097,214 @@ bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0;
 // Sums the 256-tile GEMMs add their clock stamps to (credit_set_clock_probe).
 std::atomic<uint64_t*> g_clock_probe{nullptr};
 
-// The 256-tile kernels take 160 KiB of dynamic LDS; allow it once per
-// process (the attribute belongs to the kernel, not to a device).
-template <int EPI, bool KN>
-hipError_t allow_big_lds() {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(ffn_gemm256_kernel<EPI, KN>),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, kBigLds);
-}
-template <bool KN>
-int enable_big_lds() {
-  static int status = [] {
-    for (const hipError_t e :
-         {allow_big_lds<kEpiGelu, KN>(), allow_big_lds<kEpiGeluSave, KN>(),
-          allow_big_lds<kEpiResidual, KN>(),
-          allow_big_lds<kEpiUH, KN>(), allow_big_lds<kEpiGeluBwd, KN>(),
-          allow_big_lds<kEpiStore, KN>(), allow_big_lds<kEpiStoreF32, KN>(),
-          allow_big_lds<kEpiStoreT, KN>()})
-      if (e != hipSuccess) return hip_failure(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
-    return static_cast<int>(CREDIT_OK);
-  }();
-  return status;
+// The GEMM kernels take more dynamic LDS than the default limit; allow it
+// once per process and kernel (the attribute belongs to the kernel, not to a
+// device).
+template <class Kernel>
+int allow_lds(Kernel kernel, int bytes) {
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  return e == hipSuccess ? CREDIT_OK
+                         : hip_failure(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
 }
 
-// C[M, N] = epi(A[M, K] B^T) with B [N, K] (KN false) or [K, N] (KN true):
-// the 256-tile kernel when M and N are multiples of 256, K a multiple of
-// 128 (an even number of 64-wide K-steps), the tile count a multiple of the
-// 8 XCDs and a B tile (256 * K * 2 bytes, KN: (K - 1) * N * 2 + 512), an A
-// tile and the epilogue's R tile ((255 * N + 256) * 2 bytes) fit a buffer
-// resource; otherwise the 128-tile kernel (M, N multiples of 128, K of 64).
+// How a product C[M, N] over K runs, from its sizes alone and the same for
+// (M, N) and (N, M), so that every entry point that forms a product (either
+// weight layout, recomputed or saved) adds its terms in the same order.
+//  - slices: K pieces.  Time of the units on 256 CUs (flat_us), plus, when
+//    split, kReduceUs and the fp32 sums written and read at kReduceGBs.  1024 x
+//    2048 x 8192 (128 tiles): 131 us on 32 256-tiles, 47 + 5 us in 2 slices;
+//    128 x 8192 x 28672 (64 tiles): 472 us, 103 + 5 us in 4.
+//  - bm: 256 where its rounds take less by the same count; a tall step costs
+//    less than two flat ones (fewer LDS bytes per MFMA), but 256 x 6144 x
+//    18944 gains (245 -> 196 us) where 512 x 28672 x 8192 would leave half the
+//    CUs idle (490 -> 540 us).
+//  - big: likewise (the FFN of 1024 rows x 8192 x 28672: 783 us with it
+//    against 846 on tall tiles; 512 rows, 224 tiles: 487 against 512).
+struct GemmPlan {
+  bool big;    // the 256-tile kernel
+  int bm;      // else rows per tile of ffn_gemm_tile_kernel
+  int slices;
+  int skew;    // its tile columns start their slices a step apart
+};
+constexpr int kGemmCus = 256;
+constexpr int kMaxSlices = 16;
+// Time of `units` tiles of `steps` 64-wide K-steps, from 1024-row products:
+// 0.45 us a step and 6 us beside them for a 128-row tile (0.6 us where two
+// share a CU), 0.85 and 8.4 us for a 256-row one, 1.55 and 10 us for the
+// 256-tile kernel's.
+double flat_us(int64_t units, int64_t steps) {
+  const int64_t rounds = (units + kGemmCus - 1) / kGemmCus;
+  return rounds * (steps * (rounds > 1 ? 0.6 : 0.45) + 6.0);
+}
+double tall_us(int64_t units, int64_t steps) {
+  return (units + kGemmCus - 1) / kGemmCus * (steps * 0.85 + 8.4);
+}
+double big_us(int64_t units, int64_t steps) {
+  return (units + kGemmCus - 1) / kGemmCus * (steps * 1.55 + 10.0);
+}
+constexpr int64_t kSlabBytes = int64_t{64} << 20;  // most fp32 partial sums of one product
+
+int gemm_slices(int64_t M, int64_t N, int64_t K) {
+  constexpr double kReduceUs = 4.0, kReduceGBs = 4000.0;
+  const int64_t tiles = (M / 128) * (N / 128), steps = K / kBigK;
+  int best = 1;
+  double best_us = 1e30;
+  for (int s = 1; s <= kMaxSlices && steps / s >= 8; ++s) {
+    if (s > 1 && s * M * N * 4 > kSlabBytes) break;
+    double us = flat_us(tiles * s, (steps + s - 1) / s);
+    if (s > 1) us += kReduceUs + s * M * N * 8.0 / (kReduceGBs * 1e3);
+    if (us < best_us * 0.95) {
+      best = s;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+// Shapes the 256-tile kernel can take: M and N multiples of 256, K of 128, a
+// tile count that is a multiple of the 8 XCDs, and operand tiles (256 * K * 2
+// bytes; a [K, N] B's (K - 1) * N * 2 + 512, which every accepted shape keeps
+// below 2^32) and the epilogue's R tile ((255 * N + 256) * 2 bytes) that fit
+// a buffer resource.  A GEMM that scales its A rows (RMSNorm) multiplies the
+// fp32 sums by rstd on these shapes and rounds x * rstd to bf16 first on every
+// other one, whichever kernel runs.
+bool big_shape(int64_t M, int64_t N, int64_t K) {
+  return M % kBig == 0 && N % kBig == 0 && K % (2 * kBigK) == 0 &&
+         ((M / kBig) * (N / kBig)) % 8 == 0 && K <= (1 << 22) && N <= (1 << 22);
+}
+
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K) {
+  GemmPlan p{false, 128, gemm_slices(M, N, K), 0};
+  const int64_t steps = K / kBigK / p.slices, tiles = (M / 128) * (N / 128) * p.slices;
+  double us = flat_us(tiles, steps);
+  if (M % 256 == 0 && K <= (1 << 22) && tall_us(tiles / 2, steps) < us) {
+    p.bm = 256;
+    us = tall_us(tiles / 2, steps);
+  }
+  p.big = p.slices == 1 && big_shape(M, N, K) && big_us(tiles / 4, steps) < us;
+  p.skew = M == p.bm;
+  return p;
+}
+
+// Scratch bytes: the partial sums of a product, and those of the scaled
+// product with its copy of a.
+size_t part_bytes(int64_t M, int64_t N, int64_t K) {
+  const int64_t slices = gemm_slices(M, N, K);
+  return slices > 1 ? static_cast<size_t>(slices * M * N) * sizeof(float) : 0;
+}
+size_t copy_bytes(int64_t M, int64_t F, int64_t D) {
+  return big_shape(M, F, D) ? 0 : align_up(static_cast<size_t>(M) * D * 2, 256);
+}
+size_t norm_bytes(int64_t M, int64_t F, int64_t D) {
+  return copy_bytes(M, F, D) + part_bytes(M, F, D);
+}
+
+// Device memory a call's products may use beside its own buffers: fp32
+// partial sums, and the scaled copy of x where a product rounds it first.
+struct Scratch {
+  char* base = nullptr;
+  size_t bytes = 0;
+};
+
+template <int EPI, bool KN, int BM, int ST, bool RA>
+int launch_tile_st(const uint16_t* A, const float* scale, const uint16_t* B, const uint16_t* R,
+                uint16_t* C, uint16_t* C2, float* Cf, int M, int N, int K, const GemmPlan& plan,
+                hipStream_t stream, const char* name) {
+  constexpr int kLds = ST * kTileStageBytes<BM>;
+  static const int lds = allow_lds(ffn_gemm_tile_kernel<EPI, KN, BM, ST, RA>, kLds);
+  if (lds != CREDIT_OK) return lds;
+  const int units = (M / BM) * (N / kTileN) * (EPI == kEpiPartial ? plan.slices : 1);
+  ffn_gemm_tile_kernel<EPI, KN, BM, ST, RA><<<dim3(static_cast<unsigned>(units)), dim3(256), kLds,
+                                              stream>>>(A, scale, B, R, C, C2, Cf, M, N, K,
+                                                        plan.slices, plan.skew);
+  return check_launch(name);
+}
+
+// Stages by residency: one workgroup per CU takes the LDS whole; more units
+// than CUs run two to a CU on two stages each (384 x 3584 x 12416: 128 -> 122
+// us for the FFN, 1408 x 2944 x 9856 training step 735 -> 708; a few shapes of
+// 1.1 to 1.4 units per CU lose up to 5%).
+template <int EPI, bool KN, int BM, bool RA>
+int launch_tile(const uint16_t* A, const float* scale, const uint16_t* B, const uint16_t* R,
+                uint16_t* C, uint16_t* C2, float* Cf, int M, int N, int K, const GemmPlan& plan,
+                hipStream_t stream, const char* name) {
+  if constexpr (BM == 256) {
+    return launch_tile_st<EPI, KN, BM, 3, RA>(A, scale, B, R, C, C2, Cf, M, N, K, plan, stream,
+                                              name);
+  } else {
+    const int units = (M / BM) * (N / kTileN) * (EPI == kEpiPartial ? plan.slices : 1);
+    return units > kGemmCus ? launch_tile_st<EPI, KN, BM, 2, RA>(A, scale, B, R, C, C2, Cf, M, N,
+                                                                 K, plan, stream, name)
+                            : launch_tile_st<EPI, KN, BM, 4, RA>(A, scale, B, R, C, C2, Cf, M, N,
+                                                                 K, plan, stream, name);
+  }
+}
+
+// C[M, N] = epi(A[M, K] B^T) with B [N, K] (KN false) or [K, N] (KN true);
+// M, N and K multiples of 128.  ra: the A rows are scaled by scale and rounded
+// as the product runs.  A product that is to be split and whose partial sums
+// the scratch does not hold (a smaller caller workspace) runs unsplit, one
+// workgroup covering its tile's slices in the same order, with the same bits.
 template <int EPI, bool KN = false>
 int launch_gemm(const uint16_t* A, const float* scale, const uint16_t* B, const uint16_t* R,
-                uint16_t* C, uint16_t* C2, float* Cf, int M, int N, int K, hipStream_t stream,
-                const char* name) {
-  const bool big = M % kBig == 0 && N % kBig == 0 && K % (2 * kBigK) == 0 &&
-                   ((M / kBig) * (N / kBig)) % 8 == 0 && K <= (1 << 22) && N <= (1 << 22) &&
-                   (!KN || static_cast<uint64_t>(K) * N * 2 < (uint64_t{1} << 32));
-  if (big) {
-    CREDIT_TRY(enable_big_lds<KN>());
+                uint16_t* C, uint16_t* C2, float* Cf, int M, int N, int K, const Scratch& scratch,
+                hipStream_t stream, const char* name, bool ra = false) {
+  GemmPlan plan = gemm_plan(M, N, K);
+  // The weight gradients are formed either way round (M and N swapped).
+  if (EPI == kEpiStore || EPI == kEpiStoreT) plan.skew = 0;
+  if constexpr (kEpiScaled<EPI>) {
+    if (ra)
+      return launch_tile<EPI, KN, 128, true>(A, scale, B, R, C, C2, Cf, M, N, K, plan, stream,
+                                             name);
+  }
+  if (plan.big) {
+    static const int lds = allow_lds(ffn_gemm256_kernel<EPI, KN>, kBigLds);
+    if (lds != CREDIT_OK) return lds;
     ffn_gemm256_kernel<EPI, KN><<<dim3(static_cast<unsigned>((M / kBig) * (N / kBig))),
                                   dim3(kBigThreads), kBigLds, stream>>>(
         A, scale, B, R, C, C2, Cf, M, N, K, g_clock_probe.load(std::memory_order_relaxed));
-  } else {
-    ffn_gemm_kernel<EPI, KN><<<dim3(static_cast<unsigned>((M / kBM) * (N / kBN))),
-                               dim3(kThreads), 0, stream>>>(A, scale, B, R, C, C2, Cf, M, N, K);
+    return check_launch(name);
   }
-  return check_launch(name);
+  if (plan.slices > 1 &&
+      scratch.bytes >= static_cast<size_t>(plan.slices) * M * N * sizeof(float)) {
+    float* part = reinterpret_cast<float*>(scratch.base);
+    CREDIT_TRY((plan.bm == 256
+                    ? launch_tile<kEpiPartial, KN, 256, false>(A, nullptr, B, nullptr, nullptr,
+                                                               nullptr, part, M, N, K, plan, stream,
+                                                               name)
+                    : launch_tile<kEpiPartial, KN, 128, false>(A, nullptr, B, nullptr, nullptr,
+                                                               nullptr, part, M, N, K, plan, stream,
+                                                               name)));
+    ffn_reduce_kernel<EPI><<<dim3(static_cast<unsigned>(N / 64), static_cast<unsigned>(M / 64)),
+                             dim3(256), 0, stream>>>(part, plan.slices, scale, R, C, C2, Cf, M, N);
+    return check_launch("ffn_reduce_kernel");
+  }
+  return plan.bm == 256 ? launch_tile<EPI, KN, 256, false>(A, scale, B, R, C, C2, Cf, M, N, K,
+                                                           plan, stream, name)
+                        : launch_tile<EPI, KN, 128, false>(A, scale, B, R, C, C2, Cf, M, N, K,
+                                                           plan, stream, name);
+}
+
+// The scaled product u = rstd (x W1^T) with its RMSNorm statistics: rstd, then
+// the GEMM over x with rstd in the epilogue, or on the shapes that round
+// a = bf16(x * rstd) first over the copy of a that the scratch holds.
+template <int EPI, bool KN>
+int launch_norm_gemm(const uint16_t* x, float* rstd, const uint16_t* w1, uint16_t* C, uint16_t* C2,
+                     int M, int F, int D, float eps, const Scratch& scratch, hipStream_t stream,
+                     const char* name) {
+  uint16_t* a = nullptr;
+  const bool rounds = !big_shape(M, F, D);
+  const size_t a_bytes = copy_bytes(M, F, D);
+  Scratch rest = scratch;
+  if (rounds && scratch.bytes >= norm_bytes(M, F, D)) {
+    a = reinterpret_cast<uint16_t*>(scratch.base);
+    rest = Scratch{scratch.base + a_bytes, scratch.bytes - a_bytes};
+  }
+  ffn_rstd_kernel<<<dim3(M), dim3(256), 0, stream>>>(x, rstd, a, D, eps);
+  CREDIT_TRY(check_launch("ffn_rstd_kernel"));
+  return launch_gemm<EPI, KN>(a != nullptr ? a : x, a != nullptr ? nullptr : rstd, w1, nullptr, C,
+                              C2, nullptr, M, F, D, rest, stream, name, rounds && a == nullptr);
 }
 
 int launch_transpose(const uint16_t* src, uint16_t* dst, int64_t rows, int64_t cols,
@@ -947,10 +1342,53 @@ BwdLayout bwd_layout(int64_t M, int64_t d, int64_t f) {
   return l;
 }
 
+// Scratch of the whole calls: the most any one of their products uses.
+size_t fwd_scratch(int64_t M, int64_t d, int64_t f) {
+  return std::max(norm_bytes(M, f, d), part_bytes(M, d, f));
+}
+size_t bwd_scratch(int64_t M, int64_t d, int64_t f) {
+  return std::max({norm_bytes(M, f, d), part_bytes(d, f, M), part_bytes(M, d, f)});
+}
+
+// The training forward brings no workspace and shares none: its scratch is a
+// buffer per (device, stream) of its own, in use only between the launches of
+// one call, which train_mutex keeps together when threads share a stream.  At
+// most 2 * kTrainScratch per stream, never freed while the process runs.
+constexpr size_t kTrainScratch = size_t{256} << 20;
+struct ScratchAlloc {
+  int operator()(int, void*, size_t bytes, char** out) const {
+    // Relaxed: another thread's stream may be under capture meanwhile.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    void* p = nullptr;
+    const hipError_t err = hipMalloc(&p, bytes);
+    if (err != hipSuccess) (void)hipGetLastError();  // no memory to spare: the call does without
+    CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    if (err != hipSuccess) return CREDIT_ERR_HIP;
+    *out = static_cast<char*>(p);
+    return CREDIT_OK;
+  }
+};
+std::mutex& train_mutex() {
+  static std::mutex* m = new std::mutex();
+  return *m;
+}
+int train_scratch(hipStream_t stream, size_t want, Scratch* out) {
+  static WorkspaceCache<ScratchAlloc>* cache = new WorkspaceCache<ScratchAlloc>();
+  *out = Scratch{};
+  if (want == 0) return CREDIT_OK;
+  int dev = 0;
+  CREDIT_HIP(hipGetDevice(&dev));
+  if (cache->capacity(dev, stream) < want && stream_capturing(stream)) return CREDIT_OK;
+  char* p = nullptr;
+  if (cache->get(dev, stream, want, &p) == CREDIT_OK) *out = Scratch{p, want};
+  return CREDIT_OK;
+}
+
 int check_ffn_shape(int64_t rows, int64_t d, int64_t f) {
   if (rows < 0 || d < 1 || f < 1)
     return set_error(CREDIT_ERR_BAD_SHAPE, "ffn: need rows >= 0, d >= 1, f >= 1");
-  if (rows % kBM != 0 || d % kBN != 0 || f % kBN != 0 || d % kBK != 0 || f % kBK != 0)
+  if (rows % kFfnMultiple != 0 || d % kFfnMultiple != 0 || f % kFfnMultiple != 0)
     return set_error(CREDIT_ERR_UNSUPPORTED,
                      "ffn: rows, d and f must be multiples of 128 (got %lld, %lld, %lld)",
                      static_cast<long long>(rows), static_cast<long long>(d),
@@ -969,8 +1407,15 @@ size_t ffn_workspace(int64_t rows, int64_t ffn_dim) {
          align_up(static_cast<size_t>(rows) * ffn_dim * sizeof(uint16_t), 256);
 }
 
+// What callers are told to bring: the calls' own use plus scratch for their
+// products (the forward's query does not know d, so what it names may not hold
+// a copy of a; a call runs with any scratch or none).
+size_t ffn_workspace_advised(int64_t rows, int64_t ffn_dim) {
+  return align_up(ffn_workspace(rows, ffn_dim), 256) + kSlabBytes;
+}
+
 size_t ffn_bwd_workspace(int64_t rows, int64_t d, int64_t ffn_dim) {
-  return bwd_layout(rows, d, ffn_dim).total;
+  return align_up(bwd_layout(rows, d, ffn_dim).total, 256) + bwd_scratch(rows, d, ffn_dim);
 }
 
 }  // namespace credit
@@ -1014,18 +1459,18 @@ int ffn_forward(const uint16_t* x, const uint16_t* w1, const uint16_t* w2, uint1
     return set_error(CREDIT_ERR_ALIGNMENT, "ffn: x, w1, w2 and out must be 16-byte aligned");
   if (rows == 0) return CREDIT_OK;
   char* ws = nullptr;
-  CREDIT_TRY(acquire_workspace(cfg, ffn_workspace(rows, f), &ws));
+  Scratch scratch;
+  CREDIT_TRY(acquire_workspace_with(cfg, ffn_workspace(rows, f), fwd_scratch(rows, d, f), &ws,
+                                    &scratch.base, &scratch.bytes));
   float* rstd = reinterpret_cast<float*>(ws_scratch(ws));
   uint16_t* h = reinterpret_cast<uint16_t*>(
       ws_scratch(ws) + align_up(static_cast<size_t>(rows) * sizeof(float), 256));
   hipStream_t stream = cfg_stream(cfg);
   const int M = static_cast<int>(rows), D = static_cast<int>(d), F = static_cast<int>(f);
-  ffn_rstd_kernel<<<dim3(M), dim3(256), 0, stream>>>(x, rstd, D, eps);
-  CREDIT_TRY(check_launch("ffn_rstd_kernel"));
-  CREDIT_TRY((launch_gemm<kEpiGelu, KN>(x, rstd, w1, nullptr, h, nullptr, nullptr, M, F, D,
-                                       stream, "ffn gemm1 (gelu)")));
-  return launch_gemm<kEpiResidual, KN>(h, nullptr, w2, x, out, nullptr, nullptr, M, D, F, stream,
-                                       "ffn gemm2 (residual)");
+  CREDIT_TRY((launch_norm_gemm<kEpiGelu, KN>(x, rstd, w1, h, nullptr, M, F, D, eps, scratch, stream,
+                                             "ffn gemm1 (gelu)")));
+  return launch_gemm<kEpiResidual, KN>(h, nullptr, w2, x, out, nullptr, nullptr, M, D, F, scratch,
+                                       stream, "ffn gemm2 (residual)");
 }
 
 }  // namespace
@@ -1063,13 +1508,16 @@ int ffn_train_forward(const uint16_t* x, const uint16_t* w1, const uint16_t* w2,
                        "ffn training forward: x, w1, w2, out, u and h must be 16-byte aligned");
   if (rows == 0) return CREDIT_OK;
   hipStream_t stream = cfg_stream(cfg);
+  size_t want = fwd_scratch(rows, d, f);
+  if (want > kTrainScratch) want = std::max(part_bytes(rows, f, d), part_bytes(rows, d, f));
+  std::lock_guard<std::mutex> lock(train_mutex());
+  Scratch scratch;
+  CREDIT_TRY(train_scratch(stream, want, &scratch));
   const int M = static_cast<int>(rows), D = static_cast<int>(d), F = static_cast<int>(f);
-  ffn_rstd_kernel<<<dim3(M), dim3(256), 0, stream>>>(x, rstd, D, eps);
-  CREDIT_TRY(check_launch("ffn_rstd_kernel"));
-  CREDIT_TRY((launch_gemm<kEpiGeluSave, KN>(x, rstd, w1, nullptr, h, u, nullptr, M, F, D, stream,
-                                            "ffn gemm1 (gelu, saving u and h)")));
-  return launch_gemm<kEpiResidual, KN>(h, nullptr, w2, x, out, nullptr, nullptr, M, D, F, stream,
-                                       "ffn gemm2 (residual)");
+  CREDIT_TRY((launch_norm_gemm<kEpiGeluSave, KN>(x, rstd, w1, h, u, M, F, D, eps, scratch, stream,
+                                                 "ffn gemm1 (gelu, saving u and h)")));
+  return launch_gemm<kEpiResidual, KN>(h, nullptr, w2, x, out, nullptr, nullptr, M, D, F, scratch,
+                                       stream, "ffn gemm2 (residual)");
 }
 
 }  // namespace
@@ -1160,7 +1608,9 @@ int ffn_backward(const uint16_t* x, const uint16_t* w1, const uint16_t* w2,
   }
   const BwdLayout L = bwd_layout(rows, d, f);
   char* ws = nullptr;
-  CREDIT_TRY(acquire_workspace(cfg, L.total, &ws));
+  Scratch scratch;
+  CREDIT_TRY(acquire_workspace_with(cfg, L.total, bwd_scratch(rows, d, f), &ws, &scratch.base,
+                                    &scratch.bytes));
   char* b = ws_scratch(ws);
   const float* rstd = saved ? saved->rstd : reinterpret_cast<float*>(b + L.rstd);
   const uint16_t* u = saved ? saved->u : reinterpret_cast<uint16_t*>(b + L.u);
@@ -1171,53 +1621,49 @@ int ffn_backward(const uint16_t* x, const uint16_t* w1, const uint16_t* w2,
   uint16_t* at = reinterpret_cast<uint16_t*>(b + L.at);
   float* da = reinterpret_cast<float*>(b + L.da);
   const int M = static_cast<int>(rows), D = static_cast<int>(d), F = static_cast<int>(f);
-  if (saved == nullptr) {
-    ffn_rstd_kernel<<<dim3(M), dim3(256), 0, stream>>>(x, reinterpret_cast<float*>(b + L.rstd), D,
-                                                       eps);
-    CREDIT_TRY(check_launch("ffn_rstd_kernel"));
-  }
+  // u = (x W1^T) rstd (x W1 for [in, out]), h^T = GELU(u)^T, unless saved.
+  if (saved == nullptr)
+    CREDIT_TRY((launch_norm_gemm<kEpiUH, KN>(x, reinterpret_cast<float*>(b + L.rstd), w1,
+                                             reinterpret_cast<uint16_t*>(b + L.u), ht, M, F, D,
+                                             eps, scratch, stream, "ffn bwd gemm u")));
   // The A operands of the weight gradients in the K-contiguous layout A
   // takes: a^T = bf16(x rstd)^T always, dout^T where no other form reads it.
   if (!KN || saved != nullptr) CREDIT_TRY(launch_transpose(dout, doutt, M, D, nullptr, stream));
   CREDIT_TRY(launch_transpose(x, at, M, D, rstd, stream));
-  // u = (x W1^T) rstd (x W1 for [in, out]), h^T = GELU(u)^T, unless saved.
-  if (saved == nullptr)
-    CREDIT_TRY((launch_gemm<kEpiUH, KN>(x, rstd, w1, nullptr, reinterpret_cast<uint16_t*>(b + L.u),
-                                        ht, nullptr, M, F, D, stream, "ffn bwd gemm u")));
   // du = (dout W2) * GELU'(u) (dout W2^T for [in, out]), with du^T for the
   // nn.Linear dW1 GEMM.
   CREDIT_TRY((launch_gemm<kEpiGeluBwd, !KN>(dout, nullptr, w2, u, du, KN ? nullptr : dut,
-                                            nullptr, M, F, D, stream, "ffn bwd gemm du")));
+                                            nullptr, M, F, D, scratch, stream, "ffn bwd gemm du")));
   if constexpr (!KN) {
     // dW2 [d, f] = dout^T h: h^T [f, M] as the B operand, or the saved h
     // [M, f] read as [K, N].
     if (saved == nullptr)
       CREDIT_TRY(launch_gemm<kEpiStore>(doutt, nullptr, ht, nullptr, dw2, nullptr, nullptr, D, F,
-                                        M, stream, "ffn bwd gemm dw2"));
+                                        M, scratch, stream, "ffn bwd gemm dw2"));
     else
       CREDIT_TRY((launch_gemm<kEpiStore, true>(doutt, nullptr, saved->h, nullptr, dw2, nullptr,
-                                               nullptr, D, F, M, stream, "ffn bwd gemm dw2")));
+                                               nullptr, D, F, M, scratch, stream, "ffn bwd gemm dw2")));
     // dW1 [f, d] = du^T a.
     CREDIT_TRY(launch_gemm<kEpiStore>(dut, nullptr, at, nullptr, dw1, nullptr, nullptr, F, D, M,
-                                      stream, "ffn bwd gemm dw1"));
+                                      scratch, stream, "ffn bwd gemm dw1"));
   } else {
     // dW2 [f, d] = h^T dout: h^T as A and dout [M, d] read as [K, N]; from
     // the saved h, (dout^T h)^T with h read as [K, N] and the output stored
     // transposed.
     if (saved == nullptr)
       CREDIT_TRY((launch_gemm<kEpiStore, true>(ht, nullptr, dout, nullptr, dw2, nullptr, nullptr,
-                                               F, D, M, stream, "ffn bwd gemm dw2")));
+                                               F, D, M, scratch, stream, "ffn bwd gemm dw2")));
     else
       CREDIT_TRY((launch_gemm<kEpiStoreT, true>(doutt, nullptr, saved->h, nullptr, dw2, nullptr,
-                                                nullptr, D, F, M, stream, "ffn bwd gemm dw2")));
+                                                nullptr, D, F, M, scratch, stream, "ffn bwd gemm dw2")));
     // dW1 [d, f] = a^T du: du [M, f] read as [K, N].
     CREDIT_TRY((launch_gemm<kEpiStore, true>(at, nullptr, du, nullptr, dw1, nullptr, nullptr, D, F,
-                                             M, stream, "ffn bwd gemm dw1")));
+                                             M, scratch, stream, "ffn bwd gemm dw1")));
   }
   // da [M, d] = du W1 (du W1^T for [in, out]), fp32, then dx = dout +
   // RMSNorm backward of da.
   CREDIT_TRY((launch_gemm<kEpiStoreF32, !KN>(du, nullptr, w1, nullptr, nullptr, nullptr, da, M, D,
-                                             F, stream, "ffn bwd gemm da")));
+                                             F, scratch, stream, "ffn bwd gemm da")));
   ffn_dx_kernel<<<dim3(M), dim3(256), 0, stream>>>(x, rstd, da, dout, dx, D);
   return check_launch("ffn_dx_kernel");
 }

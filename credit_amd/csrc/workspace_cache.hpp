@@ -61,6 +61,13 @@ class WorkspaceCache {
     return e == nullptr ? nullptr : e->buf.ptr;
   }
 
+  // Bytes the buffer of (device, stream) holds now (0: none yet).
+  size_t capacity(int device, void* stream) {
+    std::lock_guard<std::mutex> lock(mu_);
+    Entry* e = find(device, stream);
+    return e == nullptr ? 0 : e->buf.bytes;
+  }
+
   // Every live buffer (for maintenance that must reach all of them).
   std::vector<WsBuffer> live() {
     std::lock_guard<std::mutex> lock(mu_);

@@ -368,8 +368,8 @@ int credit_pearson_bwd_f32(const float* x, const float* y, const float* grad, fl
 /* ------------------------------------------ C5: norm-fused FFN ----------
  * out = bf16(x + h @ W2^T), h = bf16(GELU_tanh(rstd * (x @ W1^T))) with
  * rstd = 1/sqrt(mean_j x^2 + eps) per row (RMSNorm with unit weight), fp32
- * accumulation on bf16 MFMA.  (Shapes that take the 128 x 128 tile GEMM --
- * d or f not a multiple of 256 -- form h = bf16(GELU_tanh(bf16(x * rstd) @
+ * accumulation on bf16 MFMA.  (Shapes that are not whole 256 x 256
+ * tiles, a multiple of 8 of them -- d or f not a multiple of 256, few rows -- form h = bf16(GELU_tanh(bf16(x * rstd) @
  * W1^T)): the normalised input rounded to bf16 before the product.)  Weights in the nn.Linear layout:
  * w1 [f, d] and w2 [d, f] (K contiguous).  x, out [rows, d].  rows, d and
  * f must be multiples of 128; buffers 16-byte aligned.  The hidden

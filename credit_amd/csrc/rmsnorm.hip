@@ -333,6 +333,111 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_slice_kernel(
   split_leave(sa);
 }
 
+// STAGED backward: rows of at most 8192 columns, each held by a team of
+// TEAM lanes (a dwordx4 of x and of dy per lane).  One 1024-lane workgroup
+// per CU runs T = 1024 / TEAM teams over its block of rows, team t taking rows
+// t, t + T, ...; three rows' loads are in flight while a row is reduced and
+// written, all row traffic through buffer resources (a row past the block
+// has num_records 0), so nothing waits for more than the oldest row.  dw
+// accumulates per lane in fp64 registers; the teams' sums are added in team
+// order through LDS, so a workgroup leaves one fp64 partial row however many
+// teams it has.  Bound by HBM: at 4096 x 8192 the 512-lane workgroups before
+// it, two to a CU with the accumulators in LDS, left 512 partial rows
+// (33.5 MB) and ran 54.5 us, the partial reduction behind them 26 us.
+constexpr int kRowsThreads = 1024;
+constexpr size_t kRowsLds = size_t{kRowsThreads} * 8 * sizeof(double);  // 64 KiB
+
+// Workgroup barrier for LDS only: loads and stores in flight stay so.
+__device__ __forceinline__ void lds_only_barrier() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), vmcnt and expcnt at their maxima
+  __builtin_amdgcn_s_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+template <int TEAM>
+__global__ __launch_bounds__(kRowsThreads) void rmsnorm_bwd_rows_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
+    const uint16_t* __restrict__ dy, const float* __restrict__ rstd, uint16_t* __restrict__ dx,
+    double* __restrict__ dw_part, int rows, int cols, int rows_per_group) {
+  constexpr int T = kRowsThreads / TEAM;  // teams
+  constexpr int NW = TEAM / kWave;        // waves per team
+  extern __shared__ double dw_lds[];      // [team][8 TEAM]
+  __shared__ double red[2][T][NW];
+  const int lane = threadIdx.x % TEAM;
+  const int team = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / TEAM);
+  const int wave = __builtin_amdgcn_readfirstlane(lane / kWave);
+  const int r0 = blockIdx.x * rows_per_group;
+  const int r1 = r0 + rows_per_group < rows ? r0 + rows_per_group : rows;
+  const uint32_t row_bytes = static_cast<uint32_t>(cols) * 2u;
+  const uint32_t off = static_cast<uint32_t>(lane) * 16u;
+  struct Row {
+    u32x4 x, dy;
+    float rs;
+  };
+  auto load = [&](Row& b, int r) {
+    const bool in = r < r1;
+    const size_t at = static_cast<size_t>(in ? r : r0) * cols;
+    b.x = buffer_load_nt(make_rsrc(x + at, in ? row_bytes : 0u), off);
+    b.dy = buffer_load_nt(make_rsrc(dy + at, in ? row_bytes : 0u), off);
+    const float rs = rstd[in ? r : r0];
+    b.rs = in ? rs : 0.0f;  // a row past the block adds nothing, whatever rstd holds
+  };
+  const u32x4 wv = buffer_load(make_rsrc(w, row_bytes), off);
+  double acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.0;
+  // Row r of the team, with the loads of row r + 3 T issued first.  Every
+  // team runs the same number of steps (one barrier each); red alternates.
+  auto step = [&](const Row& cur, Row& ahead, int r, int parity) {
+    load(ahead, r + 3 * T);
+    const double ws = wave_reduce_sum_f64(static_cast<double>(gx8(cur.x, cur.dy, wv)));
+    if (threadIdx.x % kWave == 0) red[parity][team][wave] = ws;
+    lds_only_barrier();
+    double dot = red[parity][team][0];
+#pragma unroll
+    for (int v = 1; v < NW; ++v) dot += red[parity][team][v];
+    // c = mean(g * xhat) = rs * sum(dy*w*x) / cols
+    const float c = static_cast<float>(dot * cur.rs / cols);
+    const double rsd = static_cast<double>(cur.rs);
+    buffer_store_nt(make_rsrc(dx + static_cast<size_t>(r < r1 ? r : r0) * cols,
+                              r < r1 ? row_bytes : 0u),
+                    off, dx8(cur.x, cur.dy, wv, cur.rs, c));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // dy*x is exact in fp32 (bf16 x bf16); times rstd it is exact in fp64.
+      acc[2 * i] += static_cast<double>(bf16_lo(cur.dy[i]) * bf16_lo(cur.x[i])) * rsd;
+      acc[2 * i + 1] += static_cast<double>(bf16_hi(cur.dy[i]) * bf16_hi(cur.x[i])) * rsd;
+    }
+  };
+  Row a, b, c, d;
+  load(a, r0 + team);
+  load(b, r0 + team + T);
+  load(c, r0 + team + 2 * T);
+  // Four row buffers in turn; rows past the block are zeros that add nothing.
+  for (int base = r0; base < r1; base += 4 * T) {
+    step(a, d, base + team, 0);
+    if (base + T >= r1) break;
+    step(b, a, base + team + T, 1);
+    if (base + 2 * T >= r1) break;
+    step(c, b, base + team + 2 * T, 0);
+    if (base + 3 * T >= r1) break;
+    step(d, c, base + team + 3 * T, 1);
+  }
+  double* mine = dw_lds + 8 * (team * TEAM + lane);
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) *reinterpret_cast<f64x2*>(mine + e) = f64x2{acc[e], acc[e + 1]};
+  lds_only_barrier();
+  const int used = r1 - r0 < T ? r1 - r0 : T;  // teams that had a row
+  f64x2* out = reinterpret_cast<f64x2*>(dw_part + static_cast<size_t>(blockIdx.x) * cols);
+  for (int q = threadIdx.x; q < cols / 2; q += kRowsThreads) {
+    f64x2 t = reinterpret_cast<const f64x2*>(dw_lds)[q];
+    for (int v = 1; v < used; ++v)
+      t += reinterpret_cast<const f64x2*>(dw_lds + v * (8 * TEAM))[q];
+    out[q] = t;
+  }
+}
+
 // SPLIT variant.  The workgroup is THREADS data lanes (VPT dwordx4 of x
 // and of dy per lane and row) plus one communication wave.  Member `member`
 // of group `group` (of G) covers rows group, group + G, group + 2G, ... and
@@ -829,21 +934,35 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_rowdot_kernel(
   if (threadIdx.x == 0) rowdot[row] = static_cast<float>(t);
 }
 
-// dw[c] = sum over blocks b (in order) of part[b][c], rounded once to fp32.
+// dw[c] = sum over blocks b of part[b][c], rounded once to fp32.  A workgroup
+// takes 32 columns: lane (q, s) adds blocks s, s + 16, ... of column pair q,
+// and the 16 sums are added in order, so the order is fixed.  Sixteen loads of
+// 256 bytes are in flight at once; one lane walking all blocks of its pair
+// took 26 us for 512 blocks x 8192 columns (16 workgroups).
 __global__ __launch_bounds__(256) void rmsnorm_dw_reduce_kernel(
     const double* __restrict__ part, float* __restrict__ dw, int blocks, int cols) {
-  const int q = blockIdx.x * 256 + threadIdx.x;  // two columns
+  __shared__ f64x2 sums[16][16];
+  const int lane = threadIdx.x & 15, s = threadIdx.x >> 4;
+  const int q = blockIdx.x * 16 + lane;  // column pair
   const int nq = cols >> 1;
-  if (q >= nq) return;
-  const f64x2* p = reinterpret_cast<const f64x2*>(part) + q;
-  double a0 = 0.0, a1 = 0.0;
-#pragma unroll 8
-  for (int b = 0; b < blocks; ++b) {
-    const f64x2 v = load_nt(p + static_cast<size_t>(b) * nq);
-    a0 += v.x;
-    a1 += v.y;
+  f64x2 a{0.0, 0.0};
+  if (q < nq) {
+    const f64x2* p = reinterpret_cast<const f64x2*>(part) + q;
+#pragma unroll 4
+    for (int b = s; b < blocks; b += 16) a += load_nt(p + static_cast<size_t>(b) * nq);
   }
-  reinterpret_cast<float2_t*>(dw)[q] = float2_t{static_cast<float>(a0), static_cast<float>(a1)};
+  sums[s][lane] = a;
+  __syncthreads();
+  if (s != 0 || q >= nq) return;
+#pragma unroll
+  for (int t = 1; t < 16; ++t) a += sums[t][lane];
+  reinterpret_cast<float2_t*>(dw)[q] = float2_t{static_cast<float>(a.x), static_cast<float>(a.y)};
+}
+
+int launch_dw_reduce(const double* part, float* dw, int64_t blocks, int cols, hipStream_t stream) {
+  rmsnorm_dw_reduce_kernel<<<dim3(static_cast<unsigned>((cols / 2 + 15) / 16)), dim3(256), 0,
+                             stream>>>(part, dw, static_cast<int>(blocks), cols);
+  return check_launch("rmsnorm_dw_reduce_kernel");
 }
 
 // ------------------------------------------------------------ dispatch ---
@@ -895,6 +1014,18 @@ const BwdPick kBwd[] = {
     {rmsnorm_bwd_slice_kernel<128, 2>, 128, 256},
     {rmsnorm_bwd_slice_kernel<256, 2>, 256, 512},
     {rmsnorm_bwd_slice_kernel<512, 2>, 512, 1024},
+};
+// STAGED rows: the narrowest team that holds the row.
+using BwdRowsFn = void (*)(const uint16_t*, const uint16_t*, const uint16_t*, const float*,
+                           uint16_t*, double*, int, int, int);
+struct BwdRowsPick {
+  BwdRowsFn fn;
+  int capacity;
+};
+const BwdRowsPick kBwdRows[] = {
+    {rmsnorm_bwd_rows_kernel<64>, 64},   {rmsnorm_bwd_rows_kernel<128>, 128},
+    {rmsnorm_bwd_rows_kernel<256>, 256}, {rmsnorm_bwd_rows_kernel<512>, 512},
+    {rmsnorm_bwd_rows_kernel<1024>, 1024},
 };
 // Group kernels: four row buffers per lane.  At one dwordx4 per lane
 // (~104 VGPRs: 4 waves per SIMD, 16 per CU; 64 bytes of LDS dw
@@ -1112,6 +1243,10 @@ int resolve_bwd(const credit_cfg* cfg, int64_t rows, int64_t cols, bool vec, int
       return set_error(CREDIT_ERR_BAD_SHAPE, "rmsnorm_bwd: %lld rows per group",
                        static_cast<long long>(r));
     plan->rows_per_group = static_cast<int>(r < 1 ? 1 : r);
+  } else if (plan->variant == CREDIT_VARIANT_STAGED) {
+    // One workgroup per CU, each with a block of rows; fewer rows, one each.
+    plan->rows_per_group = static_cast<int>((rows + cu_count - 1) / cu_count);
+    if (plan->rows_per_group < 1) plan->rows_per_group = 1;
   } else {
     plan->rows_per_group = rows_per_group_for(rows, plan->members, cu_count, 2);
   }
@@ -1430,6 +1565,22 @@ extern "C" int credit_rmsnorm_bwd_bf16(const uint16_t* x, const uint16_t* w,
                        make_split_args(ws, total, static_cast<uint32_t>(plan.rows_per_group),
                                        kBwdRing, dispensers));
     CREDIT_TRY(check_launch("rmsnorm_bwd_group_kernel"));
+  } else if (plan.variant == CREDIT_VARIANT_STAGED) {
+    static const hipError_t attr = [] {
+      hipError_t e = hipSuccess;
+      for (const BwdRowsPick& p : kBwdRows)
+        if (e == hipSuccess)
+          e = hipFuncSetAttribute(reinterpret_cast<const void*>(p.fn),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  static_cast<int>(kRowsLds));
+      return e;
+    }();
+    if (attr != hipSuccess)
+      return hip_failure(attr, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
+    hipLaunchKernelGGL(pick_for(kBwdRows, plan.chunk)->fn, dim3(total), dim3(kRowsThreads),
+                       kRowsLds, stream, x, w, dy, rstd, dx, dw_part, static_cast<int>(rows), c,
+                       plan.rows_per_group);
+    CREDIT_TRY(check_launch("rmsnorm_bwd_rows_kernel"));
   } else {
     const BwdPick* pick = pick_for(kBwd, plan.chunk);
     hipLaunchKernelGGL(pick->fn, dim3(total), dim3(pick->threads), pick->lds_bytes(), stream, x,
@@ -1438,10 +1589,7 @@ extern "C" int credit_rmsnorm_bwd_bf16(const uint16_t* x, const uint16_t* w,
                        SplitArgs{});
     CREDIT_TRY(check_launch("rmsnorm_bwd_slice_kernel"));
   }
-  const unsigned reduce_blocks = static_cast<unsigned>((cols / 2 + 255) / 256);
-  rmsnorm_dw_reduce_kernel<<<dim3(reduce_blocks), dim3(256), 0, stream>>>(
-      dw_part, dw, static_cast<int>(plan.groups), c);
-  return check_launch("rmsnorm_dw_reduce_kernel");
+  return launch_dw_reduce(dw_part, dw, plan.groups, c, stream);
 }
 
 extern "C" int credit_rmsnorm_bwd_bf16_noalloc(const uint16_t* x, const uint16_t* w,
@@ -1529,8 +1677,5 @@ extern "C" int credit_rmsnorm_fwd_bwd_bf16(const uint16_t* x, const uint16_t* w,
                      make_split_args(ws, total, static_cast<uint32_t>(plan.rows_per_group),
                                      kBwdRing, plan.dispensers));
   CREDIT_TRY(check_launch("rmsnorm_fused_group_kernel"));
-  const unsigned reduce_blocks = static_cast<unsigned>((cols / 2 + 255) / 256);
-  rmsnorm_dw_reduce_kernel<<<dim3(reduce_blocks), dim3(256), 0, stream>>>(
-      dw_part, dw, static_cast<int>(plan.groups), c);
-  return check_launch("rmsnorm_dw_reduce_kernel");
+  return launch_dw_reduce(dw_part, dw, plan.groups, c, stream);
 }

@@ -1,0 +1,48 @@
+"""RMSNorm backward of rows one team of lanes holds (STAGED, at most 8192
+columns): teams of 64 to 1024 lanes, blocks of rows from one to many, rows that
+do not divide among the teams or the row buffers.
+
+fp32 dw within rtol 1e-5 / atol 1e-6 and bf16 dx within rtol 1e-2 / atol 1e-2 of
+the float64 oracle given the same fp32 rstd."""
+import numpy as np
+import pytest
+import torch
+
+from credit_amd import hip_lib
+from credit_amd.workloads import WORKLOADS
+from oracle import reference as ref
+
+pytestmark = pytest.mark.gpu
+
+
+def backward(x, w, dy, rstd, gpu):
+    ins = [t.to(gpu) for t in (x, w, dy)]
+    dx = torch.full_like(ins[0], float("nan"))
+    dw = torch.full((x.shape[1],), float("nan"), device=gpu)
+    hip_lib.rmsnorm_bwd(*ins, torch.from_numpy(rstd).to(gpu), dx, dw, hip_lib.make_cfg("staged"))
+    torch.cuda.synchronize()
+    return dx.float().cpu().numpy(), dw.cpu().numpy()
+
+
+# cols: both edges of each team width; rows: one, one per CU and one more,
+# blocks shorter and longer than the row buffers of 1 to 16 teams.
+@pytest.mark.parametrize("rows,cols", [
+    (1, 8), (1, 8192), (256, 512), (257, 520), (513, 1024), (1025, 1032), (2300, 2048),
+    (1300, 2056), (771, 4096), (3000, 4104), (1281, 8192), (9000, 256)])
+def test_staged_backward(gpu, rows, cols):
+    print(f"rmsnorm_bwd rows {rows} x {cols}", flush=True)
+    x, w, dy = WORKLOADS["rmsnorm_fwd"].make_inputs(rows, cols, seed=rows + cols)
+    rstd = ref.rmsnorm_fwd(x.float().numpy(), np.ones(cols), 1.0e-6)[1].astype(np.float32)
+    dx, dw = backward(x, w, dy, rstd, gpu)
+    edx, edw = ref.rmsnorm_bwd(x.float().numpy(), w.float().numpy(), dy.float().numpy(), rstd)
+    np.testing.assert_allclose(dw, edw, rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(dx, edx, rtol=1e-2, atol=1e-2)
+
+
+def test_staged_backward_keeps_an_infinite_rstd_to_its_row(gpu):
+    """rstd = inf in a block's first row: dw is infinite where dy * x is not
+    zero, and the row buffers past the block add nothing to it; dx of that row
+    is inf * (1 - 1 * inf * inf) = -inf."""
+    x, w, dy = (torch.ones_like(t) for t in WORKLOADS["rmsnorm_fwd"].make_inputs(2, 1024, seed=3))
+    dx, dw = backward(x, w, dy, np.array([np.inf, 1.0], np.float32), gpu)
+    assert np.all(np.isposinf(dw)) and np.all(np.isneginf(dx[0])) and np.all(np.isfinite(dx[1]))

@@ -278,8 +278,10 @@ struct SplitShape {
 };
 thread_local SplitShape g_last_split;
 
-int coresident_groups(const void* kernel, int threads, size_t dynamic_lds, int members,
-                      int64_t* groups, int* dispensers) {
+namespace {
+// Workgroups per CU and static LDS of a kernel on the current device.
+int occupancy(const void* kernel, int threads, size_t dynamic_lds, int* per_cu_out,
+              size_t* static_lds_out) {
   struct Entry {
     int device;
     const void* kernel;
@@ -311,6 +313,27 @@ int coresident_groups(const void* kernel, int threads, size_t dynamic_lds, int m
     std::lock_guard<std::mutex> lock(mu);
     cache.push_back(Entry{dev, kernel, threads, dynamic_lds, per_cu, static_lds});
   }
+  *per_cu_out = per_cu;
+  *static_lds_out = static_lds;
+  return CREDIT_OK;
+}
+}  // namespace
+
+int resident_workgroups(const void* kernel, int threads, size_t dynamic_lds, int64_t* count) {
+  int per_cu = 0;
+  size_t static_lds = 0;
+  CREDIT_TRY(occupancy(kernel, threads, dynamic_lds, &per_cu, &static_lds));
+  const DeviceProps* props = nullptr;
+  CREDIT_TRY(current_device_props(&props));
+  *count = static_cast<int64_t>(per_cu > 0 ? per_cu : 1) * props->cu_count;
+  return CREDIT_OK;
+}
+
+int coresident_groups(const void* kernel, int threads, size_t dynamic_lds, int members,
+                      int64_t* groups, int* dispensers) {
+  int per_cu = 0;
+  size_t static_lds = 0;
+  CREDIT_TRY(occupancy(kernel, threads, dynamic_lds, &per_cu, &static_lds));
   const DeviceProps* props = nullptr;
   CREDIT_TRY(current_device_props(&props));
   const int64_t resident = static_cast<int64_t>(per_cu) * props->cu_count;

@@ -191,6 +191,9 @@ char* noalloc_scratch_base(int device);
 // slots hold at least two groups: no group spans every slot of its subset.
 int coresident_groups(const void* kernel, int threads, size_t dynamic_lds, int members,
                       int64_t* groups, int* dispensers = nullptr);
+// Workgroups of `kernel` the device holds at once (queried once per device
+// and kernel): the grid of a kernel whose workgroups loop over rows.
+int resident_workgroups(const void* kernel, int threads, size_t dynamic_lds, int64_t* count);
 // Dispenser subsets of a launch of `groups` x `members` of a kernel with
 // `per_cu` workgroups resident per CU (plan::dispensers_for).
 int split_dispensers(int per_cu, int cu_count, int members);

@@ -131,6 +131,16 @@ __device__ __forceinline__ double wave_reduce_sum_f64(double v) {
   return (a + b) + (c + d);
 }
 
+// Workgroup barrier for LDS only: this wave's LDS operations complete
+// (lgkmcnt(0)), then s_barrier; signal fences keep the compiler from moving
+// memory operations across it.  Vector-memory loads stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), vmcnt and expcnt at their maxima
+  __builtin_amdgcn_s_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
 // ------------------------------------------------------ block reductions --
 // One LDS round: each wave deposits its wave-uniform value, one barrier, then
 // every thread folds the NW slots in slot order.  Callers pass a distinct

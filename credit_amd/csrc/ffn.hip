@@ -243,16 +243,6 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt(((N >> 4) << 14) | (0xF << 8) | (0x7 << 4) | (N & 15));
 }
 
-// Workgroup barrier for LDS only: this wave's LDS operations complete
-// (lgkmcnt(0)), then s_barrier; signal fences keep the compiler from moving
-// memory operations across it.  Vector-memory loads stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), vmcnt and expcnt at their maxima
-  __builtin_amdgcn_s_barrier();
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
 // One LDS-direct load: 16 bytes per lane from rsrc at voff + soff into LDS
 // at M0 = m0base + QOFF + 16 * lane.  s_nop covers the M0 write -> LDS-DMA
 // hazard.  M0 is a reserved register to the compiler, which warns that it

@@ -22,6 +22,7 @@
 // Algorithmic traffic per row: 4*cols (x) + cols (q) + 4 (scale) bytes.
 #include "api_internal.hpp"
 #include "common.hpp"
+#include "rows.hpp"
 #include "slices.hpp"
 
 namespace credit {
@@ -96,39 +97,90 @@ __global__ __launch_bounds__(THREADS) void rowwise_quant_slice_kernel(
   split_leave(sa);
 }
 
-// Two passes over the row; VEC: f32x4 loads and 4-byte q stores.
-template <int THREADS, bool VEC>
+// The four codes of a vector, at any address.
+__device__ __forceinline__ void store_codes(int8_t* q, uint32_t codes) {
+  __builtin_memcpy(q, &codes, 4);
+}
+__device__ __forceinline__ int8_t code1(float x, float inv) {
+  return static_cast<int8_t>(static_cast<int32_t>(quant1(x, inv) << 24) >> 24);
+}
+
+// Ragged rows (rows.hpp) held in one workgroup's registers: x read once.
+template <int THREADS, int VPT>
+__global__ __launch_bounds__(THREADS) void rowwise_quant_rows_kernel(
+    const float* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scale, int rows,
+    int cols) {
+  constexpr int NW = THREADS / kWave;
+  __shared__ float mred[2][NW];
+  const int tid = threadIdx.x;
+  const int G = gridDim.x;
+  const uint32_t off = static_cast<uint32_t>(tid) * 16u;
+  constexpr uint32_t kStride = THREADS * 16u;
+  f32x4 v[VPT];
+  int row = blockIdx.x;
+  const buffer_rsrc_t xr = rows::row_rsrc(x, row, rows, cols);
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) v[k] = rows::row_load(xr, off + k * kStride);
+  for (int par = 0; row < rows; row += G, par ^= 1) {
+    float lm = 0.0f;  // |x| >= 0, and past the row's end x reads 0
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) lm = fmax_nan(lm, absmax4(v[k]));
+    const float m = rows::block_max<NW>(lm, mred[par]);
+    const float inv = inv_scale(m);
+    int8_t* qr = q + static_cast<size_t>(row) * cols + 4 * tid;
+    int left = cols - 4 * tid;
+    __asm__ volatile("" : "+v"(left));  // masks formed per row, not kept across rows
+    const buffer_rsrc_t xn = rows::row_rsrc(x, row + G, rows, cols);
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+      const int n = left - 4 * k * THREADS;
+      int8_t* qk = qr + 4 * k * THREADS;
+      if (n >= 4) {
+        store_codes(qk, quant4(v[k], inv));
+      } else {
+        if (n > 0) qk[0] = code1(v[k].x, inv);
+        if (n > 1) qk[1] = code1(v[k].y, inv);
+        if (n > 2) qk[2] = code1(v[k].z, inv);
+      }
+      v[k] = rows::row_load(xn, off + k * kStride);
+    }
+    if (tid == 0) scale[row] = m / 127.0f;
+  }
+}
+
+// Two passes over the row, at any width and address.
+template <int THREADS>
 __global__ __launch_bounds__(THREADS) void rowwise_quant_read_kernel(
     const float* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scale, int cols) {
   constexpr int NW = THREADS / kWave;
   __shared__ float mred[NW];
   const int tid = threadIdx.x;
   const size_t off = static_cast<size_t>(blockIdx.x) * cols;
+  const float* xr = x + off;
   float lm = 0.0f;
-  if (VEC) {
-    const int nvec = cols >> 2;
-    const f32x4* xv = reinterpret_cast<const f32x4*>(x + off);
-    int i = tid;
-    for (; i + THREADS < nvec; i += 2 * THREADS)
-      lm = fmax_nan(lm, fmax_nan(absmax4(load_nt(xv + i)), absmax4(load_nt(xv + i + THREADS))));
-    for (; i < nvec; i += THREADS) lm = fmax_nan(lm, absmax4(load_nt(xv + i)));
-  } else {
-    for (int c = tid; c < cols; c += THREADS) lm = fmax_nan(lm, __builtin_fabsf(x[off + c]));
-  }
+  const int nvec = cols >> 2;
+  int i = tid;
+  for (; i + THREADS < nvec; i += 2 * THREADS)
+    lm = fmax_nan(lm, fmax_nan(absmax4(rows::stream_load(xr, i)),
+                               absmax4(rows::stream_load(xr, i + THREADS))));
+  for (; i < nvec; i += THREADS) lm = fmax_nan(lm, absmax4(rows::stream_load(xr, i)));
+  for (int c = 4 * nvec + tid; c < cols; c += THREADS)
+    lm = fmax_nan(lm, __builtin_fabsf(xr[c]));
   const float m = block_reduce<NW>(lm, MaxOp{}, mred);
   const float inv = inv_scale(m);
-  if (VEC) {
-    const int nvec = cols >> 2;
-    const f32x4* xv = reinterpret_cast<const f32x4*>(x + off);
-    uint32_t* qv = reinterpret_cast<uint32_t*>(q + off);
-    for (int i = tid; i < nvec; i += THREADS) __builtin_nontemporal_store(quant4(load_nt(xv + i), inv), qv + i);
-  } else {
-    for (int c = tid; c < cols; c += THREADS)
-      q[off + c] = static_cast<int8_t>(static_cast<int32_t>(quant1(x[off + c], inv) << 24) >> 24);
-  }
+  for (i = tid; i < nvec; i += THREADS)
+    store_codes(q + off + 4 * static_cast<size_t>(i), quant4(rows::stream_load(xr, i), inv));
+  for (int c = 4 * nvec + tid; c < cols; c += THREADS) q[off + c] = code1(xr[c], inv);
   if (tid == 0) scale[blockIdx.x] = m / 127.0f;
 }
 
+using QuantRowsFn = void (*)(const float*, int8_t*, float*, int, int);
+const rows::RowsPick<QuantRowsFn> kQuantRows[] = {
+    {rowwise_quant_rows_kernel<64, 4>, 64, 1024},    {rowwise_quant_rows_kernel<128, 4>, 128, 2048},
+    {rowwise_quant_rows_kernel<256, 4>, 256, 4096},  {rowwise_quant_rows_kernel<256, 8>, 256, 8192},
+    {rowwise_quant_rows_kernel<512, 8>, 512, 16384}, {rowwise_quant_rows_kernel<512, 16>, 512, 32768},
+    {rowwise_quant_rows_kernel<512, 32>, 512, 65536},
+};
 using QuantFn = void (*)(const float*, int8_t*, float*, int, int, int, int, SplitArgs);
 
 // One tensor staged: up to 16 f32x4 per lane (as the softmax forward).
@@ -172,16 +224,25 @@ extern "C" int credit_rowwise_quant_f32(const float* x, int8_t* q, float* scale,
   CREDIT_TRY(check_cfg(cfg));
   if (rows == 0) return CREDIT_OK;
   const bool vec = quant_vec(cols, x, q);
-  Plan plan;
-  CREDIT_TRY(resolve(cfg, cols, vec, kQuantCapacity, "rowwise_quant", &plan));
   hipStream_t stream = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
+  if (!vec && cfg_variant(cfg) == CREDIT_VARIANT_AUTO && rows <= (int64_t{1} << 30)) {
+    if (const auto* pick = rows::rows_pick(kQuantRows, cols)) {
+      unsigned grid = 0;
+      CREDIT_TRY(rows::rows_grid(*pick, rows, &grid));
+      hipLaunchKernelGGL(pick->fn, dim3(grid), dim3(pick->threads), 0, stream, x, q, scale,
+                         static_cast<int>(rows), c);
+      return check_launch("rowwise_quant_rows_kernel");
+    }
+  }
+  Plan plan;
+  CREDIT_TRY(resolve(cfg, cols, vec, kQuantCapacity, "rowwise_quant", &plan));
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (vec)
-      rowwise_quant_read_kernel<256, true><<<r, 256, 0, stream>>>(x, q, scale, c);
+    if (rows::stream_threads(rows) == 1024)
+      rowwise_quant_read_kernel<1024><<<r, 1024, 0, stream>>>(x, q, scale, c);
     else
-      rowwise_quant_read_kernel<256, false><<<r, 256, 0, stream>>>(x, q, scale, c);
+      rowwise_quant_read_kernel<256><<<r, 256, 0, stream>>>(x, q, scale, c);
     return check_launch("rowwise_quant_read_kernel");
   }
   const Pick<QuantFn>* pk = pick_for(kQuant, plan.chunk);

@@ -347,14 +347,6 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_slice_kernel(
 constexpr int kRowsThreads = 1024;
 constexpr size_t kRowsLds = size_t{kRowsThreads} * 8 * sizeof(double);  // 64 KiB
 
-// Workgroup barrier for LDS only: loads and stores in flight stay so.
-__device__ __forceinline__ void lds_only_barrier() {
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), vmcnt and expcnt at their maxima
-  __builtin_amdgcn_s_barrier();
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
 template <int TEAM>
 __global__ __launch_bounds__(kRowsThreads) void rmsnorm_bwd_rows_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
@@ -393,7 +385,7 @@ __global__ __launch_bounds__(kRowsThreads) void rmsnorm_bwd_rows_kernel(
     load(ahead, r + 3 * T);
     const double ws = wave_reduce_sum_f64(static_cast<double>(gx8(cur.x, cur.dy, wv)));
     if (threadIdx.x % kWave == 0) red[parity][team][wave] = ws;
-    lds_only_barrier();
+    lds_barrier();
     double dot = red[parity][team][0];
 #pragma unroll
     for (int v = 1; v < NW; ++v) dot += red[parity][team][v];
@@ -427,7 +419,7 @@ __global__ __launch_bounds__(kRowsThreads) void rmsnorm_bwd_rows_kernel(
   double* mine = dw_lds + 8 * (team * TEAM + lane);
 #pragma unroll
   for (int e = 0; e < 8; e += 2) *reinterpret_cast<f64x2*>(mine + e) = f64x2{acc[e], acc[e + 1]};
-  lds_only_barrier();
+  lds_barrier();
   const int used = r1 - r0 < T ? r1 - r0 : T;  // teams that had a row
   f64x2* out = reinterpret_cast<f64x2*>(dw_part + static_cast<size_t>(blockIdx.x) * cols);
   for (int q = threadIdx.x; q < cols / 2; q += kRowsThreads) {

@@ -23,6 +23,7 @@
 
 #include "api_internal.hpp"
 #include "common.hpp"
+#include "rows.hpp"
 #include "slices.hpp"
 
 namespace credit {
@@ -637,9 +638,94 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void softmax_bwd_group_kernel(
   split_leave(sa);
 }
 
-// Streaming forward: online (max, sum) pass, then the output pass.  VEC:
-// f32x4 loads (cols % 4 == 0, 16-byte aligned rows); else element loads.
-template <int THREADS, bool VEC>
+// ------------------------------------------------------- ragged rows -----
+// Rows that no 16-byte layout fits (rows.hpp), one row per workgroup held in
+// registers: x (and dy) are read once and the output written once, where READ
+// streams x three times in 4-byte loads.  Two or three LDS reductions per row
+// (max; sum; sum p dy), the exponentials taken about the row's own maximum and
+// summed in fp64.  logits_backward at 1024 x 50001: 391 -> 140 us (4.4 TB/s).
+constexpr int kOpFwd = 0, kOpBwd = 1, kOpLogits = 2;
+
+template <int OP, int THREADS, int VPT>
+__global__ __launch_bounds__(THREADS) void softmax_rows_kernel(
+    const float* __restrict__ a, const float* __restrict__ dy, float* __restrict__ out,
+    float* __restrict__ rowmax, float* __restrict__ lse, int rows, int cols) {
+  constexpr int NW = THREADS / kWave;
+  constexpr bool kSoft = OP != kOpBwd, kGrad = OP != kOpFwd;
+  __shared__ float mslots[NW];
+  __shared__ double sslots[2][NW];
+  const int tid = threadIdx.x;
+  const int G = gridDim.x;
+  const uint32_t off = static_cast<uint32_t>(tid) * 16u;
+  constexpr uint32_t kStride = THREADS * 16u;
+  int left = cols - 4 * tid;  // elements from the lane's first vector on
+  f32x4 v[VPT], d[kGrad ? VPT : 1];
+  int row = blockIdx.x;
+  {
+    const buffer_rsrc_t ar = rows::row_rsrc(a, row, rows, cols);
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) v[k] = rows::row_load(ar, off + k * kStride);
+    if constexpr (kGrad) {
+      const buffer_rsrc_t dr = rows::row_rsrc(dy, row, rows, cols);
+#pragma unroll
+      for (int k = 0; k < VPT; ++k) d[k] = rows::row_load(dr, off + k * kStride);
+    }
+  }
+  // The slots of one row's reductions are rewritten in the next row's, two
+  // barriers later; kOpBwd has one reduction per row and alternates.
+  for (int par = 0; row < rows; row += G, par ^= 1) {
+    float inv_s = 1.0f;
+    if constexpr (kSoft) {
+      float lm = kNegInf;
+      // Opaque: the lanes' masks are formed anew in each pass, not kept in
+      // scalar registers (8 per vector) across the rows.
+      __asm__ volatile("" : "+v"(left));
+#pragma unroll
+      for (int k = 0; k < VPT; ++k)
+        lm = fmax_nan(lm, max4(rows::keep4(v[k], left - 4 * k * THREADS, kNegInf)));
+      const float m = rows::block_max<NW>(lm, mslots);
+      double ls = 0.0;
+      __asm__ volatile("" : "+v"(left));
+#pragma unroll
+      for (int k = 0; k < VPT; ++k) {
+        v[k] = rows::keep4(prob4(v[k], m, 1.0f), left - 4 * k * THREADS, 0.0f);
+        ls += (static_cast<double>(v[k].x) + v[k].y) + (static_cast<double>(v[k].z) + v[k].w);
+      }
+      const double s = rows::block_sum<NW>(m == kNegInf ? 0.0 : ls, sslots[0]);
+      inv_s = static_cast<float>(1.0 / s);
+      if (OP == kOpFwd && tid == 0) {
+        rowmax[row] = m;
+        lse[row] = static_cast<float>(static_cast<double>(m) + ::log(s));
+      }
+    }
+    float dot = 0.0f;
+    if constexpr (kGrad) {
+      double acc = 0.0;
+#pragma unroll
+      for (int k = 0; k < VPT; ++k) {
+        if (kSoft) v[k] = v[k] * inv_s;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc += static_cast<double>(v[k][e] * d[k][e]);
+      }
+      dot = static_cast<float>(rows::block_sum<NW>(acc, sslots[kSoft ? 1 : par]));
+    }
+    const buffer_rsrc_t orow = rows::row_rsrc(out, row, rows, cols);
+    const buffer_rsrc_t an = rows::row_rsrc(a, row + G, rows, cols);
+    const buffer_rsrc_t dn = rows::row_rsrc(kGrad ? dy : a, row + G, rows, cols);
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+      rows::row_store(orow, off + k * kStride,
+                      kGrad ? grad4(v[k], d[kGrad ? k : 0], dot) : v[k] * inv_s);
+      v[k] = rows::row_load(an, off + k * kStride);
+      if constexpr (kGrad) d[k] = rows::row_load(dn, off + k * kStride);
+    }
+  }
+}
+
+// Streaming forward: online (max, sum) pass, then the output pass, in vectors
+// at any 4-byte address with a tail of single elements (4-byte loads
+// throughout ran 1 x 250001 at 12 GB/s).
+template <int THREADS>
 __global__ __launch_bounds__(THREADS) void softmax_fwd_read_kernel(
     const float* __restrict__ x, float* __restrict__ p, float* __restrict__ rowmax,
     float* __restrict__ lse, int cols) {
@@ -652,48 +738,40 @@ __global__ __launch_bounds__(THREADS) void softmax_fwd_read_kernel(
   float* pr = p + static_cast<size_t>(row) * cols;
   float m = kNegInf;  // running max of the finite path
   double s = 0.0;     // sum of e^(x - m)
-  if (VEC) {
-    const int nvec = cols >> 2;
-    const f32x4* xv = reinterpret_cast<const f32x4*>(xr);
-    int i = tid;
-    for (; i + THREADS < nvec; i += 2 * THREADS) {
-      const f32x4 a = load_nt(xv + i), b = load_nt(xv + i + THREADS);
-      online_update(fmax_nan(max4(a), max4(b)), m, s);
-      if (m != kNegInf) s += static_cast<double>(sumexp4(a, m) + sumexp4(b, m));
-    }
-    for (; i < nvec; i += THREADS) {
-      const f32x4 a = load_nt(xv + i);
-      online_update(max4(a), m, s);
-      if (m != kNegInf) s += static_cast<double>(sumexp4(a, m));
-    }
-  } else {
-    for (int c = tid; c < cols; c += THREADS) {
-      const float v = xr[c];
-      online_update(v, m, s);
-      if (m != kNegInf) s += static_cast<double>(exp_accurate(v - m));
-    }
+  const int nvec = cols >> 2;
+  int i = tid;
+  for (; i + THREADS < nvec; i += 2 * THREADS) {
+    const f32x4 a = rows::stream_load(xr, i), b = rows::stream_load(xr, i + THREADS);
+    online_update(fmax_nan(max4(a), max4(b)), m, s);
+    if (m != kNegInf) s += static_cast<double>(sumexp4(a, m) + sumexp4(b, m));
+  }
+  for (; i < nvec; i += THREADS) {
+    const f32x4 a = rows::stream_load(xr, i);
+    online_update(max4(a), m, s);
+    if (m != kNegInf) s += static_cast<double>(sumexp4(a, m));
+  }
+  for (int c = 4 * nvec + tid; c < cols; c += THREADS) {
+    const float v = xr[c];
+    online_update(v, m, s);
+    if (m != kNegInf) s += static_cast<double>(exp_accurate(v - m));
   }
   float M;
   double S;
   block_maxsum<NW>(m, s, mred, sred, &M, &S);
   const float inv_s = static_cast<float>(1.0 / S);
-  if (VEC) {
-    const int nvec = cols >> 2;
-    const f32x4* xv = reinterpret_cast<const f32x4*>(xr);
-    f32x4* pv = reinterpret_cast<f32x4*>(pr);
-    int i = tid;
-    for (; i + 3 * THREADS < nvec; i += 4 * THREADS) {
-      const f32x4 a = load_nt(xv + i), b = load_nt(xv + i + THREADS),
-                  c = load_nt(xv + i + 2 * THREADS), d = load_nt(xv + i + 3 * THREADS);
-      store_nt(pv + i, prob4(a, M, inv_s));
-      store_nt(pv + i + THREADS, prob4(b, M, inv_s));
-      store_nt(pv + i + 2 * THREADS, prob4(c, M, inv_s));
-      store_nt(pv + i + 3 * THREADS, prob4(d, M, inv_s));
-    }
-    for (; i < nvec; i += THREADS) store_nt(pv + i, prob4(load_nt(xv + i), M, inv_s));
-  } else {
-    for (int c = tid; c < cols; c += THREADS) pr[c] = exp_accurate(xr[c] - M) * inv_s;
+  i = tid;
+  for (; i + 3 * THREADS < nvec; i += 4 * THREADS) {
+    const f32x4 a = rows::stream_load(xr, i), b = rows::stream_load(xr, i + THREADS),
+                c = rows::stream_load(xr, i + 2 * THREADS),
+                d = rows::stream_load(xr, i + 3 * THREADS);
+    rows::stream_store(pr, i, prob4(a, M, inv_s));
+    rows::stream_store(pr, i + THREADS, prob4(b, M, inv_s));
+    rows::stream_store(pr, i + 2 * THREADS, prob4(c, M, inv_s));
+    rows::stream_store(pr, i + 3 * THREADS, prob4(d, M, inv_s));
   }
+  for (; i < nvec; i += THREADS)
+    rows::stream_store(pr, i, prob4(rows::stream_load(xr, i), M, inv_s));
+  for (int c = 4 * nvec + tid; c < cols; c += THREADS) pr[c] = exp_accurate(xr[c] - M) * inv_s;
   if (tid == 0) {
     // rowmax must carry NaN like torch.amax: S is NaN exactly when the row
     // holds a NaN.
@@ -748,45 +826,38 @@ __global__ __launch_bounds__(THREADS) void softmax_bwd_slice_kernel(
   split_leave(sa);
 }
 
-template <int THREADS, bool VEC>
+template <int THREADS>
 __global__ __launch_bounds__(THREADS) void softmax_bwd_read_kernel(
     const float* __restrict__ p, const float* __restrict__ dy, float* __restrict__ dx, int cols) {
   constexpr int NW = THREADS / kWave;
   __shared__ double sred[NW];
   const int tid = threadIdx.x;
   const size_t off = static_cast<size_t>(blockIdx.x) * cols;
+  const float* pr = p + off;
+  const float* dr = dy + off;
   double acc = 0.0;
-  if (VEC) {
-    const int nvec = cols >> 2;
-    const f32x4* pv = reinterpret_cast<const f32x4*>(p + off);
-    const f32x4* dv = reinterpret_cast<const f32x4*>(dy + off);
-    int i = tid;
-    for (; i + THREADS < nvec; i += 2 * THREADS) {
-      const f32x4 a = load_nt(pv + i), b = load_nt(pv + i + THREADS);
-      const f32x4 da = load_nt(dv + i), db = load_nt(dv + i + THREADS);
-      acc += static_cast<double>(dot4(a, da) + dot4(b, db));
-    }
-    for (; i < nvec; i += THREADS) acc += static_cast<double>(dot4(load_nt(pv + i), load_nt(dv + i)));
-  } else {
-    for (int c = tid; c < cols; c += THREADS) acc += static_cast<double>(p[off + c] * dy[off + c]);
+  const int nvec = cols >> 2;
+  int i = tid;
+  for (; i + THREADS < nvec; i += 2 * THREADS) {
+    const f32x4 a = rows::stream_load(pr, i), b = rows::stream_load(pr, i + THREADS);
+    const f32x4 da = rows::stream_load(dr, i), db = rows::stream_load(dr, i + THREADS);
+    acc += static_cast<double>(dot4(a, da) + dot4(b, db));
   }
+  for (; i < nvec; i += THREADS)
+    acc += static_cast<double>(dot4(rows::stream_load(pr, i), rows::stream_load(dr, i)));
+  for (int c = 4 * nvec + tid; c < cols; c += THREADS)
+    acc += static_cast<double>(pr[c] * dr[c]);
   const float d = static_cast<float>(block_reduce_sum_f64<NW>(acc, sred));
-  if (VEC) {
-    const int nvec = cols >> 2;
-    const f32x4* pv = reinterpret_cast<const f32x4*>(p + off);
-    const f32x4* dv = reinterpret_cast<const f32x4*>(dy + off);
-    f32x4* xv = reinterpret_cast<f32x4*>(dx + off);
-    int i = tid;
-    for (; i + THREADS < nvec; i += 2 * THREADS) {
-      const f32x4 a = load_nt(pv + i), b = load_nt(pv + i + THREADS);
-      const f32x4 da = load_nt(dv + i), db = load_nt(dv + i + THREADS);
-      store_nt(xv + i, grad4(a, da, d));
-      store_nt(xv + i + THREADS, grad4(b, db, d));
-    }
-    for (; i < nvec; i += THREADS) store_nt(xv + i, grad4(load_nt(pv + i), load_nt(dv + i), d));
-  } else {
-    for (int c = tid; c < cols; c += THREADS) dx[off + c] = p[off + c] * (dy[off + c] - d);
+  i = tid;
+  for (; i + THREADS < nvec; i += 2 * THREADS) {
+    const f32x4 a = rows::stream_load(pr, i), b = rows::stream_load(pr, i + THREADS);
+    const f32x4 da = rows::stream_load(dr, i), db = rows::stream_load(dr, i + THREADS);
+    rows::stream_store(dx + off, i, grad4(a, da, d));
+    rows::stream_store(dx + off, i + THREADS, grad4(b, db, d));
   }
+  for (; i < nvec; i += THREADS)
+    rows::stream_store(dx + off, i, grad4(rows::stream_load(pr, i), rows::stream_load(dr, i), d));
+  for (int c = 4 * nvec + tid; c < cols; c += THREADS) dx[off + c] = pr[c] * (dr[c] - d);
 }
 
 // ------------------------------------------- softmax-logits backward ----
@@ -886,7 +957,7 @@ __global__ __launch_bounds__(THREADS) void softmax_logits_bwd_slice_kernel(
 
 // Streaming logits backward: online (max, sum) over the logits; sum p*dy
 // (re-reading logits and dy); output pass (re-reading both again).
-template <int THREADS, bool VEC>
+template <int THREADS>
 __global__ __launch_bounds__(THREADS) void softmax_logits_bwd_read_kernel(
     const float* __restrict__ logits, const float* __restrict__ dy, float* __restrict__ dx,
     int cols) {
@@ -900,45 +971,33 @@ __global__ __launch_bounds__(THREADS) void softmax_logits_bwd_read_kernel(
   float m = kNegInf;
   double s = 0.0;
   const int nvec = cols >> 2;
-  if (VEC) {
-    const f32x4* lv = reinterpret_cast<const f32x4*>(lr);
-    for (int i = tid; i < nvec; i += THREADS) {
-      const f32x4 a = load_nt(lv + i);
-      online_update(max4(a), m, s);
-      if (m != kNegInf) s += static_cast<double>(sumexp4(a, m));
-    }
-  } else {
-    for (int c = tid; c < cols; c += THREADS) {
-      const float v = lr[c];
-      online_update(v, m, s);
-      if (m != kNegInf) s += static_cast<double>(exp_accurate(v - m));
-    }
+  for (int i = tid; i < nvec; i += THREADS) {
+    const f32x4 a = rows::stream_load(lr, i);
+    online_update(max4(a), m, s);
+    if (m != kNegInf) s += static_cast<double>(sumexp4(a, m));
+  }
+  for (int c = 4 * nvec + tid; c < cols; c += THREADS) {
+    const float v = lr[c];
+    online_update(v, m, s);
+    if (m != kNegInf) s += static_cast<double>(exp_accurate(v - m));
   }
   float M;
   double S;
   block_maxsum<NW>(m, s, mred, sred[0], &M, &S);
   const float inv_s = static_cast<float>(1.0 / S);
   double acc = 0.0;
-  if (VEC) {
-    const f32x4* lv = reinterpret_cast<const f32x4*>(lr);
-    const f32x4* dv = reinterpret_cast<const f32x4*>(dr);
-    for (int i = tid; i < nvec; i += THREADS)
-      acc += static_cast<double>(dot4(prob4(load_nt(lv + i), M, inv_s), load_nt(dv + i)));
-  } else {
-    for (int c = tid; c < cols; c += THREADS)
-      acc += static_cast<double>(exp_accurate(lr[c] - M) * inv_s * dr[c]);
-  }
+  for (int i = tid; i < nvec; i += THREADS)
+    acc += static_cast<double>(
+        dot4(prob4(rows::stream_load(lr, i), M, inv_s), rows::stream_load(dr, i)));
+  for (int c = 4 * nvec + tid; c < cols; c += THREADS)
+    acc += static_cast<double>(exp_accurate(lr[c] - M) * inv_s * dr[c]);
   const float d = static_cast<float>(block_reduce_sum_f64<NW>(acc, sred[1]));
-  if (VEC) {
-    const f32x4* lv = reinterpret_cast<const f32x4*>(lr);
-    const f32x4* dv = reinterpret_cast<const f32x4*>(dr);
-    f32x4* xv = reinterpret_cast<f32x4*>(dx + off);
-    for (int i = tid; i < nvec; i += THREADS)
-      store_nt(xv + i, grad4(prob4(load_nt(lv + i), M, inv_s), load_nt(dv + i), d));
-  } else {
-    for (int c = tid; c < cols; c += THREADS)
-      dx[off + c] = exp_accurate(lr[c] - M) * inv_s * (dr[c] - d);
-  }
+  for (int i = tid; i < nvec; i += THREADS)
+    rows::stream_store(dx + off, i,
+                       grad4(prob4(rows::stream_load(lr, i), M, inv_s), rows::stream_load(dr, i),
+                             d));
+  for (int c = 4 * nvec + tid; c < cols; c += THREADS)
+    dx[off + c] = exp_accurate(lr[c] - M) * inv_s * (dr[c] - d);
 }
 
 // ------------------------------------------------------------ dispatch ---
@@ -972,6 +1031,36 @@ const Pick<BwdFn> kLogits[] = {
     {softmax_logits_bwd_slice_kernel<512, 8>, 512, 4096},
     {softmax_logits_bwd_slice_kernel<1024, 8>, 1024, 8192},
 };
+
+// Ragged rows: 4 to 32 f32x4 per lane and tensor.
+using RowsFn = void (*)(const float*, const float*, float*, float*, float*, int, int);
+#define CREDIT_ROWS_TABLE(OP, LAST)                                                     \
+  {{softmax_rows_kernel<OP, 64, 4>, 64, 1024},    {softmax_rows_kernel<OP, 128, 4>, 128, 2048}, \
+   {softmax_rows_kernel<OP, 256, 4>, 256, 4096},  {softmax_rows_kernel<OP, 256, 8>, 256, 8192}, \
+   {softmax_rows_kernel<OP, 512, 8>, 512, 16384}, {softmax_rows_kernel<OP, 512, 16>, 512, 32768}, \
+   {softmax_rows_kernel<OP, 512, LAST>, 512, 2048 * LAST}}
+const rows::RowsPick<RowsFn> kFwdRows[] = CREDIT_ROWS_TABLE(kOpFwd, 32);
+const rows::RowsPick<RowsFn> kBwdRows[] = CREDIT_ROWS_TABLE(kOpBwd, 26);
+const rows::RowsPick<RowsFn> kLogitsRows[] = CREDIT_ROWS_TABLE(kOpLogits, 26);
+#undef CREDIT_ROWS_TABLE
+
+// AUTO on a shape without the 16-byte layout: the rows kernel that holds the
+// row.  nullptr: READ (explicit, or wider rows).
+template <int N>
+const rows::RowsPick<RowsFn>* ragged_pick(const rows::RowsPick<RowsFn> (&table)[N],
+                                          const credit_cfg* cfg, int64_t rows, int64_t cols,
+                                          bool vec) {
+  if (vec || cfg_variant(cfg) != CREDIT_VARIANT_AUTO || rows > (int64_t{1} << 30)) return nullptr;
+  return rows::rows_pick(table, cols);
+}
+int launch_rows(const rows::RowsPick<RowsFn>& pick, const float* a, const float* dy, float* out,
+                float* rowmax, float* lse, int64_t rows, int64_t cols, hipStream_t stream) {
+  unsigned grid = 0;
+  CREDIT_TRY(rows::rows_grid(pick, rows, &grid));
+  hipLaunchKernelGGL(pick.fn, dim3(grid), dim3(pick.threads), 0, stream, a, dy, out, rowmax, lse,
+                     static_cast<int>(rows), static_cast<int>(cols));
+  return check_launch("softmax_rows_kernel");
+}
 
 using BwdGroupFn = void (*)(const float*, const float*, float*, int, int, int, int, int,
                             SplitArgs);
@@ -1123,16 +1212,19 @@ extern "C" int credit_softmax_fwd_f32(const float* x, float* p, float* rowmax, f
   CREDIT_TRY(check_aligned(p, 4, "p"));
   CREDIT_TRY(check_cfg(cfg));
   if (rows == 0) return CREDIT_OK;
-  Plan plan;
-  CREDIT_TRY(resolve_fwd(cfg, cols, vec_ok(cols, {x, p}), &plan));
+  const bool vec = vec_ok(cols, {x, p});
   hipStream_t stream = cfg_stream(cfg);
+  if (const auto* pick = ragged_pick(kFwdRows, cfg, rows, cols, vec))
+    return launch_rows(*pick, x, nullptr, p, rowmax, lse, rows, cols, stream);
+  Plan plan;
+  CREDIT_TRY(resolve_fwd(cfg, cols, vec, &plan));
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (vec_ok(cols, {x, p}))
-      softmax_fwd_read_kernel<256, true><<<r, 256, 0, stream>>>(x, p, rowmax, lse, c);
+    if (rows::stream_threads(rows) == 1024)
+      softmax_fwd_read_kernel<1024><<<r, 1024, 0, stream>>>(x, p, rowmax, lse, c);
     else
-      softmax_fwd_read_kernel<256, false><<<r, 256, 0, stream>>>(x, p, rowmax, lse, c);
+      softmax_fwd_read_kernel<256><<<r, 256, 0, stream>>>(x, p, rowmax, lse, c);
     return check_launch("softmax_fwd_read_kernel");
   }
   if (fwd_group_ok(plan)) {
@@ -1174,16 +1266,18 @@ extern "C" int credit_softmax_bwd_f32(const float* p, const float* dy, float* dx
   CREDIT_TRY(check_cfg(cfg));
   if (rows == 0) return CREDIT_OK;
   const bool vec = vec_ok(cols, {p, dy, dx});
+  hipStream_t stream = cfg_stream(cfg);
+  if (const auto* pick = ragged_pick(kBwdRows, cfg, rows, cols, vec))
+    return launch_rows(*pick, p, dy, dx, nullptr, nullptr, rows, cols, stream);
   Plan plan;
   CREDIT_TRY(resolve_bwd(cfg, cols, vec, &plan));
-  hipStream_t stream = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (vec)
-      softmax_bwd_read_kernel<256, true><<<r, 256, 0, stream>>>(p, dy, dx, c);
+    if (rows::stream_threads(rows) == 1024)
+      softmax_bwd_read_kernel<1024><<<r, 1024, 0, stream>>>(p, dy, dx, c);
     else
-      softmax_bwd_read_kernel<256, false><<<r, 256, 0, stream>>>(p, dy, dx, c);
+      softmax_bwd_read_kernel<256><<<r, 256, 0, stream>>>(p, dy, dx, c);
     return check_launch("softmax_bwd_read_kernel");
   }
   if (bwd_group_ok(plan)) {
@@ -1226,16 +1320,18 @@ extern "C" int credit_softmax_logits_bwd_f32(const float* logits, const float* d
   CREDIT_TRY(check_cfg(cfg));
   if (rows == 0) return CREDIT_OK;
   const bool vec = vec_ok(cols, {logits, dy, dx});
+  hipStream_t stream = cfg_stream(cfg);
+  if (const auto* pick = ragged_pick(kLogitsRows, cfg, rows, cols, vec))
+    return launch_rows(*pick, logits, dy, dx, nullptr, nullptr, rows, cols, stream);
   Plan plan;
   CREDIT_TRY(resolve(cfg, cols, vec, kBwdCapacity, "softmax_logits_bwd", &plan));
-  hipStream_t stream = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (vec)
-      softmax_logits_bwd_read_kernel<256, true><<<r, 256, 0, stream>>>(logits, dy, dx, c);
+    if (rows::stream_threads(rows) == 1024)
+      softmax_logits_bwd_read_kernel<1024><<<r, 1024, 0, stream>>>(logits, dy, dx, c);
     else
-      softmax_logits_bwd_read_kernel<256, false><<<r, 256, 0, stream>>>(logits, dy, dx, c);
+      softmax_logits_bwd_read_kernel<256><<<r, 256, 0, stream>>>(logits, dy, dx, c);
     return check_launch("softmax_logits_bwd_read_kernel");
   }
   const Pick<BwdFn>* pk = pick_for(kLogits, plan.chunk);

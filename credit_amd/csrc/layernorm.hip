@@ -33,8 +33,11 @@
 //            rows).
 // Algorithmic traffic per row: 2*cols (x) + 2*cols (y) + 8 (mean, rstd) bytes,
 // plus 4*cols once for gamma and beta.
+#include <initializer_list>
+
 #include "api_internal.hpp"
 #include "common.hpp"
+#include "rows.hpp"
 
 namespace credit {
 namespace {
@@ -443,6 +446,101 @@ __global__ __launch_bounds__(THREADS) void layernorm_fwd_read_kernel(
   }
 }
 
+// ------------------------------------------------------- ragged rows -----
+// AUTO on rows that fit no 16-byte layout (rows.hpp), of at most 65536
+// columns: the row read once into one workgroup's registers, its sum and its
+// squared deviations from the mean taken per element in fp64 (READ's
+// arithmetic), where READ streams it three times in 2-byte loads.  4096 x
+// 5002: 39.5 -> 22.5 us, x 5001: 39.7 -> 35 us.
+template <bool ODD, int THREADS, int VPT>
+__global__ __launch_bounds__(THREADS) void layernorm_fwd_rows_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma,
+    const uint16_t* __restrict__ beta, uint16_t* __restrict__ y, float* __restrict__ mean_out,
+    float* __restrict__ rstd_out, int rows, int cols, float eps) {
+  constexpr int NW = THREADS / kWave;
+  __shared__ double red[2][NW];
+  const int tid = threadIdx.x;
+  const int G = gridDim.x;
+  const uint32_t off = static_cast<uint32_t>(tid) * 16u;
+  constexpr uint32_t kStride = THREADS * 16u;
+  int left = cols - 8 * tid;  // elements from the lane's first vector on
+  const rows::HalfRow gr = rows::half_row<ODD, true>(gamma, 0, rows, cols);
+  const rows::HalfRow br = rows::half_row<ODD, true>(beta, 0, rows, cols);
+  u32x4 v[VPT];
+  int row = blockIdx.x;
+  auto load = [&](int r) {
+    const rows::HalfRow xr = rows::half_row<ODD, true>(x, r, rows, cols);
+#pragma unroll
+    for (int k = 0; k < VPT; ++k)
+      v[k] = rows::half_load<ODD>(xr, off + k * kStride, left - 8 * k * THREADS);
+  };
+  load(row);
+  for (; row < rows; row += G) {
+    double s = 0.0;  // past the row's end x reads 0
+#pragma unroll
+    for (int k = 0; k < VPT; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        s += static_cast<double>(bf16_lo(v[k][e])) + static_cast<double>(bf16_hi(v[k][e]));
+    const double mean = rows::block_sum<NW>(s, red[0]) / cols;
+    const float mu = static_cast<float>(mean);
+    double q = 0.0;
+    // Opaque: each pass unpacks the row and forms its masks anew instead of
+    // keeping them in registers (VPT 8: 226 -> 94 VGPRs).
+    __asm__ volatile("" : "+v"(left));
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) __asm__ volatile("" : "+v"(v[k]));
+#pragma unroll
+    for (int k = 0; k < VPT; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int n = left - 8 * k * THREADS - 2 * e;
+        const double lo = n > 0 ? bf16_lo(v[k][e]) - mean : 0.0;
+        const double hi = n > 1 ? bf16_hi(v[k][e]) - mean : 0.0;
+        q += lo * lo;
+        q += hi * hi;
+      }
+    const double var = rows::block_sum<NW>(q, red[1]) / cols;
+    const float rs = static_cast<float>(1.0 / __builtin_sqrt((var > 0.0 ? var : 0.0) + eps));
+    __asm__ volatile("" : "+v"(left));
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) __asm__ volatile("" : "+v"(v[k]));
+    const rows::HalfRow yr = rows::half_row<ODD, false>(y, row, rows, cols);
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+      const int n = left - 8 * k * THREADS;
+      const u32x4 gv = rows::half_load<ODD, false>(gr, off + k * kStride, n);
+      const u32x4 bv = rows::half_load<ODD, false>(br, off + k * kStride, n);
+      rows::half_store<ODD>(yr, off + k * kStride, n, norm8(v[k], gv, bv, mu, rs));
+    }
+    if (tid == 0) {
+      mean_out[row] = mu;
+      rstd_out[row] = rs;
+    }
+    load(row + G);
+  }
+}
+
+using RowsFn = void (*)(const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, float*,
+                        float*, int, int, float);
+// Odd widths shift every vector into place, work that gains from more lanes at
+// any row count (16384 x 1001: 24.7 us on 128 lanes, 31.1 on 64).
+template <bool ODD>
+struct RowsTable {
+  static constexpr rows::RowsPick<RowsFn> table[] = {
+      {layernorm_fwd_rows_kernel<ODD, 64, 1>, 64, 512, !ODD},
+      {layernorm_fwd_rows_kernel<ODD, 128, 1>, 128, 1024, !ODD},
+      {layernorm_fwd_rows_kernel<ODD, 256, 1>, 256, 2048, !ODD},
+      {layernorm_fwd_rows_kernel<ODD, 256, 2>, 256, 4096, !ODD},
+      {layernorm_fwd_rows_kernel<ODD, 64, 4>, 64, 2048},
+      {layernorm_fwd_rows_kernel<ODD, 128, 4>, 128, 4096},
+      {layernorm_fwd_rows_kernel<ODD, 256, 4>, 256, 8192},
+      {layernorm_fwd_rows_kernel<ODD, 256, 8>, 256, 16384},
+      {layernorm_fwd_rows_kernel<ODD, 512, 8>, 512, 32768},
+      {layernorm_fwd_rows_kernel<ODD, 512, 16>, 512, 65536},
+  };
+};
+
 using StagedFn = void (*)(const uint16_t*, const uint16_t*, const uint16_t*,
                           uint16_t*, float*, float*, int, float);
 
@@ -575,12 +673,30 @@ extern "C" int credit_layernorm_fwd_bf16(const uint16_t* x, const uint16_t* gamm
                       reinterpret_cast<uintptr_t>(gamma) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(beta) % 16 == 0;
   const int64_t nvec = cols / 8;
+  bool dwords = rows <= (int64_t{1} << 30);
+  for (const void* p : {static_cast<const void*>(x), static_cast<const void*>(gamma),
+                        static_cast<const void*>(beta), static_cast<const void*>(y)})
+    dwords = dwords && reinterpret_cast<uintptr_t>(p) % 4 == 0;
+  if (!vec_ok && dwords && cfg_variant(cfg) == CREDIT_VARIANT_AUTO) {
+    const auto* rp = cols % 2 != 0 ? rows::rows_pick(RowsTable<true>::table, rows, cols)
+                                   : rows::rows_pick(RowsTable<false>::table, rows, cols);
+    if (rp != nullptr) {
+      unsigned grid = 0;
+      CREDIT_TRY(rows::rows_grid(*rp, rows, &grid));
+      hipLaunchKernelGGL(rp->fn, dim3(grid), dim3(rp->threads), 0, stream, x, gamma, beta, y,
+                         mean, rstd, static_cast<int>(rows), c, eps);
+      return check_launch("layernorm_fwd_rows_kernel");
+    }
+  }
   Plan plan;
   CREDIT_TRY(resolve(cfg, cols, vec_ok, &plan));
   const dim3 row_grid(static_cast<unsigned>(rows));
   if (plan.variant == CREDIT_VARIANT_READ) {
     if (vec_ok)
       layernorm_fwd_read_kernel<256, true><<<row_grid, dim3(256), 0, stream>>>(
+          x, gamma, beta, y, mean, rstd, c, eps);
+    else if (rows::stream_threads(rows) == 1024)
+      layernorm_fwd_read_kernel<1024, false><<<row_grid, dim3(1024), 0, stream>>>(
           x, gamma, beta, y, mean, rstd, c, eps);
     else
       layernorm_fwd_read_kernel<256, false><<<row_grid, dim3(256), 0, stream>>>(

@@ -457,7 +457,7 @@ __global__ __launch_bounds__(THREADS) void layernorm_bwd_read_kernel(
 // once, sums per element in fp64 as READ, gamma re-read from L2 with each row.
 // The next row's loads are issued behind the output loop, not inside it, so
 // that its gamma loads wait for no HBM load.  fp32 at 3000 x 5003: 73.5 -> 39.1 us (4.6 TB/s).
-template <class T, int THREADS, int VPT>
+template <class T, bool ODD, int THREADS, int VPT>
 __global__ __launch_bounds__(THREADS) void layernorm_bwd_rows_kernel(
     const T* __restrict__ x, const T* __restrict__ dy, const T* __restrict__ gamma,
     T* __restrict__ dx, int rows, int cols, float eps) {
@@ -471,17 +471,31 @@ __global__ __launch_bounds__(THREADS) void layernorm_bwd_rows_kernel(
   const int G = gridDim.x;
   const uint32_t off = static_cast<uint32_t>(tid) * 16u;
   constexpr uint32_t kStride = THREADS * 16u;
-  const buffer_rsrc_t grs = make_rsrc(gamma, static_cast<uint32_t>(cols * sizeof(T)));
+  auto row_of = [&](const T* base, int r, auto load) {
+    if constexpr (E == 8)
+      return rows::half_row<ODD, decltype(load)::value>(base, r, rows, cols);
+    else
+      return rows::row_rsrc(base, r, rows, cols);
+  };
+  auto get = [&](const auto& r, int k, int left, auto nt) {
+    if constexpr (E == 8)
+      return rows::half_load<ODD, decltype(nt)::value>(r, off + k * kStride,
+                                                       left - E * k * THREADS);
+    else
+      return __builtin_bit_cast(raw, decltype(nt)::value ? buffer_load_nt(r, off + k * kStride)
+                                                         : buffer_load(r, off + k * kStride));
+  };
+  const auto grs = row_of(gamma, 0, std::true_type{});
   int left = cols - E * tid;  // elements from the lane's first vector on
   raw xv[VPT], dv[VPT];
   int row = blockIdx.x;
   auto load = [&](int r) {
-    const buffer_rsrc_t xr = rows::row_rsrc(x, r, rows, cols);
-    const buffer_rsrc_t dr = rows::row_rsrc(dy, r, rows, cols);
+    const auto xr = row_of(x, r, std::true_type{});
+    const auto dr = row_of(dy, r, std::true_type{});
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      xv[k] = __builtin_bit_cast(raw, buffer_load_nt(xr, off + k * kStride));
-      dv[k] = __builtin_bit_cast(raw, buffer_load_nt(dr, off + k * kStride));
+      xv[k] = get(xr, k, left, std::true_type{});
+      dv[k] = get(dr, k, left, std::true_type{});
     }
   };
   load(row);
@@ -502,11 +516,12 @@ __global__ __launch_bounds__(THREADS) void layernorm_bwd_rows_kernel(
     const RowStats st = stats_from(a1, a2, x0, cols, eps);
     opaque_regs<VPT>(xv);
     opaque_regs<VPT>(dv);
+    __asm__ volatile("" : "+v"(left));
     // Past the row's end dy reads 0, so g = dy * gamma adds nothing.
     double b1 = 0.0, b2 = 0.0;
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      const raw gv = __builtin_bit_cast(raw, buffer_load(grs, off + k * kStride));
+      const raw gv = get(grs, k, left, std::false_type{});
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const float gg = V::get(dv[k], e) * V::get(gv, e);
@@ -515,21 +530,25 @@ __global__ __launch_bounds__(THREADS) void layernorm_bwd_rows_kernel(
       }
     }
     rows::block_sum2<NW>(b1, b2, red2);
+    __asm__ volatile("" : "+v"(left));
     const float mg = static_cast<float>(b1 / cols);
     const float mgx = static_cast<float>(b2 / cols);
     opaque_regs<VPT>(xv);
     opaque_regs<VPT>(dv);
-    const buffer_rsrc_t ors = rows::row_rsrc(dx, row, rows, cols);
+    const auto ors = row_of(dx, row, std::false_type{});
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      const raw gv = __builtin_bit_cast(raw, buffer_load(grs, off + k * kStride));
+      const raw gv = get(grs, k, left, std::false_type{});
       float o[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const float xh = (V::get(xv[k], e) - st.mean) * st.rstd;
         o[e] = (V::get(dv[k], e) * V::get(gv, e) - mg - xh * mgx) * st.rstd;
       }
-      buffer_store_nt(ors, off + k * kStride, __builtin_bit_cast(u32x4, V::pack(o)));
+      if constexpr (E == 8)
+        rows::half_store<ODD>(ors, off + k * kStride, left - E * k * THREADS, V::pack(o));
+      else
+        rows::row_store(ors, off + k * kStride, V::pack(o));
     }
     load(row + G);
   }
@@ -537,16 +556,20 @@ __global__ __launch_bounds__(THREADS) void layernorm_bwd_rows_kernel(
 
 template <class T>
 using RowsFn = void (*)(const T*, const T*, const T*, T*, int, int, float);
-template <class T>
+template <class T, bool ODD>
 struct RowsTable {
   static constexpr int kE = Vec<T>::kN;
   static constexpr rows::RowsPick<RowsFn<T>> table[] = {
-      {layernorm_bwd_rows_kernel<T, 64, 4>, 64, 256 * kE},
-      {layernorm_bwd_rows_kernel<T, 128, 4>, 128, 512 * kE},
-      {layernorm_bwd_rows_kernel<T, 256, 4>, 256, 1024 * kE},
-      {layernorm_bwd_rows_kernel<T, 256, 8>, 256, 2048 * kE},
-      {layernorm_bwd_rows_kernel<T, 512, 8>, 512, 4096 * kE},
-      {layernorm_bwd_rows_kernel<T, 512, 16>, 512, 8192 * kE},
+      {layernorm_bwd_rows_kernel<T, ODD, 64, 1>, 64, 64 * kE, true},
+      {layernorm_bwd_rows_kernel<T, ODD, 128, 1>, 128, 128 * kE, true},
+      {layernorm_bwd_rows_kernel<T, ODD, 256, 1>, 256, 256 * kE, true},
+      {layernorm_bwd_rows_kernel<T, ODD, 256, 2>, 256, 512 * kE, true},
+      {layernorm_bwd_rows_kernel<T, ODD, 64, 4>, 64, 256 * kE},
+      {layernorm_bwd_rows_kernel<T, ODD, 128, 4>, 128, 512 * kE},
+      {layernorm_bwd_rows_kernel<T, ODD, 256, 4>, 256, 1024 * kE},
+      {layernorm_bwd_rows_kernel<T, ODD, 256, 8>, 256, 2048 * kE},
+      {layernorm_bwd_rows_kernel<T, ODD, 512, 8>, 512, 4096 * kE},
+      {layernorm_bwd_rows_kernel<T, ODD, 512, 16>, 512, 8192 * kE},
   };
 };
 
@@ -737,13 +760,17 @@ int layernorm_bwd(const T* x, const T* dy, const T* gamma, T* dx, int64_t rows, 
   }
   hipStream_t stream = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
-  // Rows at 4-byte addresses without the 16-byte layout.
-  bool dwords = cols * sizeof(T) % 4 == 0 && rows <= (int64_t{1} << 30);
+  // Buffers at 4-byte addresses without the 16-byte layout.
+  bool dwords = rows <= (int64_t{1} << 30);
   for (const void* p : {static_cast<const void*>(x), static_cast<const void*>(dy),
                         static_cast<const void*>(gamma), static_cast<const void*>(dx)})
     dwords = dwords && reinterpret_cast<uintptr_t>(p) % 4 == 0;
   if (!vec && dwords && cfg_variant(cfg) == CREDIT_VARIANT_AUTO) {
-    if (const auto* pick = rows::rows_pick(RowsTable<T>::table, cols)) {
+    const rows::RowsPick<RowsFn<T>>* pick = rows::rows_pick(RowsTable<T, false>::table, rows, cols);
+    if constexpr (std::is_same_v<T, uint16_t>) {
+      if (cols % 2 != 0) pick = rows::rows_pick(RowsTable<T, true>::table, rows, cols);
+    }
+    if (pick != nullptr) {
       unsigned grid = 0;
       CREDIT_TRY(rows::rows_grid(*pick, rows, &grid));
       hipLaunchKernelGGL(pick->fn, dim3(grid), dim3(pick->threads), 0, stream, x, dy, gamma, dx,

@@ -176,6 +176,10 @@ __global__ __launch_bounds__(THREADS) void rowwise_quant_read_kernel(
 
 using QuantRowsFn = void (*)(const float*, int8_t*, float*, int, int);
 const rows::RowsPick<QuantRowsFn> kQuantRows[] = {
+    {rowwise_quant_rows_kernel<64, 1>, 64, 256, true},
+    {rowwise_quant_rows_kernel<128, 1>, 128, 512, true},
+    {rowwise_quant_rows_kernel<256, 1>, 256, 1024, true},
+    {rowwise_quant_rows_kernel<256, 2>, 256, 2048, true},
     {rowwise_quant_rows_kernel<64, 4>, 64, 1024},    {rowwise_quant_rows_kernel<128, 4>, 128, 2048},
     {rowwise_quant_rows_kernel<256, 4>, 256, 4096},  {rowwise_quant_rows_kernel<256, 8>, 256, 8192},
     {rowwise_quant_rows_kernel<512, 8>, 512, 16384}, {rowwise_quant_rows_kernel<512, 16>, 512, 32768},
@@ -228,7 +232,7 @@ extern "C" int credit_rowwise_quant_f32(const float* x, int8_t* q, float* scale,
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
   if (!vec && cfg_variant(cfg) == CREDIT_VARIANT_AUTO && rows <= (int64_t{1} << 30)) {
-    if (const auto* pick = rows::rows_pick(kQuantRows, cols)) {
+    if (const auto* pick = rows::rows_pick(kQuantRows, rows, cols)) {
       unsigned grid = 0;
       CREDIT_TRY(rows::rows_grid(*pick, rows, &grid));
       hipLaunchKernelGGL(pick->fn, dim3(grid), dim3(pick->threads), 0, stream, x, q, scale,

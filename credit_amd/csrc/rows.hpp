@@ -1,8 +1,8 @@
-// Rows whose width or alignment fits no 16-byte layout (fp32 at any width,
-// bf16 at even widths): what the kernels that hold such a row in one
-// workgroup's registers share.
+// Rows whose width or alignment fits no 16-byte layout: what the kernels that
+// hold such a row in one workgroup's registers share.
 //
-// A row starts at any 4-byte address.  dwordx4 buffer loads and stores need no
+// An fp32 row, or a bf16 row of even width, starts at any 4-byte address (bf16
+// rows of odd width: HalfRow below).  dwordx4 buffer loads and stores need no
 // more than that, and a raw buffer's range check works per dword: with
 // num_records the row's bytes, the row's last vector reads zeros past the end
 // and its stores there are dropped, so a ragged row runs the same
@@ -38,6 +38,74 @@ __device__ __forceinline__ void row_store(buffer_rsrc_t r, uint32_t offset, f32x
 __device__ __forceinline__ f32x4 keep4(f32x4 v, int left, float fill) {
   return f32x4{left > 0 ? v.x : fill, left > 1 ? v.y : fill, left > 2 ? v.z : fill,
                left > 3 ? v.w : fill};
+}
+
+// A bf16 row of a tensor at a 4-byte address.  ODD (odd widths): every other
+// row starts in the upper half of a dword.  It is then read from the dword's
+// start, one dword further, and shifted into place; on the rows that start on
+// a dword the last element shares its dword with the next row and travels by
+// itself.  No access leaves the row's own elements but the half dword before
+// an odd row's start, the previous row's last element.
+struct HalfRow {
+  buffer_rsrc_t dwords;  // the whole dwords from the row's first (half) dword on
+  buffer_rsrc_t halves;  // the same to the row's last byte (ODD stores)
+  uint32_t shift;        // 16 on an odd row, else 0
+  uint32_t last;         // the row's last element (ODD loads)
+};
+template <bool ODD, bool LOAD>
+__device__ __forceinline__ HalfRow half_row(const uint16_t* base, int row, int rows, int cols) {
+  const bool live = row < rows;
+  const size_t at = static_cast<size_t>(live ? row : 0) * cols;
+  const uint32_t odd = ODD ? static_cast<uint32_t>(at) & 1u : 0u;
+  const uint32_t bytes = live ? (static_cast<uint32_t>(cols) + odd) * 2u : 0u;
+  HalfRow r;
+  r.dwords = make_rsrc(base + at - odd, bytes & ~3u);
+  r.halves = make_rsrc(base + at - odd, bytes);
+  r.shift = odd * 16u;
+  r.last = ODD && LOAD && live ? base[at + cols - 1] : 0u;
+  return r;
+}
+// Elements 8 i .. 8 i + 7 of the row, off = 16 i, left = cols - 8 i; zeros past
+// the row's end.
+template <bool ODD, bool NT = true>
+__device__ __forceinline__ u32x4 half_load(const HalfRow& r, uint32_t off, int left) {
+  u32x4 v = NT ? buffer_load_nt(r.dwords, off) : buffer_load(r.dwords, off);
+  if constexpr (ODD) {
+    const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(r.dwords, off + 16u, 0, 0);
+    v = u32x4{__builtin_amdgcn_alignbit(v.y, v.x, r.shift),
+              __builtin_amdgcn_alignbit(v.z, v.y, r.shift),
+              __builtin_amdgcn_alignbit(v.w, v.z, r.shift),
+              __builtin_amdgcn_alignbit(w, v.w, r.shift)};
+    // An odd width's last element is the low half of its dword; past it an
+    // odd row's last vector holds zeros already.
+#pragma unroll
+    for (int d = 0; d < 4; ++d) v[d] = left == 2 * d + 1 ? r.last : v[d];
+  }
+  return v;
+}
+template <bool ODD>
+__device__ __forceinline__ void half_store(const HalfRow& r, uint32_t off, int left, u32x4 v) {
+  if (!ODD) {
+    buffer_store_nt(r.dwords, off, v);
+  } else if (r.shift == 0) {
+    buffer_store_nt(r.dwords, off, v);
+    // The last element, alone in its row's last half dword.
+    const uint32_t e = left == 1 ? v.x : left == 3 ? v.y : left == 5 ? v.z : v.w;
+    const bool here = left > 0 && left < 8;
+    __builtin_amdgcn_raw_buffer_store_b16(static_cast<short>(e), r.halves,
+                                          here ? off + 2u * (left - 1) : 0xFFFFFFF0u, 0, 0);
+  } else {
+    // Element 0 in the upper half of the first dword, 1 to 6 in the next
+    // three, 7 in the lower half of the fifth.
+    typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+    __builtin_amdgcn_raw_buffer_store_b16(static_cast<short>(v.x), r.halves, off + 2u, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b96(
+        u32x3{__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+              __builtin_amdgcn_alignbit(v.w, v.z, 16)},
+        r.dwords, off + 4u, 0, kBufferNt);
+    __builtin_amdgcn_raw_buffer_store_b16(static_cast<short>(v.w >> 16), r.halves, off + 16u, 0,
+                                          0);
+  }
 }
 
 // Block reductions on an LDS-only barrier (loads and stores in flight stay
@@ -99,13 +167,19 @@ struct RowsPick {
   Fn fn;
   int threads;
   int64_t capacity;  // elements
+  bool few = false;  // for at most kFewRows rows
 };
 
-// The narrowest entry that holds `cols`; nullptr: none.
+// The first entry that holds `cols`; nullptr: none.  A lone row's time is its
+// lanes' serial work, so the tables open with narrow rows spread over many
+// lanes, taken up to kFewRows rows (softmax logits backward 1 x 1134: 4.5 ->
+// 3.4 us a call); with more, fewer lanes of more vectors keep more rows in
+// flight (softmax forward 16384 x 770: 20.6 us on 64 lanes, 25.2 on 256).
+constexpr int64_t kFewRows = 2048;
 template <class Fn, int N>
-const RowsPick<Fn>* rows_pick(const RowsPick<Fn> (&table)[N], int64_t cols) {
+const RowsPick<Fn>* rows_pick(const RowsPick<Fn> (&table)[N], int64_t rows, int64_t cols) {
   for (const RowsPick<Fn>& p : table)
-    if (cols <= p.capacity) return &p;
+    if (cols <= p.capacity && (rows <= kFewRows || !p.few)) return &p;
   return nullptr;
 }
 

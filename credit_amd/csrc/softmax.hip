@@ -1032,12 +1032,14 @@ const Pick<BwdFn> kLogits[] = {
     {softmax_logits_bwd_slice_kernel<1024, 8>, 1024, 8192},
 };
 
-// Ragged rows: 4 to 32 f32x4 per lane and tensor.
+// Ragged rows: 1 to 32 f32x4 per lane and tensor.
 using RowsFn = void (*)(const float*, const float*, float*, float*, float*, int, int);
-#define CREDIT_ROWS_TABLE(OP, LAST)                                                     \
-  {{softmax_rows_kernel<OP, 64, 4>, 64, 1024},    {softmax_rows_kernel<OP, 128, 4>, 128, 2048}, \
-   {softmax_rows_kernel<OP, 256, 4>, 256, 4096},  {softmax_rows_kernel<OP, 256, 8>, 256, 8192}, \
-   {softmax_rows_kernel<OP, 512, 8>, 512, 16384}, {softmax_rows_kernel<OP, 512, 16>, 512, 32768}, \
+#define CREDIT_ROWS_TABLE(OP, LAST)                                                              \
+  {{softmax_rows_kernel<OP, 64, 1>, 64, 256, true},     {softmax_rows_kernel<OP, 128, 1>, 128, 512, true}, \
+   {softmax_rows_kernel<OP, 256, 1>, 256, 1024, true},  {softmax_rows_kernel<OP, 256, 2>, 256, 2048, true}, \
+   {softmax_rows_kernel<OP, 64, 4>, 64, 1024},          {softmax_rows_kernel<OP, 128, 4>, 128, 2048},  \
+   {softmax_rows_kernel<OP, 256, 4>, 256, 4096},        {softmax_rows_kernel<OP, 256, 8>, 256, 8192},  \
+   {softmax_rows_kernel<OP, 512, 8>, 512, 16384},       {softmax_rows_kernel<OP, 512, 16>, 512, 32768}, \
    {softmax_rows_kernel<OP, 512, LAST>, 512, 2048 * LAST}}
 const rows::RowsPick<RowsFn> kFwdRows[] = CREDIT_ROWS_TABLE(kOpFwd, 32);
 const rows::RowsPick<RowsFn> kBwdRows[] = CREDIT_ROWS_TABLE(kOpBwd, 26);
@@ -1051,7 +1053,7 @@ const rows::RowsPick<RowsFn>* ragged_pick(const rows::RowsPick<RowsFn> (&table)[
                                           const credit_cfg* cfg, int64_t rows, int64_t cols,
                                           bool vec) {
   if (vec || cfg_variant(cfg) != CREDIT_VARIANT_AUTO || rows > (int64_t{1} << 30)) return nullptr;
-  return rows::rows_pick(table, cols);
+  return rows::rows_pick(table, rows, cols);
 }
 int launch_rows(const rows::RowsPick<RowsFn>& pick, const float* a, const float* dy, float* out,
                 float* rowmax, float* lse, int64_t rows, int64_t cols, hipStream_t stream) {

@@ -115,10 +115,17 @@ def test_ragged_quant(gpu, rows, cols, shift):
     assert np.array_equal(scale[i].cpu().numpy(), es.astype(np.float32))
 
 
+# Even and odd widths (odd: every other row starts inside a dword), buffers at
+# 4-byte (shift 2) and 2-byte (shift 1, streamed) addresses, both edges of the
+# register tables and the first width past them.
+NORM_SHAPES = [(3, 30, 2), (4, 31, 0), (5, 1002, 0), (6, 1023, 0), (4000, 1030, 0), (4001, 1001, 2),
+               (700, 5003, 0), (9, 2047, 0), (9, 2049, 0), (600, 8194, 0), (601, 8191, 0),
+               (300, 16390, 2), (300, 16383, 0), (270, 32766, 0), (270, 32767, 0), (3, 32770, 0),
+               (3, 32769, 1), (2, 65534, 0), (3, 65535, 0), (2, 65538, 0), (3, 65537, 0)]
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows,cols,shift", [
-    (3, 30, 2), (5, 1002, 0), (6, 1023, 0), (4000, 1030, 0), (700, 5003, 0), (600, 8194, 0),
-    (300, 16390, 2), (270, 32766, 0), (3, 32770, 0), (2, 65534, 0), (2, 65538, 0)])
+@pytest.mark.parametrize("rows,cols,shift", NORM_SHAPES)
 def test_ragged_layernorm_backward(gpu, rows, cols, shift, dtype):
     print(f"ragged layernorm backward {rows} x {cols} + {shift} {dtype}", flush=True)
     name = "layernorm_backward" + ("_bf16" if dtype == torch.bfloat16 else "")
@@ -136,3 +143,23 @@ def test_ragged_layernorm_backward(gpu, rows, cols, shift, dtype):
     np.testing.assert_allclose(dx[i].float().cpu().numpy(), expect,
                                **(FP32 if dtype == torch.float32 else BF16))
     assert not bool(torch.isnan(dx).any())
+
+
+@pytest.mark.parametrize("rows,cols,shift", NORM_SHAPES)
+def test_ragged_layernorm_forward(gpu, rows, cols, shift):
+    print(f"ragged layernorm forward {rows} x {cols} + {shift}", flush=True)
+    x, gamma, beta = WORKLOADS["layernorm_fwd"].make_inputs(rows, cols, seed=rows + cols)
+    x[: rows // 2] += 3.0  # an offset the variance takes out
+    y, gy = output((rows, cols), torch.bfloat16, shift, gpu)
+    mean, rstd = torch.empty(rows, device=gpu), torch.empty(rows, device=gpu)
+    hip_lib.layernorm_fwd(place(x, shift, gpu), place(gamma, shift, gpu), place(beta, shift, gpu),
+                          y, mean, rstd, hip_lib.LAYERNORM_EPS, hip_lib.make_cfg())
+    torch.cuda.synchronize()
+    check_guards(gy)
+    i = sample(rows)
+    ey, em, er = ref.layernorm_fwd(x[i].float().numpy(), gamma.float().numpy(),
+                                   beta.float().numpy())
+    np.testing.assert_allclose(y[i].float().cpu().numpy(), ey, **BF16)
+    np.testing.assert_allclose(mean[i].cpu().numpy(), em, **FP32)
+    np.testing.assert_allclose(rstd[i].cpu().numpy(), er, **FP32)
+    assert not bool(torch.isnan(y).any())

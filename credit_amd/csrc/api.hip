@@ -159,6 +159,10 @@ bool stream_capturing(hipStream_t stream) {
   return true;
 }
 
+bool keeps_scratch(hipStream_t stream) {
+  return stream != hipStreamPerThread && !stream_capturing(stream);
+}
+
 int acquire_workspace_with(const credit_cfg* cfg, size_t own, size_t extra, char** base,
                            char** spare, size_t* spare_bytes) {
   const size_t at = align_up(own, 256);

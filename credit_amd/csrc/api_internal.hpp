@@ -130,6 +130,11 @@ inline size_t split_slot_bytes(int64_t groups, int members, int k_values, int ri
 int acquire_workspace(const credit_cfg* cfg, size_t bytes, char** base);
 // Whether `stream` is being captured into a graph (nothing can be allocated).
 bool stream_capturing(hipStream_t stream);
+// Whether a call on `stream` may use scratch that the library keeps per stream
+// and no caller has been told of: not under capture (a graph replays on any
+// stream, beside the eager calls of the one it was captured on) and not on the
+// per-thread default stream, one handle for as many streams as threads.
+bool keeps_scratch(hipStream_t stream);
 // A workspace of `own` scratch bytes and, where they can be had, `extra` more
 // behind them (*spare, *spare_bytes) that the call can do without: the rest of
 // a caller's workspace, or the library's buffer unless it would have to grow
@@ -238,6 +243,17 @@ size_t rmsnorm_bwd_workspace(int64_t rows, int64_t cols, int variant, int split,
                              int cu_count);
 size_t rmsnorm_fused_workspace(int64_t rows, int64_t cols, int variant, int split,
                                int cu_count);
+
+// Few wide fp32 rows in two launches (widerows.hip).  `vec`: every buffer takes
+// 16-byte vectors.  *taken false: the call's other kernels run it.
+enum class WideSoftmax { kForward, kBackward, kLogits };
+int wide_softmax(WideSoftmax op, const float* a, const float* dy, float* out, float* rowmax,
+                 float* lse, int64_t rows, int64_t cols, bool vec, const credit_cfg* cfg,
+                 bool* taken);
+int wide_quant(const float* x, int8_t* q, float* scale, int64_t rows, int64_t cols, bool vec,
+               const credit_cfg* cfg, bool* taken);
+int wide_layernorm_bwd(const float* x, const float* dy, const float* gamma, float* dx, int64_t rows,
+                       int64_t cols, float eps, bool vec, const credit_cfg* cfg, bool* taken);
 
 // CU count of the current device, or 256 (MI355X) when none is visible.
 int cu_count_or_default();

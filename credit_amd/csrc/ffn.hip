@@ -1342,9 +1342,12 @@ size_t bwd_scratch(int64_t M, int64_t d, int64_t f) {
 
 // The training forward brings no workspace and shares none: its scratch is a
 // buffer per (device, stream) of its own, in use only between the launches of
-// one call, which train_mutex keeps together when threads share a stream.  At
-// most 2 * kTrainScratch per stream, never freed while the process runs.
+// one call, which train_mutex keeps together when threads share a stream; a
+// captured call goes without (keeps_scratch), with the same bits.  At most 2 *
+// kTrainScratch for each of the first kTrainStreams, kept while the process
+// runs.
 constexpr size_t kTrainScratch = size_t{256} << 20;
+constexpr size_t kTrainStreams = 16;
 struct ScratchAlloc {
   int operator()(int, void*, size_t bytes, char** out) const {
     // Relaxed: another thread's stream may be under capture meanwhile.
@@ -1369,7 +1372,7 @@ int train_scratch(hipStream_t stream, size_t want, Scratch* out) {
   if (want == 0) return CREDIT_OK;
   int dev = 0;
   CREDIT_HIP(hipGetDevice(&dev));
-  if (cache->capacity(dev, stream) < want && stream_capturing(stream)) return CREDIT_OK;
+  if (!keeps_scratch(stream) || !cache->room(dev, stream, kTrainStreams)) return CREDIT_OK;
   char* p = nullptr;
   if (cache->get(dev, stream, want, &p) == CREDIT_OK) *out = Scratch{p, want};
   return CREDIT_OK;

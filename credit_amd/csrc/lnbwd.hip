@@ -760,6 +760,11 @@ int layernorm_bwd(const T* x, const T* dy, const T* gamma, T* dx, int64_t rows, 
   }
   hipStream_t stream = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
+  if constexpr (std::is_same_v<T, float>) {
+    bool taken = false;
+    CREDIT_TRY(wide_layernorm_bwd(x, dy, gamma, dx, rows, cols, eps, vec, cfg, &taken));
+    if (taken) return CREDIT_OK;
+  }
   // Buffers at 4-byte addresses without the 16-byte layout.
   bool dwords = rows <= (int64_t{1} << 30);
   for (const void* p : {static_cast<const void*>(x), static_cast<const void*>(dy),

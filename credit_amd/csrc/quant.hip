@@ -22,6 +22,7 @@
 // Algorithmic traffic per row: 4*cols (x) + cols (q) + 4 (scale) bytes.
 #include "api_internal.hpp"
 #include "common.hpp"
+#include "quant_codes.hpp"
 #include "rows.hpp"
 #include "slices.hpp"
 
@@ -29,28 +30,6 @@ namespace credit {
 namespace {
 
 using namespace slices;
-
-__device__ __forceinline__ float absmax4(f32x4 v) {
-  return fmax_nan(fmax_nan(__builtin_fabsf(v.x), __builtin_fabsf(v.y)),
-                  fmax_nan(__builtin_fabsf(v.z), __builtin_fabsf(v.w)));
-}
-
-__device__ __forceinline__ uint32_t quant1(float x, float inv) {
-  float q = __builtin_rintf(x * inv);
-  q = __builtin_fminf(127.0f, __builtin_fmaxf(-127.0f, q));
-  return static_cast<uint32_t>(static_cast<int32_t>(q)) & 0xFFu;
-}
-
-// Four int8 codes packed little-endian (element 0 in the low byte).
-__device__ __forceinline__ uint32_t quant4(f32x4 v, float inv) {
-  return quant1(v.x, inv) | (quant1(v.y, inv) << 8) | (quant1(v.z, inv) << 16) |
-         (quant1(v.w, inv) << 24);
-}
-
-// inv as the reference's torch function computes it.
-__device__ __forceinline__ float inv_scale(float max_abs) {
-  return max_abs > 0.0f ? (1.0f / max_abs) * 127.0f : 0.0f;
-}
 
 template <int THREADS, int VPT>
 __device__ __forceinline__ void rowwise_quant_slice_kernel_body(
@@ -95,14 +74,6 @@ __global__ __launch_bounds__(THREADS) void rowwise_quant_slice_kernel(
     int chunk, int members, int rows, SplitArgs sa) {
   rowwise_quant_slice_kernel_body<THREADS, VPT>(x, q, scale, cols, chunk, members, rows, sa);
   split_leave(sa);
-}
-
-// The four codes of a vector, at any address.
-__device__ __forceinline__ void store_codes(int8_t* q, uint32_t codes) {
-  __builtin_memcpy(q, &codes, 4);
-}
-__device__ __forceinline__ int8_t code1(float x, float inv) {
-  return static_cast<int8_t>(static_cast<int32_t>(quant1(x, inv) << 24) >> 24);
 }
 
 // Ragged rows (rows.hpp) held in one workgroup's registers: x read once.
@@ -231,6 +202,9 @@ extern "C" int credit_rowwise_quant_f32(const float* x, int8_t* q, float* scale,
   hipStream_t stream = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
+  bool taken = false;
+  CREDIT_TRY(wide_quant(x, q, scale, rows, cols, vec, cfg, &taken));
+  if (taken) return CREDIT_OK;
   if (!vec && cfg_variant(cfg) == CREDIT_VARIANT_AUTO && rows <= (int64_t{1} << 30)) {
     if (const auto* pick = rows::rows_pick(kQuantRows, rows, cols)) {
       unsigned grid = 0;

@@ -1216,6 +1216,10 @@ extern "C" int credit_softmax_fwd_f32(const float* x, float* p, float* rowmax, f
   if (rows == 0) return CREDIT_OK;
   const bool vec = vec_ok(cols, {x, p});
   hipStream_t stream = cfg_stream(cfg);
+  bool taken = false;
+  CREDIT_TRY(wide_softmax(WideSoftmax::kForward, x, nullptr, p, rowmax, lse, rows, cols, vec, cfg,
+                          &taken));
+  if (taken) return CREDIT_OK;
   if (const auto* pick = ragged_pick(kFwdRows, cfg, rows, cols, vec))
     return launch_rows(*pick, x, nullptr, p, rowmax, lse, rows, cols, stream);
   Plan plan;
@@ -1269,6 +1273,10 @@ extern "C" int credit_softmax_bwd_f32(const float* p, const float* dy, float* dx
   if (rows == 0) return CREDIT_OK;
   const bool vec = vec_ok(cols, {p, dy, dx});
   hipStream_t stream = cfg_stream(cfg);
+  bool taken = false;
+  CREDIT_TRY(wide_softmax(WideSoftmax::kBackward, p, dy, dx, nullptr, nullptr, rows, cols, vec, cfg,
+                          &taken));
+  if (taken) return CREDIT_OK;
   if (const auto* pick = ragged_pick(kBwdRows, cfg, rows, cols, vec))
     return launch_rows(*pick, p, dy, dx, nullptr, nullptr, rows, cols, stream);
   Plan plan;
@@ -1323,6 +1331,10 @@ extern "C" int credit_softmax_logits_bwd_f32(const float* logits, const float* d
   if (rows == 0) return CREDIT_OK;
   const bool vec = vec_ok(cols, {logits, dy, dx});
   hipStream_t stream = cfg_stream(cfg);
+  bool taken = false;
+  CREDIT_TRY(wide_softmax(WideSoftmax::kLogits, logits, dy, dx, nullptr, nullptr, rows, cols, vec, cfg,
+                          &taken));
+  if (taken) return CREDIT_OK;
   if (const auto* pick = ragged_pick(kLogitsRows, cfg, rows, cols, vec))
     return launch_rows(*pick, logits, dy, dx, nullptr, nullptr, rows, cols, stream);
   Plan plan;

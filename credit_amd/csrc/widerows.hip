@@ -1,0 +1,426 @@
+// Few wide fp32 rows in two launches: each row cut into chunks of at most 4096
+// columns, one workgroup per chunk.  The first launch leaves every chunk's
+// partial sums (fp64) in memory, the second merges its row's and writes the
+// outputs.  No workgroup waits for another, so the calls need nothing of the
+// device's other work (the SPLIT kernels do), and any width and 4-byte address
+// is taken (rows.hpp).  The inputs are read twice, the second time from the L2
+// and the MALL while they fit.
+// Bound by two launches (6.7-7 us a call from one stream) up to about a million
+// elements, by HBM at large ones: the two reads and the write move 6.2 TB/s at
+// 256 x 200003.  Against one workgroup per row (registers, then two streamed
+// passes) and SPLIT groups, us:
+//                       1 x 200003  64 x 40003  384 x 200003  16 x 131072
+//   softmax forward       47 -> 7    17 -> 8.6    197 -> 158   10.6 -> 8.0
+//   softmax logits bwd   110 -> 7    21 -> 11     373 -> 265   13.9 -> 10.3
+//   LayerNorm backward   154 -> 7    38 -> 11     466 -> 260   15.1 -> 10.5
+//   quantisation          18 -> 7   9.2 -> 6.6    136 -> 125   11.0 -> 6.8
+#include <algorithm>
+#include <mutex>
+
+#include "api_internal.hpp"
+#include "common.hpp"
+#include "quant_codes.hpp"
+#include "rows.hpp"
+#include "workspace_cache.hpp"
+
+namespace credit {
+namespace {
+
+constexpr int kThreads = 256;
+constexpr int kNW = kThreads / kWave;
+constexpr int kVpt = 4;
+constexpr int kChunk = kThreads * kVpt * 4;  // columns a workgroup holds
+constexpr int kMaxParts = kWave;             // one wave merges a row's chunks
+constexpr int kValues = 5;                   // fp64 values per chunk
+constexpr int kMaxRows = 2048;
+constexpr float kNegInf = -__builtin_inff();
+
+// Where a workgroup is: its row and its chunk's columns.
+struct Place {
+  int row, part, parts, c0, n;
+  double* out;         // the chunk's partials, [value][part] of the row
+  const double* row_partials;
+};
+__device__ __forceinline__ Place place(double* partials, int cols, int chunk, int parts) {
+  Place p;
+  p.row = blockIdx.y;
+  p.part = blockIdx.x;
+  p.parts = parts;
+  p.c0 = p.part * chunk;
+  p.n = cols - p.c0 < chunk ? cols - p.c0 : chunk;
+  double* r = partials + static_cast<size_t>(p.row) * kValues * parts;
+  p.out = r + p.part;
+  p.row_partials = r;
+  return p;
+}
+template <class T>
+__device__ __forceinline__ buffer_rsrc_t chunk_rsrc(const T* base, const Place& p, int cols) {
+  return make_rsrc(base + static_cast<size_t>(p.row) * cols + p.c0,
+                   static_cast<uint32_t>(p.n * sizeof(T)));
+}
+__device__ __forceinline__ void chunk_load(f32x4 (&v)[kVpt], buffer_rsrc_t r) {
+#pragma unroll
+  for (int k = 0; k < kVpt; ++k)
+    v[k] = __builtin_bit_cast(f32x4, buffer_load(r, (threadIdx.x + k * kThreads) * 16u));
+}
+// Elements of the chunk from the lane's k-th vector on.
+__device__ __forceinline__ int left_of(const Place& p, int k) {
+  return p.n - 4 * static_cast<int>(threadIdx.x + k * kThreads);
+}
+// Value k of the row's chunks, one per lane (`none` past the last).
+__device__ __forceinline__ double partial(const Place& p, int k, double none) {
+  const int lane = threadIdx.x & (kWave - 1);
+  return lane < p.parts ? p.row_partials[k * p.parts + lane] : none;
+}
+
+__device__ __forceinline__ float max4(f32x4 v) {
+  return fmax_nan(fmax_nan(v.x, v.y), fmax_nan(v.z, v.w));
+}
+__device__ __forceinline__ double rescale(double a, double b) {
+  return a == -__builtin_inf() ? 0.0 : ::exp(a - b);
+}
+
+// ------------------------------------------------------------- softmax ----
+// Partials: max m, s = sum e^(x - m), t = sum e^(x - m) dy (logits backward);
+// t = sum p dy (backward).
+template <WideSoftmax OP>
+__global__ __launch_bounds__(kThreads) void softmax_chunks_kernel(
+    const float* __restrict__ a, const float* __restrict__ dy, double* __restrict__ partials,
+    int cols, int chunk, int parts) {
+  __shared__ float mslots[kNW];
+  __shared__ double slots[2][kNW];
+  const Place p = place(partials, cols, chunk, parts);
+  f32x4 v[kVpt], d[kVpt];
+  chunk_load(v, chunk_rsrc(a, p, cols));
+  if (OP != WideSoftmax::kForward) chunk_load(d, chunk_rsrc(dy, p, cols));
+  float m = 0.0f;
+  if (OP != WideSoftmax::kBackward) {
+    float lm = kNegInf;
+#pragma unroll
+    for (int k = 0; k < kVpt; ++k)
+      lm = fmax_nan(lm, max4(rows::keep4(v[k], left_of(p, k), kNegInf)));
+    m = rows::block_max<kNW>(lm, mslots);
+  }
+  double s = 0.0, t = 0.0;
+#pragma unroll
+  for (int k = 0; k < kVpt; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float w = v[k][e];
+      if (OP != WideSoftmax::kBackward) {
+        w = m == kNegInf || left_of(p, k) <= e ? 0.0f : exp_accurate(w - m);
+        s += w;
+      }
+      if (OP != WideSoftmax::kForward) t += static_cast<double>(w * d[k][e]);
+    }
+  rows::block_sum2<kNW>(s, t, slots);
+  if (threadIdx.x == 0) {
+    p.out[0] = m;
+    p.out[p.parts] = s;
+    p.out[2 * p.parts] = t;
+  }
+}
+
+template <WideSoftmax OP>
+__global__ __launch_bounds__(kThreads) void softmax_outputs_kernel(
+    const float* __restrict__ a, const float* __restrict__ dy, float* __restrict__ out,
+    float* __restrict__ rowmax, float* __restrict__ lse, double* __restrict__ partials, int cols,
+    int chunk, int parts) {
+  const Place p = place(partials, cols, chunk, parts);
+  f32x4 v[kVpt], d[kVpt];
+  chunk_load(v, chunk_rsrc(a, p, cols));
+  if (OP != WideSoftmax::kForward) chunk_load(d, chunk_rsrc(dy, p, cols));
+  float m = 0.0f, inv_s = 1.0f, dot = 0.0f;
+  if (OP != WideSoftmax::kBackward) {
+    const double mi = partial(p, 0, -__builtin_inf()), si = partial(p, 1, 0.0);
+    m = wave_reduce(static_cast<float>(mi), MaxOp{});
+    const double f = rescale(mi, m);
+    const double s = wave_reduce_sum_f64(si == 0.0 ? 0.0 : si * f);
+    inv_s = static_cast<float>(1.0 / s);
+    if (OP == WideSoftmax::kLogits)
+      dot = static_cast<float>(wave_reduce_sum_f64(partial(p, 2, 0.0) * f) / s);
+    if (OP == WideSoftmax::kForward && p.part == 0 && threadIdx.x == 0) {
+      rowmax[p.row] = m;
+      lse[p.row] = static_cast<float>(static_cast<double>(m) + ::log(s));
+    }
+  } else {
+    dot = static_cast<float>(wave_reduce_sum_f64(partial(p, 2, 0.0)));
+  }
+  const buffer_rsrc_t r = chunk_rsrc(out, p, cols);
+#pragma unroll
+  for (int k = 0; k < kVpt; ++k) {
+    f32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float w =
+          OP == WideSoftmax::kBackward ? v[k][e] : exp_accurate(v[k][e] - m) * inv_s;
+      o[e] = OP == WideSoftmax::kForward ? w : w * (d[k][e] - dot);
+    }
+    rows::row_store(r, (threadIdx.x + k * kThreads) * 16u, o);
+  }
+}
+
+// -------------------------------------------------------- quantisation ----
+__global__ __launch_bounds__(kThreads) void quant_chunks_kernel(const float* __restrict__ x,
+                                                                double* __restrict__ partials,
+                                                                int cols, int chunk, int parts) {
+  __shared__ float mslots[kNW];
+  const Place p = place(partials, cols, chunk, parts);
+  f32x4 v[kVpt];
+  chunk_load(v, chunk_rsrc(x, p, cols));
+  float lm = 0.0f;  // |x| >= 0, and past the chunk x reads 0
+#pragma unroll
+  for (int k = 0; k < kVpt; ++k)
+    lm = fmax_nan(lm, absmax4(v[k]));
+  const float m = rows::block_max<kNW>(lm, mslots);
+  if (threadIdx.x == 0) p.out[0] = m;
+}
+
+__global__ __launch_bounds__(kThreads) void quant_outputs_kernel(
+    const float* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scale,
+    double* __restrict__ partials, int cols, int chunk, int parts) {
+  const Place p = place(partials, cols, chunk, parts);
+  f32x4 v[kVpt];
+  chunk_load(v, chunk_rsrc(x, p, cols));
+  const float m = wave_reduce(static_cast<float>(partial(p, 0, 0.0)), MaxOp{});
+  const float inv = inv_scale(m);
+  int8_t* qr = q + static_cast<size_t>(p.row) * cols + p.c0;
+#pragma unroll
+  for (int k = 0; k < kVpt; ++k) {
+    const int left = left_of(p, k);
+    int8_t* dst = qr + 4 * (threadIdx.x + k * kThreads);
+    if (left >= 4) {
+      store_codes(dst, quant4(v[k], inv));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 3; ++e)
+        if (left > e) dst[e] = code1(v[k][e], inv);
+    }
+  }
+  if (p.part == 0 && threadIdx.x == 0) scale[p.row] = m / 127.0f;
+}
+
+// -------------------------------------------------- LayerNorm backward ----
+// Partials about the row's first element x0, in fp64: sum(x - x0),
+// sum((x - x0)^2), sum g and sum g (x - x0) with g = dy * gamma; with d the
+// mean less x0, sum g xhat = rstd (sum g (x - x0) - d sum g).
+__global__ __launch_bounds__(kThreads) void layernorm_bwd_chunks_kernel(
+    const float* __restrict__ x, const float* __restrict__ dy, const float* __restrict__ gamma,
+    double* __restrict__ partials, int cols, int chunk, int parts) {
+  __shared__ double slots[2][2][kNW];
+  const Place p = place(partials, cols, chunk, parts);
+  f32x4 v[kVpt], d[kVpt], g[kVpt];
+  chunk_load(v, chunk_rsrc(x, p, cols));
+  chunk_load(d, chunk_rsrc(dy, p, cols));
+  chunk_load(g, make_rsrc(gamma + p.c0, static_cast<uint32_t>(p.n) * 4u));
+  const float x0 = x[static_cast<size_t>(p.row) * cols];
+  double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
+#pragma unroll
+  for (int k = 0; k < kVpt; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const double c = left_of(p, k) > e ? static_cast<double>(v[k][e]) - x0 : 0.0;
+      const double gg = d[k][e] * g[k][e];  // 0 past the chunk
+      s1 += c;
+      s2 += c * c;
+      s3 += gg;
+      s4 += gg * c;
+    }
+  rows::block_sum2<kNW>(s1, s2, slots[0]);
+  rows::block_sum2<kNW>(s3, s4, slots[1]);
+  if (threadIdx.x == 0) {
+    p.out[0] = s1;
+    p.out[p.parts] = s2;
+    p.out[2 * p.parts] = s3;
+    p.out[3 * p.parts] = s4;
+    p.out[4 * p.parts] = x0;
+  }
+}
+
+__global__ __launch_bounds__(kThreads) void layernorm_bwd_outputs_kernel(
+    const float* __restrict__ x, const float* __restrict__ dy, const float* __restrict__ gamma,
+    float* __restrict__ dx, double* __restrict__ partials, int cols, int chunk, int parts,
+    float eps) {
+  const Place p = place(partials, cols, chunk, parts);
+  f32x4 v[kVpt], d[kVpt], g[kVpt];
+  chunk_load(v, chunk_rsrc(x, p, cols));
+  chunk_load(d, chunk_rsrc(dy, p, cols));
+  chunk_load(g, make_rsrc(gamma + p.c0, static_cast<uint32_t>(p.n) * 4u));
+  const double x0 = p.row_partials[4 * p.parts];  // dx may be x: not from x
+  double s[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) s[k] = wave_reduce_sum_f64(partial(p, k, 0.0));
+  const double off = s[0] / cols;
+  const double var = s[1] / cols - off * off;
+  const double rs = 1.0 / __builtin_sqrt((var < 0.0 ? 0.0 : var) + eps);  // NaN stays NaN
+  const float mean = static_cast<float>(x0 + off);
+  const float rstd = static_cast<float>(rs);
+  const float mg = static_cast<float>(s[2] / cols);
+  const float mgx = static_cast<float>(rs * (s[3] - off * s[2]) / cols);
+  const buffer_rsrc_t r = chunk_rsrc(dx, p, cols);
+#pragma unroll
+  for (int k = 0; k < kVpt; ++k) {
+    f32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float xh = (v[k][e] - mean) * rstd;
+      o[e] = (d[k][e] * g[k][e] - mg - xh * mgx) * rstd;
+    }
+    rows::row_store(r, (threadIdx.x + k * kThreads) * 16u, o);
+  }
+}
+
+// ---------------------------------------------------------------- host ----
+// The partials live in a buffer per (device, stream) of their own (5 MiB, for
+// the first kMaxStreams of them, kept while the process runs): calls that
+// brought no workspace before bring none now and share none with the other
+// operations.  One call's two launches stay together under pair_mutex when
+// threads share a stream.
+constexpr size_t kMaxStreams = 64;
+constexpr size_t kPartialBytes = size_t{kMaxRows} * kMaxParts * kValues * sizeof(double);
+struct PartialAlloc {
+  int operator()(int, void*, size_t bytes, char** out) const {
+    // Relaxed: another thread's stream may be under capture meanwhile.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    void* p = nullptr;
+    const hipError_t err = hipMalloc(&p, bytes);
+    if (err != hipSuccess) (void)hipGetLastError();
+    CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+    if (err != hipSuccess) return CREDIT_ERR_HIP;
+    *out = static_cast<char*>(p);
+    return CREDIT_OK;
+  }
+};
+std::mutex& pair_mutex() {
+  static std::mutex* m = new std::mutex();
+  return *m;
+}
+
+struct WidePlan {
+  dim3 grid;
+  int chunk = 0, parts = 0;
+  double* partials = nullptr;
+};
+
+// Where AUTO takes this path.  Ragged rows of up to kFewWide rows leave most of
+// the chip idle on a workgroup each: from 16384 columns on (8195: the same or
+// 0.4 us slower; quantisation, one pass of a narrow output, from 32768).  More
+// rows fill it, and the kernels that hold a row in registers read it once
+// (softmax logits backward 256 x 40003: 30 us, 33.5 here); past `many` columns
+// they stream it more than once, or so few rows fit that latency shows
+// (LayerNorm backward 384 x 40003: 76 us, 49 here).  Rows of whole 16-byte
+// vectors have faster kernels, SPLIT among them: at most 32 rows, wide ones and
+// little data (softmax forward 16 x 16384: 6.0 us, 6.9 here; 16 x 65536: 16,
+// 7.4; logits backward 64 x 32768: 9.4, 10.1; 64 x 131072: 22, 27).  16 x
+// 262144 would gain too (forward 13.4, 9.9 here) but AUTO is known to run SPLIT
+// there (credit_last_split_shape).  A caller's workspace is SPLIT's.
+struct WideRule {
+  int64_t few, many, vec;  // columns, exclusive
+};
+constexpr WideRule kSoftmaxFwdRule{16384, 32768, 24576};
+constexpr WideRule kSoftmaxBwdRule{16384, 53248, 24576};
+constexpr WideRule kLayerNormRule{16384, 32768, 24576};
+constexpr WideRule kQuantRule{32768, 65536, 98304};
+constexpr int64_t kFewWide = 128;
+bool wide_wanted(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_t cols,
+                 bool vec) {
+  if (cfg_variant(cfg) != CREDIT_VARIANT_AUTO || rows > kMaxRows ||
+      cols > int64_t{kMaxParts} * kChunk)
+    return false;
+  if (vec)
+    return (cfg == nullptr || cfg->workspace == nullptr) && rows <= 32 && cols > rule.vec &&
+           rows * cols <= int64_t{1} << 21;
+  return cols > (rows <= kFewWide ? rule.few : rule.many);
+}
+
+// Chunks per row: enough workgroups for three to a CU, at least 1024 columns
+// and at most kChunk each.  Holds the pair's lock from then on.  False: the
+// call's other kernels take it.
+bool wide_plan(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_t cols, bool vec,
+               WidePlan* plan, std::unique_lock<std::mutex>* lock) {
+  if (!wide_wanted(rule, cfg, rows, cols, vec)) return false;
+  const int64_t least = (cols + kChunk - 1) / kChunk;
+  const int64_t most = std::min<int64_t>(kMaxParts, std::max<int64_t>(least, cols / 1024));
+  const int64_t want = std::clamp<int64_t>((768 + rows - 1) / rows, least, most);
+  plan->chunk = static_cast<int>(((cols + want - 1) / want + 3) / 4 * 4);
+  plan->parts = static_cast<int>((cols + plan->chunk - 1) / plan->chunk);
+  plan->grid = dim3(static_cast<unsigned>(plan->parts), static_cast<unsigned>(rows));
+  static WorkspaceCache<PartialAlloc>* cache = new WorkspaceCache<PartialAlloc>();
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  hipStream_t stream = cfg_stream(cfg);
+  if (!keeps_scratch(stream)) return false;
+  *lock = std::unique_lock<std::mutex>(pair_mutex());
+  char* base = nullptr;
+  if (!cache->room(dev, stream, kMaxStreams) ||
+      cache->get(dev, stream, kPartialBytes, &base) != CREDIT_OK)
+    return false;
+  plan->partials = reinterpret_cast<double*>(base);
+  return true;
+}
+
+template <WideSoftmax OP>
+int launch_softmax(const WidePlan& w, const float* a, const float* dy, float* out, float* rowmax,
+                   float* lse, int cols, hipStream_t stream) {
+  softmax_chunks_kernel<OP><<<w.grid, kThreads, 0, stream>>>(a, dy, w.partials, cols, w.chunk,
+                                                             w.parts);
+  CREDIT_TRY(check_launch("softmax_chunks_kernel"));
+  softmax_outputs_kernel<OP><<<w.grid, kThreads, 0, stream>>>(a, dy, out, rowmax, lse, w.partials,
+                                                              cols, w.chunk, w.parts);
+  return check_launch("softmax_outputs_kernel");
+}
+
+}  // namespace
+
+int wide_softmax(WideSoftmax op, const float* a, const float* dy, float* out, float* rowmax,
+                 float* lse, int64_t rows, int64_t cols, bool vec, const credit_cfg* cfg,
+                 bool* taken) {
+  const WideRule& rule = op == WideSoftmax::kForward ? kSoftmaxFwdRule : kSoftmaxBwdRule;
+  std::unique_lock<std::mutex> lock;
+  WidePlan w;
+  if (!(*taken = wide_plan(rule, cfg, rows, cols, vec, &w, &lock))) return CREDIT_OK;
+  hipStream_t s = cfg_stream(cfg);
+  const int c = static_cast<int>(cols);
+  switch (op) {
+    case WideSoftmax::kForward:
+      return launch_softmax<WideSoftmax::kForward>(w, a, dy, out, rowmax, lse, c, s);
+    case WideSoftmax::kBackward:
+      return launch_softmax<WideSoftmax::kBackward>(w, a, dy, out, rowmax, lse, c, s);
+    default:
+      return launch_softmax<WideSoftmax::kLogits>(w, a, dy, out, rowmax, lse, c, s);
+  }
+}
+
+int wide_quant(const float* x, int8_t* q, float* scale, int64_t rows, int64_t cols, bool vec,
+               const credit_cfg* cfg, bool* taken) {
+  std::unique_lock<std::mutex> lock;
+  WidePlan w;
+  if (!(*taken = wide_plan(kQuantRule, cfg, rows, cols, vec, &w, &lock))) return CREDIT_OK;
+  hipStream_t s = cfg_stream(cfg);
+  const int c = static_cast<int>(cols);
+  quant_chunks_kernel<<<w.grid, kThreads, 0, s>>>(x, w.partials, c, w.chunk, w.parts);
+  CREDIT_TRY(check_launch("quant_chunks_kernel"));
+  quant_outputs_kernel<<<w.grid, kThreads, 0, s>>>(x, q, scale, w.partials, c, w.chunk, w.parts);
+  return check_launch("quant_outputs_kernel");
+}
+
+int wide_layernorm_bwd(const float* x, const float* dy, const float* gamma, float* dx, int64_t rows,
+                       int64_t cols, float eps, bool vec, const credit_cfg* cfg, bool* taken) {
+  std::unique_lock<std::mutex> lock;
+  WidePlan w;
+  if (!(*taken = wide_plan(kLayerNormRule, cfg, rows, cols, vec, &w, &lock))) return CREDIT_OK;
+  hipStream_t s = cfg_stream(cfg);
+  const int c = static_cast<int>(cols);
+  layernorm_bwd_chunks_kernel<<<w.grid, kThreads, 0, s>>>(x, dy, gamma, w.partials, c, w.chunk,
+                                                          w.parts);
+  CREDIT_TRY(check_launch("layernorm_bwd_chunks_kernel"));
+  layernorm_bwd_outputs_kernel<<<w.grid, kThreads, 0, s>>>(x, dy, gamma, dx, w.partials, c,
+                                                           w.chunk, w.parts, eps);
+  return check_launch("layernorm_bwd_outputs_kernel");
+}
+
+}  // namespace credit

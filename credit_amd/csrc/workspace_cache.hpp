@@ -68,6 +68,12 @@ class WorkspaceCache {
     return e == nullptr ? 0 : e->buf.bytes;
   }
 
+  // Whether (device, stream) has an entry, or may have one of at most `most`.
+  bool room(int device, void* stream, size_t most) {
+    std::lock_guard<std::mutex> lock(mu_);
+    return find(device, stream) != nullptr || entries_.size() < most;
+  }
+
   // Every live buffer (for maintenance that must reach all of them).
   std::vector<WsBuffer> live() {
     std::lock_guard<std::mutex> lock(mu_);

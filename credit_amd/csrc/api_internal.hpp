@@ -244,7 +244,7 @@ size_t rmsnorm_bwd_workspace(int64_t rows, int64_t cols, int variant, int split,
 size_t rmsnorm_fused_workspace(int64_t rows, int64_t cols, int variant, int split,
                                int cu_count);
 
-// Few wide fp32 rows in two launches (widerows.hip).  `vec`: every buffer takes
+// Few wide rows in two launches (widerows.hip).  `vec`: every buffer takes
 // 16-byte vectors.  *taken false: the call's other kernels run it.
 enum class WideSoftmax { kForward, kBackward, kLogits };
 int wide_softmax(WideSoftmax op, const float* a, const float* dy, float* out, float* rowmax,
@@ -252,8 +252,13 @@ int wide_softmax(WideSoftmax op, const float* a, const float* dy, float* out, fl
                  bool* taken);
 int wide_quant(const float* x, int8_t* q, float* scale, int64_t rows, int64_t cols, bool vec,
                const credit_cfg* cfg, bool* taken);
-int wide_layernorm_bwd(const float* x, const float* dy, const float* gamma, float* dx, int64_t rows,
-                       int64_t cols, float eps, bool vec, const credit_cfg* cfg, bool* taken);
+// bf16: buffers at 4-byte addresses.
+template <class T>
+int wide_layernorm_bwd(const T* x, const T* dy, const T* gamma, T* dx, int64_t rows, int64_t cols,
+                       float eps, bool vec, const credit_cfg* cfg, bool* taken);
+int wide_layernorm_fwd(const uint16_t* x, const uint16_t* gamma, const uint16_t* beta,
+                       uint16_t* y, float* mean, float* rstd, int64_t rows, int64_t cols,
+                       float eps, bool vec, const credit_cfg* cfg, bool* taken);
 
 // CU count of the current device, or 256 (MI355X) when none is visible.
 int cu_count_or_default();

@@ -677,6 +677,11 @@ extern "C" int credit_layernorm_fwd_bf16(const uint16_t* x, const uint16_t* gamm
   for (const void* p : {static_cast<const void*>(x), static_cast<const void*>(gamma),
                         static_cast<const void*>(beta), static_cast<const void*>(y)})
     dwords = dwords && reinterpret_cast<uintptr_t>(p) % 4 == 0;
+  bool taken = false;
+  if (dwords)
+    CREDIT_TRY(wide_layernorm_fwd(x, gamma, beta, y, mean, rstd, rows, cols, eps, vec_ok, cfg,
+                                  &taken));
+  if (taken) return CREDIT_OK;
   if (!vec_ok && dwords && cfg_variant(cfg) == CREDIT_VARIANT_AUTO) {
     const auto* rp = cols % 2 != 0 ? rows::rows_pick(RowsTable<true>::table, rows, cols)
                                    : rows::rows_pick(RowsTable<false>::table, rows, cols);

@@ -754,22 +754,21 @@ int layernorm_bwd(const T* x, const T* dy, const T* gamma, T* dx, int64_t rows, 
   for (const void* p : {static_cast<const void*>(x), static_cast<const void*>(dy),
                         static_cast<const void*>(gamma), static_cast<const void*>(dx)})
     vec = vec && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+  // Buffers at 4-byte addresses (the 16-byte layout's among them).
+  bool dwords = rows <= (int64_t{1} << 30);
+  for (const void* p : {static_cast<const void*>(x), static_cast<const void*>(dy),
+                        static_cast<const void*>(gamma), static_cast<const void*>(dx)})
+    dwords = dwords && reinterpret_cast<uintptr_t>(p) % 4 == 0;
+  bool taken = false;
+  if (dwords)
+    CREDIT_TRY(wide_layernorm_bwd(x, dy, gamma, dx, rows, cols, eps, vec, cfg, &taken));
+  if (taken) return CREDIT_OK;
   if constexpr (std::is_same_v<T, uint16_t>) {
     if (const int p = ln_group_members(cfg, cols / E, vec))
       return layernorm_bwd_group(x, dy, gamma, dx, rows, cols, eps, p, cfg);
   }
   hipStream_t stream = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
-  if constexpr (std::is_same_v<T, float>) {
-    bool taken = false;
-    CREDIT_TRY(wide_layernorm_bwd(x, dy, gamma, dx, rows, cols, eps, vec, cfg, &taken));
-    if (taken) return CREDIT_OK;
-  }
-  // Buffers at 4-byte addresses without the 16-byte layout.
-  bool dwords = rows <= (int64_t{1} << 30);
-  for (const void* p : {static_cast<const void*>(x), static_cast<const void*>(dy),
-                        static_cast<const void*>(gamma), static_cast<const void*>(dx)})
-    dwords = dwords && reinterpret_cast<uintptr_t>(p) % 4 == 0;
   if (!vec && dwords && cfg_variant(cfg) == CREDIT_VARIANT_AUTO) {
     const rows::RowsPick<RowsFn<T>>* pick = rows::rows_pick(RowsTable<T, false>::table, rows, cols);
     if constexpr (std::is_same_v<T, uint16_t>) {

@@ -52,18 +52,26 @@ struct HalfRow {
   uint32_t shift;        // 16 on an odd row, else 0
   uint32_t last;         // the row's last element (ODD loads)
 };
+// `n` elements (0: none) from element `at` on; more: the row goes on behind
+// them (n a multiple of 8), so that an odd start's last dword, half of it the
+// next element's, may be read whole.
+template <bool ODD, bool LOAD>
+__device__ __forceinline__ HalfRow half_span(const uint16_t* base, size_t at, uint32_t n,
+                                             bool more) {
+  const uint32_t odd = ODD ? static_cast<uint32_t>(at) & 1u : 0u;
+  const uint32_t bytes = n > 0 ? (n + odd) * 2u : 0u;
+  HalfRow r;
+  r.dwords = make_rsrc(base + at - odd, (bytes + (ODD && more ? 2u : 0u)) & ~3u);
+  r.halves = make_rsrc(base + at - odd, bytes);
+  r.shift = odd * 16u;
+  r.last = ODD && LOAD && n > 0 ? base[at + n - 1] : 0u;
+  return r;
+}
 template <bool ODD, bool LOAD>
 __device__ __forceinline__ HalfRow half_row(const uint16_t* base, int row, int rows, int cols) {
   const bool live = row < rows;
-  const size_t at = static_cast<size_t>(live ? row : 0) * cols;
-  const uint32_t odd = ODD ? static_cast<uint32_t>(at) & 1u : 0u;
-  const uint32_t bytes = live ? (static_cast<uint32_t>(cols) + odd) * 2u : 0u;
-  HalfRow r;
-  r.dwords = make_rsrc(base + at - odd, bytes & ~3u);
-  r.halves = make_rsrc(base + at - odd, bytes);
-  r.shift = odd * 16u;
-  r.last = ODD && LOAD && live ? base[at + cols - 1] : 0u;
-  return r;
+  return half_span<ODD, LOAD>(base, static_cast<size_t>(live ? row : 0) * cols,
+                              live ? static_cast<uint32_t>(cols) : 0u, false);
 }
 // Elements 8 i .. 8 i + 7 of the row, off = 16 i, left = cols - 8 i; zeros past
 // the row's end.

@@ -1,4 +1,4 @@
-// Few wide fp32 rows in two launches: each row cut into chunks of at most 4096
+// Few wide rows in two launches: each row cut into chunks of at most 4096
 // columns, one workgroup per chunk.  The first launch leaves every chunk's
 // partial sums (fp64) in memory, the second merges its row's and writes the
 // outputs.  No workgroup waits for another, so the calls need nothing of the
@@ -14,8 +14,12 @@
 //   softmax logits bwd   110 -> 7    21 -> 11     373 -> 265   13.9 -> 10.3
 //   LayerNorm backward   154 -> 7    38 -> 11     466 -> 260   15.1 -> 10.5
 //   quantisation          18 -> 7   9.2 -> 6.6    136 -> 125   11.0 -> 6.8
+// and in bf16      1 x 200003  128 x 40003  1000 x 100002  16 x 131072
+//   LayerNorm fwd   84 -> 7.8   20 -> 11.7   245 -> 105      9.4 -> 7.7
+//   LayerNorm bwd  101 -> 7.3   28 -> 15.5   324 -> 173     12.5 -> 9.2
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "api_internal.hpp"
 #include "common.hpp"
@@ -200,32 +204,170 @@ __global__ __launch_bounds__(kThreads) void quant_outputs_kernel(
   if (p.part == 0 && threadIdx.x == 0) scale[p.row] = m / 127.0f;
 }
 
-// -------------------------------------------------- LayerNorm backward ----
-// Partials about the row's first element x0, in fp64: sum(x - x0),
-// sum((x - x0)^2), sum g and sum g (x - x0) with g = dy * gamma; with d the
+// ----------------------------------------------------------- LayerNorm ----
+// 16 elements of a chunk per lane, as floats: four fp32 vectors or two bf16
+// ones (ODD: bf16 rows of odd width).
+template <class T, bool ODD>
+struct Lanes {
+  static constexpr int kN = std::is_same_v<T, float> ? 4 : 8;  // elements a vector
+  static constexpr int kV = 16 / kN;
+  // Elements of the chunk from the lane's k-th vector on.
+  __device__ static int left(const Place& p, int k) {
+    return p.n - kN * static_cast<int>(threadIdx.x + k * kThreads);
+  }
+  // Zeros past the chunk.
+  __device__ static void load(float (&f)[16], const T* base, size_t at, const Place& p,
+                              bool more) {
+    if constexpr (kN == 4) {
+      const buffer_rsrc_t r = make_rsrc(base + at, static_cast<uint32_t>(p.n) * 4u);
+#pragma unroll
+      for (int k = 0; k < kV; ++k) {
+        const f32x4 v =
+            __builtin_bit_cast(f32x4, buffer_load(r, (threadIdx.x + k * kThreads) * 16u));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[4 * k + e] = v[e];
+      }
+    } else {
+      const rows::HalfRow r =
+          rows::half_span<ODD, true>(base, at, static_cast<uint32_t>(p.n), more);
+#pragma unroll
+      for (int k = 0; k < kV; ++k) {
+        const u32x4 v =
+            rows::half_load<ODD, false>(r, (threadIdx.x + k * kThreads) * 16u, left(p, k));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          f[8 * k + 2 * e] = bf16_lo(v[e]);
+          f[8 * k + 2 * e + 1] = bf16_hi(v[e]);
+        }
+      }
+    }
+  }
+  __device__ static void store(const float (&f)[16], T* base, size_t at, const Place& p) {
+    if constexpr (kN == 4) {
+      const buffer_rsrc_t r = make_rsrc(base + at, static_cast<uint32_t>(p.n) * 4u);
+#pragma unroll
+      for (int k = 0; k < kV; ++k)
+        rows::row_store(r, (threadIdx.x + k * kThreads) * 16u,
+                        f32x4{f[4 * k], f[4 * k + 1], f[4 * k + 2], f[4 * k + 3]});
+    } else {
+      const rows::HalfRow r =
+          rows::half_span<ODD, false>(base, at, static_cast<uint32_t>(p.n), false);
+#pragma unroll
+      for (int k = 0; k < kV; ++k) {
+        u32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = pack_bf16x2(f[8 * k + 2 * e], f[8 * k + 2 * e + 1]);
+        rows::half_store<ODD>(r, (threadIdx.x + k * kThreads) * 16u, left(p, k), v);
+      }
+    }
+  }
+  __device__ static float first(const T* row) {
+    if constexpr (kN == 4)
+      return *row;
+    else
+      return bf16_to_f32(*row);
+  }
+};
+
+// Partials about the row's first element x0, in fp64: sum(x - x0) and
+// sum((x - x0)^2).
+template <class L>
+__device__ __forceinline__ void deviations(const float (&x)[16], float x0, const Place& p,
+                                           double* s1, double* s2) {
+  *s1 = *s2 = 0.0;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const double c =
+        L::left(p, j / L::kN) > j % L::kN ? static_cast<double>(x[j]) - x0 : 0.0;
+    *s1 += c;
+    *s2 += c * c;
+  }
+}
+struct RowStats {
+  double off;  // the mean less x0
+  float mean, rstd;
+  double rs;
+};
+// From partials 0 and 1; x0 is kept in the last (dx may be x: not from x).
+__device__ __forceinline__ RowStats row_stats(const Place& p, int cols, float eps) {
+  RowStats st;
+  st.off = wave_reduce_sum_f64(partial(p, 0, 0.0)) / cols;
+  const double var = wave_reduce_sum_f64(partial(p, 1, 0.0)) / cols - st.off * st.off;
+  st.rs = 1.0 / __builtin_sqrt((var < 0.0 ? 0.0 : var) + eps);  // NaN stays NaN
+  st.mean = static_cast<float>(p.row_partials[(kValues - 1) * p.parts] + st.off);
+  st.rstd = static_cast<float>(st.rs);
+  return st;
+}
+
+template <bool ODD>
+__global__ __launch_bounds__(kThreads) void layernorm_fwd_chunks_kernel(
+    const uint16_t* __restrict__ x, double* __restrict__ partials, int cols, int chunk,
+    int parts) {
+  using L = Lanes<uint16_t, ODD>;
+  __shared__ double slots[2][kNW];
+  const Place p = place(partials, cols, chunk, parts);
+  const size_t at = static_cast<size_t>(p.row) * cols;
+  float v[16];
+  L::load(v, x, at + p.c0, p, p.part + 1 < parts);
+  const float x0 = L::first(x + at);
+  double s1, s2;
+  deviations<L>(v, x0, p, &s1, &s2);
+  rows::block_sum2<kNW>(s1, s2, slots);
+  if (threadIdx.x == 0) {
+    p.out[0] = s1;
+    p.out[p.parts] = s2;
+    p.out[(kValues - 1) * p.parts] = x0;
+  }
+}
+
+template <bool ODD>
+__global__ __launch_bounds__(kThreads) void layernorm_fwd_outputs_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma,
+    const uint16_t* __restrict__ beta, uint16_t* __restrict__ y, float* __restrict__ mean_out,
+    float* __restrict__ rstd_out, double* __restrict__ partials, int cols, int chunk, int parts,
+    float eps) {
+  using L = Lanes<uint16_t, ODD>;
+  const Place p = place(partials, cols, chunk, parts);
+  const size_t at = static_cast<size_t>(p.row) * cols + p.c0;
+  const bool more = p.part + 1 < parts;
+  float v[16], g[16], b[16];
+  L::load(v, x, at, p, more);
+  L::load(g, gamma, p.c0, p, more);
+  L::load(b, beta, p.c0, p, more);
+  const RowStats st = row_stats(p, cols, eps);
+#pragma unroll
+  for (int j = 0; j < 16; ++j) v[j] = (v[j] - st.mean) * st.rstd * g[j] + b[j];
+  L::store(v, y, at, p);
+  if (p.part == 0 && threadIdx.x == 0) {
+    mean_out[p.row] = st.mean;
+    rstd_out[p.row] = st.rstd;
+  }
+}
+
+// Two partials more, with g = dy * gamma: sum g and sum g (x - x0); with d the
 // mean less x0, sum g xhat = rstd (sum g (x - x0) - d sum g).
+template <class T, bool ODD>
 __global__ __launch_bounds__(kThreads) void layernorm_bwd_chunks_kernel(
-    const float* __restrict__ x, const float* __restrict__ dy, const float* __restrict__ gamma,
+    const T* __restrict__ x, const T* __restrict__ dy, const T* __restrict__ gamma,
     double* __restrict__ partials, int cols, int chunk, int parts) {
+  using L = Lanes<T, ODD>;
   __shared__ double slots[2][2][kNW];
   const Place p = place(partials, cols, chunk, parts);
-  f32x4 v[kVpt], d[kVpt], g[kVpt];
-  chunk_load(v, chunk_rsrc(x, p, cols));
-  chunk_load(d, chunk_rsrc(dy, p, cols));
-  chunk_load(g, make_rsrc(gamma + p.c0, static_cast<uint32_t>(p.n) * 4u));
-  const float x0 = x[static_cast<size_t>(p.row) * cols];
-  double s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0;
+  const size_t at = static_cast<size_t>(p.row) * cols;
+  const bool more = p.part + 1 < parts;
+  float v[16], d[16], g[16];
+  L::load(v, x, at + p.c0, p, more);
+  L::load(d, dy, at + p.c0, p, more);
+  L::load(g, gamma, p.c0, p, more);
+  const float x0 = L::first(x + at);
+  double s1, s2, s3 = 0.0, s4 = 0.0;
+  deviations<L>(v, x0, p, &s1, &s2);
 #pragma unroll
-  for (int k = 0; k < kVpt; ++k)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const double c = left_of(p, k) > e ? static_cast<double>(v[k][e]) - x0 : 0.0;
-      const double gg = d[k][e] * g[k][e];  // 0 past the chunk
-      s1 += c;
-      s2 += c * c;
-      s3 += gg;
-      s4 += gg * c;
-    }
+  for (int j = 0; j < 16; ++j) {
+    const double gg = d[j] * g[j];  // 0 past the chunk
+    s3 += gg;
+    s4 += gg * (static_cast<double>(v[j]) - x0);
+  }
   rows::block_sum2<kNW>(s1, s2, slots[0]);
   rows::block_sum2<kNW>(s3, s4, slots[1]);
   if (threadIdx.x == 0) {
@@ -233,41 +375,34 @@ __global__ __launch_bounds__(kThreads) void layernorm_bwd_chunks_kernel(
     p.out[p.parts] = s2;
     p.out[2 * p.parts] = s3;
     p.out[3 * p.parts] = s4;
-    p.out[4 * p.parts] = x0;
+    p.out[(kValues - 1) * p.parts] = x0;
   }
 }
 
+template <class T, bool ODD>
 __global__ __launch_bounds__(kThreads) void layernorm_bwd_outputs_kernel(
-    const float* __restrict__ x, const float* __restrict__ dy, const float* __restrict__ gamma,
-    float* __restrict__ dx, double* __restrict__ partials, int cols, int chunk, int parts,
+    const T* __restrict__ x, const T* __restrict__ dy, const T* __restrict__ gamma,
+    T* __restrict__ dx, double* __restrict__ partials, int cols, int chunk, int parts,
     float eps) {
+  using L = Lanes<T, ODD>;
   const Place p = place(partials, cols, chunk, parts);
-  f32x4 v[kVpt], d[kVpt], g[kVpt];
-  chunk_load(v, chunk_rsrc(x, p, cols));
-  chunk_load(d, chunk_rsrc(dy, p, cols));
-  chunk_load(g, make_rsrc(gamma + p.c0, static_cast<uint32_t>(p.n) * 4u));
-  const double x0 = p.row_partials[4 * p.parts];  // dx may be x: not from x
-  double s[4];
+  const size_t at = static_cast<size_t>(p.row) * cols + p.c0;
+  const bool more = p.part + 1 < parts;
+  float v[16], d[16], g[16];
+  L::load(v, x, at, p, more);
+  L::load(d, dy, at, p, more);
+  L::load(g, gamma, p.c0, p, more);
+  const RowStats st = row_stats(p, cols, eps);
+  const double b1 = wave_reduce_sum_f64(partial(p, 2, 0.0));
+  const double b2 = wave_reduce_sum_f64(partial(p, 3, 0.0));
+  const float mg = static_cast<float>(b1 / cols);
+  const float mgx = static_cast<float>(st.rs * (b2 - st.off * b1) / cols);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) s[k] = wave_reduce_sum_f64(partial(p, k, 0.0));
-  const double off = s[0] / cols;
-  const double var = s[1] / cols - off * off;
-  const double rs = 1.0 / __builtin_sqrt((var < 0.0 ? 0.0 : var) + eps);  // NaN stays NaN
-  const float mean = static_cast<float>(x0 + off);
-  const float rstd = static_cast<float>(rs);
-  const float mg = static_cast<float>(s[2] / cols);
-  const float mgx = static_cast<float>(rs * (s[3] - off * s[2]) / cols);
-  const buffer_rsrc_t r = chunk_rsrc(dx, p, cols);
-#pragma unroll
-  for (int k = 0; k < kVpt; ++k) {
-    f32x4 o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float xh = (v[k][e] - mean) * rstd;
-      o[e] = (d[k][e] * g[k][e] - mg - xh * mgx) * rstd;
-    }
-    rows::row_store(r, (threadIdx.x + k * kThreads) * 16u, o);
+  for (int j = 0; j < 16; ++j) {
+    const float xh = (v[j] - st.mean) * st.rstd;
+    v[j] = (d[j] * g[j] - mg - xh * mgx) * st.rstd;
   }
+  L::store(v, dx, at, p);
 }
 
 // ---------------------------------------------------------------- host ----
@@ -314,13 +449,17 @@ struct WidePlan {
 // little data (softmax forward 16 x 16384: 6.0 us, 6.9 here; 16 x 65536: 16,
 // 7.4; logits backward 64 x 32768: 9.4, 10.1; 64 x 131072: 22, 27).  16 x
 // 262144 would gain too (forward 13.4, 9.9 here) but AUTO is known to run SPLIT
-// there (credit_last_split_shape).  A caller's workspace is SPLIT's.
+// there (credit_last_split_shape).  A caller's workspace is SPLIT's.  bf16 rows
+// are half the bytes: LayerNorm forward 16 x 16386 7.1 us, 7.6 here, 64 x 16387
+// 9.6, 8.5; aligned 16 x 32768 5.5, 7.2, 32 x 65536 8.5, 7.0.
 struct WideRule {
   int64_t few, many, vec;  // columns, exclusive
 };
 constexpr WideRule kSoftmaxFwdRule{16384, 32768, 24576};
 constexpr WideRule kSoftmaxBwdRule{16384, 53248, 24576};
-constexpr WideRule kLayerNormRule{16384, 32768, 24576};
+constexpr WideRule kLnBwdRule{16384, 32768, 24576};
+constexpr WideRule kLnBwdHalfRule{16384, 32768, 49152};
+constexpr WideRule kLnFwdRule{20480, 32768, 49152};
 constexpr WideRule kQuantRule{32768, 65536, 98304};
 constexpr int64_t kFewWide = 128;
 bool wide_wanted(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_t cols,
@@ -343,7 +482,7 @@ bool wide_plan(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_
   const int64_t least = (cols + kChunk - 1) / kChunk;
   const int64_t most = std::min<int64_t>(kMaxParts, std::max<int64_t>(least, cols / 1024));
   const int64_t want = std::clamp<int64_t>((768 + rows - 1) / rows, least, most);
-  plan->chunk = static_cast<int>(((cols + want - 1) / want + 3) / 4 * 4);
+  plan->chunk = static_cast<int>(((cols + want - 1) / want + 7) / 8 * 8);
   plan->parts = static_cast<int>((cols + plan->chunk - 1) / plan->chunk);
   plan->grid = dim3(static_cast<unsigned>(plan->parts), static_cast<unsigned>(rows));
   static WorkspaceCache<PartialAlloc>* cache = new WorkspaceCache<PartialAlloc>();
@@ -408,19 +547,53 @@ int wide_quant(const float* x, int8_t* q, float* scale, int64_t rows, int64_t co
   return check_launch("quant_outputs_kernel");
 }
 
-int wide_layernorm_bwd(const float* x, const float* dy, const float* gamma, float* dx, int64_t rows,
-                       int64_t cols, float eps, bool vec, const credit_cfg* cfg, bool* taken) {
+template <class T>
+int wide_layernorm_bwd(const T* x, const T* dy, const T* gamma, T* dx, int64_t rows, int64_t cols,
+                       float eps, bool vec, const credit_cfg* cfg, bool* taken) {
   std::unique_lock<std::mutex> lock;
   WidePlan w;
-  if (!(*taken = wide_plan(kLayerNormRule, cfg, rows, cols, vec, &w, &lock))) return CREDIT_OK;
+  const WideRule& rule = std::is_same_v<T, float> ? kLnBwdRule : kLnBwdHalfRule;
+  if (!(*taken = wide_plan(rule, cfg, rows, cols, vec, &w, &lock))) return CREDIT_OK;
   hipStream_t s = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
-  layernorm_bwd_chunks_kernel<<<w.grid, kThreads, 0, s>>>(x, dy, gamma, w.partials, c, w.chunk,
-                                                          w.parts);
-  CREDIT_TRY(check_launch("layernorm_bwd_chunks_kernel"));
-  layernorm_bwd_outputs_kernel<<<w.grid, kThreads, 0, s>>>(x, dy, gamma, dx, w.partials, c,
-                                                           w.chunk, w.parts, eps);
-  return check_launch("layernorm_bwd_outputs_kernel");
+  const auto launch = [&](auto odd) {
+    constexpr bool kOdd = decltype(odd)::value;
+    layernorm_bwd_chunks_kernel<T, kOdd><<<w.grid, kThreads, 0, s>>>(x, dy, gamma, w.partials, c,
+                                                                     w.chunk, w.parts);
+    CREDIT_TRY(check_launch("layernorm_bwd_chunks_kernel"));
+    layernorm_bwd_outputs_kernel<T, kOdd><<<w.grid, kThreads, 0, s>>>(
+        x, dy, gamma, dx, w.partials, c, w.chunk, w.parts, eps);
+    return check_launch("layernorm_bwd_outputs_kernel");
+  };
+  if constexpr (std::is_same_v<T, uint16_t>) {
+    if (cols % 2 != 0) return launch(std::true_type{});
+  }
+  return launch(std::false_type{});
+}
+template int wide_layernorm_bwd<float>(const float*, const float*, const float*, float*, int64_t,
+                                       int64_t, float, bool, const credit_cfg*, bool*);
+template int wide_layernorm_bwd<uint16_t>(const uint16_t*, const uint16_t*, const uint16_t*,
+                                          uint16_t*, int64_t, int64_t, float, bool,
+                                          const credit_cfg*, bool*);
+
+int wide_layernorm_fwd(const uint16_t* x, const uint16_t* gamma, const uint16_t* beta,
+                       uint16_t* y, float* mean, float* rstd, int64_t rows, int64_t cols,
+                       float eps, bool vec, const credit_cfg* cfg, bool* taken) {
+  std::unique_lock<std::mutex> lock;
+  WidePlan w;
+  if (!(*taken = wide_plan(kLnFwdRule, cfg, rows, cols, vec, &w, &lock))) return CREDIT_OK;
+  hipStream_t s = cfg_stream(cfg);
+  const int c = static_cast<int>(cols);
+  const auto launch = [&](auto odd) {
+    constexpr bool kOdd = decltype(odd)::value;
+    layernorm_fwd_chunks_kernel<kOdd><<<w.grid, kThreads, 0, s>>>(x, w.partials, c, w.chunk,
+                                                                  w.parts);
+    CREDIT_TRY(check_launch("layernorm_fwd_chunks_kernel"));
+    layernorm_fwd_outputs_kernel<kOdd><<<w.grid, kThreads, 0, s>>>(
+        x, gamma, beta, y, mean, rstd, w.partials, c, w.chunk, w.parts, eps);
+    return check_launch("layernorm_fwd_outputs_kernel");
+  };
+  return cols % 2 != 0 ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 }  // namespace credit

@@ -1,10 +1,10 @@
-"""Few wide fp32 rows in two launches of chunks: both sides of the width and row
+"""Few wide rows in two launches of chunks: both sides of the width and row
 rules, the widest row, chunks of a few columns less than the others, a last
 column by itself, whole vectors, outputs in place of an input, special values,
 and a captured call (which takes another kernel).
 
 fp32 within rtol 1e-5 / atol 1e-6 of the float64 oracle (maxima, int8 codes and
-scales bit for bit)."""
+scales bit for bit), bf16 within rtol 1e-2 / atol 1e-2."""
 import numpy as np
 import pytest
 import torch
@@ -12,7 +12,7 @@ import torch
 from credit_amd import hip_lib
 from credit_amd.workloads import WORKLOADS
 from oracle import reference as ref
-from test_gpu_ragged_rows import FP32, check_guards, output, place, sample
+from test_gpu_ragged_rows import BF16, FP32, check_guards, output, place, sample
 
 pytestmark = pytest.mark.gpu
 
@@ -134,3 +134,37 @@ def test_wide_softmax_captured(gpu):
             np.testing.assert_allclose(a.cpu().numpy(), b.cpu().numpy(), **FP32)
     e = ref.softmax_fwd(xs[1].cpu().numpy())
     np.testing.assert_allclose(eager[1][0].cpu().numpy(), e[0], **FP32)
+
+
+# bf16: odd widths (chunks of odd rows start inside a dword), even ones, whole
+# vectors, a last chunk of few elements.
+HALF_SHAPES = [(1, 16385, 0), (4, 20001, 2), (129, 33001, 0), (3, 262143, 0), (2, 262142, 2),
+               (5, 98311, 0), (7, 32770, 0), (32, 24584, 0), (16, 131072, 0), (300, 66003, 0),
+               (6, 40003, 1)]
+
+
+@pytest.mark.parametrize("rows,cols,shift", HALF_SHAPES)
+def test_wide_layernorm_bf16(gpu, rows, cols, shift):
+    print(f"wide bf16 layernorm {rows} x {cols} + {shift}", flush=True)
+    x, gamma, beta = WORKLOADS["layernorm_fwd"].make_inputs(rows, cols, seed=rows + cols)
+    x[: rows // 2] += 3.0
+    xs, gs, bs = (place(t, shift, gpu) for t in (x, gamma, beta))
+    y, gy = output((rows, cols), torch.bfloat16, shift, gpu)
+    mean, rstd = torch.empty(rows, device=gpu), torch.empty(rows, device=gpu)
+    hip_lib.layernorm_fwd(xs, gs, bs, y, mean, rstd, hip_lib.LAYERNORM_EPS, hip_lib.make_cfg())
+    dy = WORKLOADS["layernorm_backward_bf16"].make_inputs(rows, cols, seed=rows + cols)[1]
+    ds = place(dy, shift, gpu)
+    dx, gd = output((rows, cols), torch.bfloat16, shift, gpu)
+    hip_lib.layernorm_backward(xs, ds, gs, dx, hip_lib.LAYERNORM_EPS, hip_lib.make_cfg())
+    torch.cuda.synchronize()
+    check_guards(gy, gd)
+    i = sample(rows)
+    ey, em, er = ref.layernorm_fwd(x[i].float().numpy(), gamma.float().numpy(),
+                                   beta.float().numpy())
+    np.testing.assert_allclose(y[i].float().cpu().numpy(), ey, **BF16)
+    np.testing.assert_allclose(mean[i].cpu().numpy(), em, **FP32)
+    np.testing.assert_allclose(rstd[i].cpu().numpy(), er, **FP32)
+    expect = ref.layernorm_backward(x[i].float().numpy(), dy[i].float().numpy(),
+                                    gamma.float().numpy())
+    np.testing.assert_allclose(dx[i].float().cpu().numpy(), expect, **BF16)
+    assert not bool(torch.isnan(y).any()) and not bool(torch.isnan(dx).any())

@@ -202,42 +202,25 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_fwd_read_kernel(
 }
 
 // ------------------------------------------------------------ backward ---
-// mode of the backward slice kernel: where the row reduction c comes from.
-constexpr int kBwdExchange = 0;  // ticketed group of `members`, one exchange per row
-constexpr int kBwdWhole = 1;     // members == 1: the member holds the whole row
-constexpr int kBwdGiven = 2;     // c precomputed in rowdot[] (READ variant)
-
-// Member `member` of group `group` covers rows [group*R, group*R + R) and
-// vectors [member*chunk, ...) of each.  Per lane: VPT dwordx4 of x and of dy
-// for the current row plus the same for the next row, whose loads are
-// issued before the current row's reduction and exchange wait, so HBM
-// traffic continues through them.  The dw accumulators (8*VPT fp64 per
-// lane) live in LDS, laid out [slot][lane] so each lane's read-add-write
-// touches consecutive banks; that keeps VGPRs low enough for two
-// workgroups per CU.
+// READ's second pass: the row reductions are in rowdot[].  Slice `member` of
+// group `group` covers rows [group*R, group*R + R) and vectors [member*chunk,
+// ...) of each.  Per lane: VPT dwordx4 of x and of dy for the current row plus
+// the same for the next row, so HBM traffic continues through a row's
+// arithmetic.  The dw accumulators (8*VPT fp64 per lane) live in LDS, laid out
+// [slot][lane] so each lane's read-add-write touches consecutive banks; that
+// keeps VGPRs low enough for two workgroups per CU.
 template <int THREADS, int VPT>
-__device__ __forceinline__ void rmsnorm_bwd_slice_kernel_body(
+__global__ __launch_bounds__(THREADS) void rmsnorm_bwd_slice_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
     const uint16_t* __restrict__ dy, const float* __restrict__ rstd,
     const float* __restrict__ rowdot, uint16_t* __restrict__ dx,
     double* __restrict__ dw_part, int rows, int cols, int chunk, int members,
-    int rows_per_group, int mode, SplitArgs sa) {
-  constexpr int NW = THREADS / kWave;
+    int rows_per_group) {
   constexpr int kSlots = 8 * VPT;
   extern __shared__ double dw_lds[];  // [kSlots][THREADS]
-  __shared__ double red[2][NW];
   const int tid = threadIdx.x;
-  SplitGroup g;
-  int group, member;
-  if (mode == kBwdExchange) {
-    g = split_join(sa, members, 1);
-    group = g.group;
-    member = g.member;
-    if (group * rows_per_group >= rows) return;  // padding group
-  } else {
-    group = blockIdx.x / members;
-    member = blockIdx.x - group * members;
-  }
+  const int group = blockIdx.x / members;
+  const int member = blockIdx.x - group * members;
   const int nvec = cols >> 3;
   const int v0 = member * chunk;
   const int vlen = nvec - v0 < chunk ? nvec - v0 : chunk;
@@ -264,23 +247,7 @@ __device__ __forceinline__ void rmsnorm_bwd_slice_kernel_body(
   for (int r = r0; r < r1; ++r) {
     if (r + 1 < r1) load_row(xn, dn, r + 1);
     const float rs = rstd[r];
-    double dot;
-    if (mode == kBwdGiven) {
-      dot = static_cast<double>(rowdot[r]);
-    } else {
-      float part = 0.0f;
-#pragma unroll
-      for (int k = 0; k < VPT; ++k) {
-        const int idx = tid + k * THREADS;
-        if (idx < vlen) part += gx8(xv[k], dv[k], wr[idx]);
-      }
-      dot = block_reduce_sum_f64<NW>(static_cast<double>(part), red[r & 1]);
-      if (mode == kBwdExchange) {
-        if (tid == 0) split_publish(g, 0, dot);
-        split_exchange(g);
-        dot = split_sum(g, 0);
-      }
-    }
+    const double dot = static_cast<double>(rowdot[r]);
     // c = mean(g * xhat) = rs * sum(dy*w*x) / cols
     const float c = static_cast<float>(dot * rs / cols);
     const double rsd = static_cast<double>(rs);
@@ -320,17 +287,6 @@ __device__ __forceinline__ void rmsnorm_bwd_slice_kernel_body(
       q[3] = f64x2{a[6 * THREADS], a[7 * THREADS]};
     }
   }
-}
-
-template <int THREADS, int VPT>
-__global__ __launch_bounds__(THREADS) void rmsnorm_bwd_slice_kernel(
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-    const uint16_t* __restrict__ dy, const float* __restrict__ rstd,
-    const float* __restrict__ rowdot, uint16_t* __restrict__ dx,
-    double* __restrict__ dw_part, int rows, int cols, int chunk, int members,
-    int rows_per_group, int mode, SplitArgs sa) {
-  rmsnorm_bwd_slice_kernel_body<THREADS, VPT>(x, w, dy, rstd, rowdot, dx, dw_part, rows, cols, chunk, members, rows_per_group, mode, sa);
-  split_leave(sa);
 }
 
 // STAGED backward: rows of at most 8192 columns, each held by a team of
@@ -961,8 +917,7 @@ int launch_dw_reduce(const double* part, float* dw, int64_t blocks, int cols, hi
 using FwdSliceFn = void (*)(const uint16_t*, const uint16_t*, uint16_t*, float*, int, int,
                             int, int, float, SplitArgs);
 using BwdSliceFn = void (*)(const uint16_t*, const uint16_t*, const uint16_t*, const float*,
-                            const float*, uint16_t*, double*, int, int, int, int, int, int,
-                            SplitArgs);
+                            const float*, uint16_t*, double*, int, int, int, int, int);
 
 struct FwdPick {
   FwdSliceFn fn;
@@ -1528,18 +1483,16 @@ extern "C" int credit_rmsnorm_bwd_bf16(const uint16_t* x, const uint16_t* w,
   float* rowdot = reinterpret_cast<float*>(
       ws.extra + align_up(static_cast<size_t>(plan.groups) * cols * sizeof(double), 256));
   const int c = static_cast<int>(cols);
-  int mode = kBwdWhole;
-  if (plan.variant == CREDIT_VARIANT_SPLIT) mode = kBwdExchange;
+  const bool exchange = plan.variant == CREDIT_VARIANT_SPLIT;
   // Ticketed launches cover whole dispenser subsets (padding groups exit).
-  const int64_t grid_groups = mode == kBwdExchange ? padded_groups(plan.groups) : plan.groups;
+  const int64_t grid_groups = exchange ? padded_groups(plan.groups) : plan.groups;
   const uint32_t total = static_cast<uint32_t>(grid_groups * plan.members);
   if (plan.variant == CREDIT_VARIANT_READ) {
-    mode = kBwdGiven;
     rmsnorm_bwd_rowdot_kernel<256>
         <<<dim3(static_cast<unsigned>(rows)), dim3(256), 0, stream>>>(x, w, dy, rowdot, c);
     CREDIT_TRY(check_launch("rmsnorm_bwd_rowdot_kernel"));
   }
-  if (mode == kBwdExchange) {
+  if (exchange) {
     const BwdGroupPick* pick = pick_for(kBwdGroup, plan.chunk);
     int64_t fit = 0;
     int dispensers = 0;
@@ -1577,8 +1530,7 @@ extern "C" int credit_rmsnorm_bwd_bf16(const uint16_t* x, const uint16_t* w,
     const BwdPick* pick = pick_for(kBwd, plan.chunk);
     hipLaunchKernelGGL(pick->fn, dim3(total), dim3(pick->threads), pick->lds_bytes(), stream, x,
                        w, dy, rstd, rowdot, dx, dw_part, static_cast<int>(rows), c,
-                       static_cast<int>(plan.chunk), plan.members, plan.rows_per_group, mode,
-                       SplitArgs{});
+                       static_cast<int>(plan.chunk), plan.members, plan.rows_per_group);
     CREDIT_TRY(check_launch("rmsnorm_bwd_slice_kernel"));
   }
   return launch_dw_reduce(dw_part, dw, plan.groups, c, stream);

@@ -288,12 +288,16 @@ struct RowStats {
   float mean, rstd;
   double rs;
 };
-// From partials 0 and 1; x0 is kept in the last (dx may be x: not from x).
+// From partials 0 and 1; x0 is kept in the last (dx may be x: not from x).  The
+// variance of a row with an infinity or NaN is NaN: 0 in the forward, as in
+// layernorm.hip, and NaN in the backward, whose dx is NaN then.
+template <bool FORWARD>
 __device__ __forceinline__ RowStats row_stats(const Place& p, int cols, float eps) {
   RowStats st;
   st.off = wave_reduce_sum_f64(partial(p, 0, 0.0)) / cols;
   const double var = wave_reduce_sum_f64(partial(p, 1, 0.0)) / cols - st.off * st.off;
-  st.rs = 1.0 / __builtin_sqrt((var < 0.0 ? 0.0 : var) + eps);  // NaN stays NaN
+  const bool zero = FORWARD ? !(var > 0.0) : var < 0.0;
+  st.rs = 1.0 / __builtin_sqrt((zero ? 0.0 : var) + eps);
   st.mean = static_cast<float>(p.row_partials[(kValues - 1) * p.parts] + st.off);
   st.rstd = static_cast<float>(st.rs);
   return st;
@@ -309,7 +313,8 @@ __global__ __launch_bounds__(kThreads) void layernorm_fwd_chunks_kernel(
   const size_t at = static_cast<size_t>(p.row) * cols;
   float v[16];
   L::load(v, x, at + p.c0, p, p.part + 1 < parts);
-  const float x0 = L::first(x + at);
+  float x0 = L::first(x + at);
+  if (__builtin_isinf(x0)) x0 = 0.0f;  // the row's mean is infinite, not NaN
   double s1, s2;
   deviations<L>(v, x0, p, &s1, &s2);
   rows::block_sum2<kNW>(s1, s2, slots);
@@ -334,7 +339,7 @@ __global__ __launch_bounds__(kThreads) void layernorm_fwd_outputs_kernel(
   L::load(v, x, at, p, more);
   L::load(g, gamma, p.c0, p, more);
   L::load(b, beta, p.c0, p, more);
-  const RowStats st = row_stats(p, cols, eps);
+  const RowStats st = row_stats<true>(p, cols, eps);
 #pragma unroll
   for (int j = 0; j < 16; ++j) v[j] = (v[j] - st.mean) * st.rstd * g[j] + b[j];
   L::store(v, y, at, p);
@@ -392,7 +397,7 @@ __global__ __launch_bounds__(kThreads) void layernorm_bwd_outputs_kernel(
   L::load(v, x, at, p, more);
   L::load(d, dy, at, p, more);
   L::load(g, gamma, p.c0, p, more);
-  const RowStats st = row_stats(p, cols, eps);
+  const RowStats st = row_stats<false>(p, cols, eps);
   const double b1 = wave_reduce_sum_f64(partial(p, 2, 0.0));
   const double b2 = wave_reduce_sum_f64(partial(p, 3, 0.0));
   const float mg = static_cast<float>(b1 / cols);

@@ -168,3 +168,21 @@ def test_wide_layernorm_bf16(gpu, rows, cols, shift):
                                     gamma.float().numpy())
     np.testing.assert_allclose(dx[i].float().cpu().numpy(), expect, **BF16)
     assert not bool(torch.isnan(y).any()) and not bool(torch.isnan(dx).any())
+
+
+@pytest.mark.parametrize("cols", [40003, 65536])
+def test_wide_layernorm_edge_rows(gpu, cols):
+    """Rows that start with, hold or are infinities, and with a NaN: outputs,
+    mean and rstd as the READ variant gives them."""
+    x = torch.randn(5, cols, generator=torch.Generator().manual_seed(2))
+    x[0, 0] = float("inf")
+    x[1, cols - 1] = -float("inf")
+    x[2] = float("inf")
+    x[3, 0] = float("nan")
+    gamma, beta = torch.ones(cols, device=gpu).bfloat16(), torch.zeros(cols, device=gpu).bfloat16()
+    ins = (x.bfloat16().to(gpu), gamma, beta)
+    got, want = (hip_lib.allocate_outputs("layernorm_fwd", ins) for _ in range(2))
+    hip_lib.layernorm_fwd(*ins, *got, hip_lib.LAYERNORM_EPS, hip_lib.make_cfg())
+    hip_lib.layernorm_fwd(*ins, *want, hip_lib.LAYERNORM_EPS, hip_lib.make_cfg(variant="read"))
+    for g, w, tol in zip(got, want, (BF16, FP32, FP32)):
+        np.testing.assert_allclose(g.float().cpu().numpy(), w.float().cpu().numpy(), **tol)

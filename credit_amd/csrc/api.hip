@@ -240,6 +240,23 @@ NoAllocScope::NoAllocScope() : prev_(g_in_noalloc) { g_in_noalloc = true; }
 NoAllocScope::~NoAllocScope() { g_in_noalloc = prev_; }
 bool in_noalloc_call() { return g_in_noalloc; }
 
+int prepare_split(const credit_cfg* cfg) {
+  int device = 0;
+  CREDIT_HIP(hipGetDevice(&device));
+  HostFlag flag;
+  CREDIT_TRY(host_watchdog_flag(device, &flag, false));
+  if (flag.host != nullptr && workspace_cache().capacity(device, cfg_stream(cfg)) >= kScratchOffset)
+    return CREDIT_OK;
+  // Relaxed: another thread's stream may be under capture meanwhile.
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  int status = host_watchdog_flag(device, &flag, true);
+  char* base = nullptr;
+  if (status == CREDIT_OK) status = acquire_workspace(cfg, 0, &base);
+  CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  return status;
+}
+
 int acquire_split_workspace(const credit_cfg* cfg, int64_t groups, int members,
                             int k_values, int ring, size_t extra_bytes, SplitWorkspace* out) {
   int device = 0;

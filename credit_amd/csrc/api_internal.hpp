@@ -163,6 +163,9 @@ inline size_t split_workspace_bytes(int64_t groups, int members, int k_values, i
 }
 int acquire_split_workspace(const credit_cfg* cfg, int64_t groups, int members,
                             int k_values, int ring, size_t extra_bytes, SplitWorkspace* out);
+// Creates what a split launch on the stream allocates the first time, for a
+// call that takes another path now and SPLIT once the stream is captured.
+int prepare_split(const credit_cfg* cfg);
 
 // Marks the calls this thread makes inside an allocation-free entry point
 // (credit_*_noalloc): the split workspace then uses the device's host-mapped

@@ -498,6 +498,11 @@ bool wide_plan(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_
   }
   hipStream_t stream = cfg_stream(cfg);
   if (!keeps_scratch(stream)) return false;
+  // Whole vectors run SPLIT under capture, where nothing can be allocated.
+  if (vec && prepare_split(cfg) != CREDIT_OK) {
+    (void)hipGetLastError();
+    return false;
+  }
   *lock = std::unique_lock<std::mutex>(pair_mutex());
   char* base = nullptr;
   if (!cache->room(dev, stream, kMaxStreams) ||

@@ -136,6 +136,36 @@ def test_wide_softmax_captured(gpu):
     np.testing.assert_allclose(eager[1][0].cpu().numpy(), e[0], **FP32)
 
 
+@pytest.mark.parametrize("name,rows,cols", [
+    ("softmax_fwd", 16, 131072), ("softmax_bwd", 16, 131072),
+    ("softmax_logits_backward", 8, 262144), ("layernorm_backward", 8, 131072),
+    ("layernorm_fwd", 16, 131072), ("layernorm_backward_bf16", 16, 131072),
+    ("rowwise_quant", 16, 131072)])
+def test_wide_aligned_captured_after_a_warm_up(gpu, name, rows, cols):
+    """One eager call on a new stream readies it for the captured one, which
+    runs SPLIT: its workspace is there."""
+    print(f"captured {name} {rows} x {cols}", flush=True)
+    ins = tuple(t.to(gpu) for t in WORKLOADS[name].make_inputs(rows, cols, seed=5))
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    eager, captured = (hip_lib.allocate_outputs(name, ins) for _ in range(2))
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        hip_lib.bind(name, ins, eager)()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        hip_lib.bind(name, ins, captured)()
+    for _ in range(3):
+        for t in captured:
+            t.zero_()
+        graph.replay()
+        with torch.cuda.stream(stream):
+            hip_lib.bind(name, ins, eager)()
+        torch.cuda.synchronize()
+        for a, b in zip(captured, eager):
+            tol = BF16 if a.dtype == torch.bfloat16 else FP32
+            np.testing.assert_allclose(a.float().cpu().numpy(), b.float().cpu().numpy(), **tol)
+
+
 # bf16: odd widths (chunks of odd rows start inside a dword), even ones, whole
 # vectors, a last chunk of few elements.
 HALF_SHAPES = [(1, 16385, 0), (4, 20001, 2), (129, 33001, 0), (3, 262143, 0), (2, 262142, 2),

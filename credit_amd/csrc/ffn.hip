@@ -25,10 +25,10 @@
 //  3. GEMM2 with epilogue kEpiResidual: out = bf16(acc + x).
 // Each GEMM runs on ffn_gemm256_kernel (256 x 256 x 64 tiles, four waves,
 // LDS-direct operand loads; the C5 path) or on ffn_gemm_tile_kernel (128 or 256
-// x 128 x 64 tiles, K split over workgroups where the tiles leave CUs idle),
-// whichever gemm_plan's count says is done sooner.  The backward
-// (credit_ffn_rmsnorm_gelu_bwd_bf16) runs five GEMMs on the same two kernels
-// with its own epilogues.
+// x 128 x 64 tiles, K split over workgroups where the tiles leave CUs idle), or
+// ffn_gemm_held_kernel (128-tiles, several to a CU), whichever gemm_plan's count
+// says is done sooner.  The backward (credit_ffn_rmsnorm_gelu_bwd_bf16) runs
+// five GEMMs on the same kernels with its own epilogues.
 #include <algorithm>
 #include <atomic>
 #include <initializer_list>
@@ -638,14 +638,55 @@ __global__ __launch_bounds__(kBigThreads) void ffn_gemm256_kernel(
   clock_probe_add(probe, false);
 }
 
+// The epilogue of registers q .. q + 3 of a 32 x 32 tile: rows mb .. mb + 3 of
+// column n.
+template <int EPI>
+__device__ __forceinline__ void store_quad(const f32x16& acc, int q, const float (&sc)[4],
+                                           const uint16_t* R, uint16_t* C, uint16_t* C2, float* Cf,
+                                           int mb, int n, int M, int N) {
+  const size_t idx = static_cast<size_t>(mb) * N + n;
+  EpiValue v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float rv = kEpiReadsR<EPI> ? bf16_to_f32(R[idx + static_cast<size_t>(e) * N]) : 0.0f;
+    v[e] = epilogue_value<EPI>(acc[q + e], sc[e], rv);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; e += 2) {
+    const size_t at = idx + static_cast<size_t>(e) * N;
+    if constexpr (EPI == kEpiStoreF32) {
+      Cf[at] = v[e].c;
+      Cf[at + N] = v[e + 1].c;
+    } else if constexpr (EPI != kEpiStoreT) {
+      const uint32_t p = pack_bf16x2(v[e].c, v[e + 1].c);
+      C[at] = static_cast<uint16_t>(p);
+      C[at + N] = static_cast<uint16_t>(p >> 16);
+    }
+    if constexpr (EPI == kEpiGeluSave) {
+      const uint32_t p = pack_bf16x2(v[e].c2, v[e + 1].c2);
+      C2[at] = static_cast<uint16_t>(p);
+      C2[at + N] = static_cast<uint16_t>(p >> 16);
+    }
+  }
+  const size_t tdx = static_cast<size_t>(n) * M + mb;
+  if constexpr (EPI == kEpiStoreT) {
+    *reinterpret_cast<uint2*>(C + tdx) =
+        uint2{pack_bf16x2(v[0].c, v[1].c), pack_bf16x2(v[2].c, v[3].c)};
+  } else if constexpr (EPI == kEpiUH || EPI == kEpiGeluBwd) {
+    if (EPI == kEpiUH || C2 != nullptr)
+      *reinterpret_cast<uint2*>(C2 + tdx) =
+          uint2{pack_bf16x2(v[0].c2, v[1].c2), pack_bf16x2(v[2].c2, v[3].c2)};
+  }
+}
+
 // ------------------------------------------------- BM x 128 tiles, split K --
 // The GEMM of every shape the 256-tile kernel does not fill the chip with:
 // BM x 128 x 64 tiles (BM 128 or 256) of four waves in a 2 x 2 grid, wave
 // (wm, wn) owning a BM/2 x 64 block as BM/64 x 2 v_mfma_f32_32x32x16_bf16
 // tiles, and K cut into `slices` pieces whose fp32 sums are added in slice
 // order.
-//  - One operand ring for A and B: ST stages of (BM + 128) rows x 64 K, filled by the LDS-direct loads of the 256-tile kernel (the same row
-//    swizzle; KN: the stage's B part is 64 K-rows of 256 bytes, chunk c of
+//  - One operand ring for A and B: ST stages of (BM + 128) rows x 64 K, filled
+//    by the LDS-direct loads of the 256-tile kernel (the same row swizzle; KN: the stage's B part is 64 K-rows of 256 bytes, chunk c of
 //    K-row r at position c ^ 4 (r & 3)).
 //  - K-step k reads stage k % ST.  Iteration it runs four sub-steps of k = 16,
 //    each reading the next one's fragments while its MFMAs issue.  Before the
@@ -882,50 +923,114 @@ __global__ __launch_bounds__(256) void ffn_gemm_tile_kernel(
       const int mb = m0 + wm * (BM / 2) + i * 32 + 8 * q + 4 * (lane >> 5);
       float sc[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sc[e] = kEpiScaled<EPI> && !RA && scale != nullptr ? scale[mb + e] : 1.0f;
+      for (int e = 0; e < 4; ++e)
+        sc[e] = kEpiScaled<EPI> && !RA && scale != nullptr ? scale[mb + e] : 1.0f;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int n = n0 + wn * 64 + j * 32 + (lane & 31);
-        const size_t idx = static_cast<size_t>(mb) * N + n;
-        EpiValue v[4];
+        if constexpr (EPI == kEpiPartial) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if constexpr (EPI == kEpiPartial) {
-            part[idx + static_cast<size_t>(e) * N] = acc[i][j][4 * q + e];
-          } else {
-            const float rv =
-                kEpiReadsR<EPI> ? bf16_to_f32(R[idx + static_cast<size_t>(e) * N]) : 0.0f;
-            v[e] = epilogue_value<EPI>(total[i][j][4 * q + e], sc[e], rv);
-          }
-        }
-        if constexpr (EPI == kEpiPartial) continue;
-#pragma unroll
-        for (int e = 0; e < 4; e += 2) {
-          const size_t at = idx + static_cast<size_t>(e) * N;
-          if constexpr (EPI == kEpiStoreF32) {
-            Cf[at] = v[e].c;
-            Cf[at + N] = v[e + 1].c;
-          } else if constexpr (EPI != kEpiStoreT) {
-            const uint32_t p = pack_bf16x2(v[e].c, v[e + 1].c);
-            C[at] = static_cast<uint16_t>(p);
-            C[at + N] = static_cast<uint16_t>(p >> 16);
-          }
-          if constexpr (EPI == kEpiGeluSave) {
-            const uint32_t p = pack_bf16x2(v[e].c2, v[e + 1].c2);
-            C2[at] = static_cast<uint16_t>(p);
-            C2[at + N] = static_cast<uint16_t>(p >> 16);
-          }
-        }
-        const size_t tdx = static_cast<size_t>(n) * M + mb;
-        if constexpr (EPI == kEpiStoreT) {
-          *reinterpret_cast<uint2*>(C + tdx) =
-              uint2{pack_bf16x2(v[0].c, v[1].c), pack_bf16x2(v[2].c, v[3].c)};
-        } else if constexpr (EPI == kEpiUH || EPI == kEpiGeluBwd) {
-          if (EPI == kEpiUH || C2 != nullptr)
-            *reinterpret_cast<uint2*>(C2 + tdx) =
-                uint2{pack_bf16x2(v[0].c2, v[1].c2), pack_bf16x2(v[2].c2, v[3].c2)};
+          for (int e = 0; e < 4; ++e)
+            part[static_cast<size_t>(mb + e) * N + n] = acc[i][j][4 * q + e];
+        } else {
+          store_quad<EPI>(total[i][j], 4 * q, sc, R, C, C2, Cf, mb, n, M, N);
         }
       }
+    }
+}
+
+// ------------------------------------------- 128 x 128 tiles, many to a CU --
+// More 128-tiles than CUs, unsplit, B [N, K]: one LDS buffer of 36 KiB and the
+// next K-step in registers, so that three workgroups share a CU and cover each
+// other's barriers and epilogues, where the ring of ffn_gemm_tile_kernel lets
+// two: 600 tiles of 28 K-steps 55 us against 67 there, 624 of 24 46 against
+// 60, 275 of 66 67 against 84, 621 of 18 35 against 48, 1125 of 50 158 against
+// 166, 847 of 46 118 against 120 (688 TFLOP/s).  Bound by the LDS reads of 64 x 64 a wave
+// and the two barriers of a step.  The same MFMAs in the same order as the
+// other kernels' unsplit products: the same bits.
+constexpr int kHeldStride = kBigK + 8;  // bf16 per LDS row: 16 bytes of padding spread the banks
+
+template <int EPI>
+__global__ __launch_bounds__(256) void ffn_gemm_held_kernel(
+    const uint16_t* __restrict__ A, const float* __restrict__ scale,
+    const uint16_t* __restrict__ B, const uint16_t* __restrict__ R, uint16_t* __restrict__ C,
+    uint16_t* __restrict__ C2, float* __restrict__ Cf, int M, int N, int K) {
+  __shared__ __attribute__((aligned(16))) uint16_t As[kTileN * kHeldStride];
+  __shared__ __attribute__((aligned(16))) uint16_t Bs[kTileN * kHeldStride];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wm = tid >> 7, wn = (tid >> 6) & 1;
+  // Consecutive workgroups walk down M: the weight rows stay in the L2.
+  const int tiles_m = M / kTileN;
+  const int m0 = static_cast<int>(blockIdx.x) % tiles_m * kTileN;
+  const int n0 = static_cast<int>(blockIdx.x) / tiles_m * kTileN;
+
+  // Lane t moves 16-byte chunk t % 8 of rows t / 8 + 32 i, of A and of B.
+  const int row = tid >> 3, chunk = tid & 7;
+  const u32x4* a_src[4];
+  const u32x4* b_src[4];
+  u32x4 ra[4], rb[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const size_t r = row + 32 * i;
+    a_src[i] = reinterpret_cast<const u32x4*>(A + (m0 + r) * K) + chunk;
+    b_src[i] = reinterpret_cast<const u32x4*>(B + (n0 + r) * K) + chunk;
+    ra[i] = *a_src[i];
+    rb[i] = *b_src[i];
+  }
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[t >> 1][t & 1][r] = 0.0f;
+
+  const int steps = K / kBigK;
+  for (int k = 0; k < steps; ++k) {
+    __syncthreads();  // the last step's fragments are read
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = (row + 32 * i) * kHeldStride + chunk * 8;
+      *reinterpret_cast<u32x4*>(As + at) = ra[i];
+      *reinterpret_cast<u32x4*>(Bs + at) = rb[i];
+    }
+    __syncthreads();
+    if (k + 1 < steps) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ra[i] = a_src[i][(k + 1) * (kBigK / 8)];
+        rb[i] = b_src[i][(k + 1) * (kBigK / 8)];
+      }
+    }
+#pragma unroll
+    for (int kk = 0; kk < kBigK; kk += 16) {
+      const int at = (lane & 31) * kHeldStride + kk + (lane >> 5) * 8;
+      bf16x8_t af[2], bf[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        af[i] = *reinterpret_cast<const bf16x8_t*>(As + at + (wm * 64 + i * 32) * kHeldStride);
+        bf[i] = *reinterpret_cast<const bf16x8_t*>(Bs + at + (wn * 64 + i * 32) * kHeldStride);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
+    }
+  }
+
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int mb = m0 + wm * 64 + i * 32 + 8 * q + 4 * (lane >> 5);
+      float sc[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        sc[e] = kEpiScaled<EPI> && scale != nullptr ? scale[mb + e] : 1.0f;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        store_quad<EPI>(acc[i][j], 4 * q, sc, R, C, C2, Cf, mb, n0 + wn * 64 + j * 32 + (lane & 31),
+                        M, N);
     }
 }
 
@@ -1098,8 +1203,8 @@ int allow_lds(Kernel kernel, int bytes) {
                          : hip_failure(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
 }
 
-// How a product C[M, N] over K runs, from its sizes alone and the same for
-// (M, N) and (N, M), so that every entry point that forms a product (either
+// How a product C[M, N] over K runs.  The slices follow from the sizes alone and
+// are the same for (M, N) and (N, M), so that every entry point that forms a product (either
 // weight layout, recomputed or saved) adds its terms in the same order.
 //  - slices: K pieces.  Time of the units on 256 CUs (flat_us), plus, when
 //    split, kReduceUs and the fp32 sums written and read at kReduceGBs.  1024 x
@@ -1109,6 +1214,8 @@ int allow_lds(Kernel kernel, int bytes) {
 //    less than two flat ones (fewer LDS bytes per MFMA), but 256 x 6144 x
 //    18944 gains (245 -> 196 us) where 512 x 28672 x 8192 would leave half the
 //    CUs idle (490 -> 540 us).
+//  - held: more tiles than CUs, unsplit, of a [N, K] B; not with one M-tile,
+//    whose tile columns start skewed.
 //  - big: likewise (the FFN of 1024 rows x 8192 x 28672: 783 us with it
 //    against 846 on tall tiles; 512 rows, 224 tiles: 487 against 512).
 struct GemmPlan {
@@ -1116,6 +1223,7 @@ struct GemmPlan {
   int bm;      // else rows per tile of ffn_gemm_tile_kernel
   int slices;
   int skew;    // its tile columns start their slices a step apart
+  bool held;   // ffn_gemm_held_kernel
 };
 constexpr int kGemmCus = 256;
 constexpr int kMaxSlices = 16;
@@ -1132,6 +1240,12 @@ double tall_us(int64_t units, int64_t steps) {
 }
 double big_us(int64_t units, int64_t steps) {
   return (units + kGemmCus - 1) / kGemmCus * (steps * 1.55 + 10.0);
+}
+// More units than CUs on ffn_gemm_held_kernel: 0.6 us a step for each of a
+// CU's tiles and the 6 us once (600 tiles of 28 steps 56, measured 55; 736 of 16
+// 35, 33; 1125 of 50 156, 158).
+double held_us(int64_t units, int64_t steps) {
+  return (units + kGemmCus - 1) / kGemmCus * (steps * 0.6) + 6.0;
 }
 constexpr int64_t kSlabBytes = int64_t{64} << 20;  // most fp32 partial sums of one product
 
@@ -1164,15 +1278,18 @@ bool big_shape(int64_t M, int64_t N, int64_t K) {
          ((M / kBig) * (N / kBig)) % 8 == 0 && K <= (1 << 22) && N <= (1 << 22);
 }
 
-GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K) {
-  GemmPlan p{false, 128, gemm_slices(M, N, K), 0};
+GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, bool kn) {
+  GemmPlan p{false, 128, gemm_slices(M, N, K), 0, false};
   const int64_t steps = K / kBigK / p.slices, tiles = (M / 128) * (N / 128) * p.slices;
-  double us = flat_us(tiles, steps);
+  p.held = !kn && p.slices == 1 && tiles > kGemmCus && M > 128;
+  double us = p.held ? held_us(tiles, steps) : flat_us(tiles, steps);
   if (M % 256 == 0 && K <= (1 << 22) && tall_us(tiles / 2, steps) < us) {
     p.bm = 256;
+    p.held = false;
     us = tall_us(tiles / 2, steps);
   }
   p.big = p.slices == 1 && big_shape(M, N, K) && big_us(tiles / 4, steps) < us;
+  p.held = p.held && !p.big;
   p.skew = M == p.bm;
   return p;
 }
@@ -1240,7 +1357,7 @@ template <int EPI, bool KN = false>
 int launch_gemm(const uint16_t* A, const float* scale, const uint16_t* B, const uint16_t* R,
                 uint16_t* C, uint16_t* C2, float* Cf, int M, int N, int K, const Scratch& scratch,
                 hipStream_t stream, const char* name, bool ra = false) {
-  GemmPlan plan = gemm_plan(M, N, K);
+  GemmPlan plan = gemm_plan(M, N, K, KN);
   // The weight gradients are formed either way round (M and N swapped).
   if (EPI == kEpiStore || EPI == kEpiStoreT) plan.skew = 0;
   if constexpr (kEpiScaled<EPI>) {
@@ -1255,6 +1372,13 @@ int launch_gemm(const uint16_t* A, const float* scale, const uint16_t* B, const 
                                   dim3(kBigThreads), kBigLds, stream>>>(
         A, scale, B, R, C, C2, Cf, M, N, K, g_clock_probe.load(std::memory_order_relaxed));
     return check_launch(name);
+  }
+  if constexpr (!KN) {
+    if (plan.held) {
+      ffn_gemm_held_kernel<EPI><<<dim3(static_cast<unsigned>((M / kTileN) * (N / kTileN))),
+                                  dim3(256), 0, stream>>>(A, scale, B, R, C, C2, Cf, M, N, K);
+      return check_launch(name);
+    }
   }
   if (plan.slices > 1 &&
       scratch.bytes >= static_cast<size_t>(plan.slices) * M * N * sizeof(float)) {

@@ -84,3 +84,34 @@ def test_train_forward_captured_first(gpu, rows, d, f):
         torch.cuda.synchronize()
         for a, b in zip(captured, eager):
             assert torch.equal(a, b), i
+
+
+# More 128-tiles than CUs in GEMM1 (258 tiles of two K-steps; 270 of five), in
+# GEMM2 (272 of 18) and in the weight gradients.
+@pytest.mark.parametrize("rows,d,f", [(384, 128, 11008), (640, 640, 6912), (2176, 2048, 1152)])
+def test_more_tiles_than_cus(gpu, rows, d, f):
+    """Several workgroups to a CU in the nn.Linear layout, the ring kernel in the
+    [in, out] one: the same additions in the same order."""
+    print(f"ffn held rows={rows} d={d} f={f}", flush=True)
+    x, w1, w2 = make(rows, d, f, "linear", gpu)
+    k1, k2 = w1.t().contiguous(), w2.t().contiguous()
+    out = run(x, w1, w2, "linear")
+    assert torch.equal(run(x, k1, k2, "in_out"), out)
+    expect = ref.ffn_rmsnorm_gelu(x.float().cpu().numpy(), k1.float().cpu().numpy(),
+                                  k2.float().cpu().numpy(), EPS)
+    np.testing.assert_allclose(out.float().cpu().numpy(), expect, rtol=1e-2, atol=1e-2)
+    dout = torch.randn(rows, d, generator=torch.Generator().manual_seed(f)).to(gpu, torch.bfloat16)
+    grads = []
+    for a, b, kn in ((w1, w2, False), (k1, k2, True)):
+        y, rstd = torch.empty_like(x), torch.empty(rows, device=gpu)
+        u = torch.empty(rows, f, device=gpu, dtype=torch.bfloat16)
+        h, g = torch.empty_like(u), (torch.empty_like(x), torch.empty_like(a), torch.empty_like(b))
+        hip_lib.ffn_train_forward(x, a, b, y, rstd, u, h, EPS, hip_lib.make_cfg(), kn)
+        hip_lib.ffn_backward_saved(x, a, b, dout, rstd, u, h, *g, hip_lib.make_cfg(), kn)
+        torch.cuda.synchronize()
+        assert torch.equal(y, out)
+        grads.append((g[0], g[1].t() if kn else g[1], g[2].t() if kn else g[2]))
+    # Unit-variance dout: as far apart as two bf16 roundings of one sum.
+    for a, b in zip(*grads):
+        scale = a.float().abs().max().item()
+        assert (a.float() - b.float()).abs().max().item() <= 2.0 ** -7 * scale

@@ -452,7 +452,9 @@ struct WidePlan {
 // (LayerNorm backward 384 x 40003: 76 us, 49 here).  Rows of whole 16-byte
 // vectors have faster kernels, SPLIT among them: at most 32 rows, wide ones and
 // little data (softmax forward 16 x 16384: 6.0 us, 6.9 here; 16 x 65536: 16,
-// 7.4; logits backward 64 x 32768: 9.4, 10.1; 64 x 131072: 22, 27).  16 x
+// 7.4; logits backward 64 x 32768: 9.4, 10.1; 64 x 131072: 22, 27).
+// Quantisation holds rows of up to 65536 columns in one workgroup (16 x 65536:
+// 6.7, 7.0); wider ones ran in SPLIT groups (16 x 70952: 8.0, 7.0).  16 x
 // 262144 would gain too (forward 13.4, 9.9 here) but AUTO is known to run SPLIT
 // there (credit_last_split_shape).  A caller's workspace is SPLIT's.  bf16 rows
 // are half the bytes: LayerNorm forward 16 x 16386 7.1 us, 7.6 here, 64 x 16387
@@ -465,7 +467,7 @@ constexpr WideRule kSoftmaxBwdRule{16384, 53248, 24576};
 constexpr WideRule kLnBwdRule{16384, 32768, 24576};
 constexpr WideRule kLnBwdHalfRule{16384, 32768, 49152};
 constexpr WideRule kLnFwdRule{20480, 32768, 49152};
-constexpr WideRule kQuantRule{32768, 65536, 98304};
+constexpr WideRule kQuantRule{32768, 65536, 65536};
 constexpr int64_t kFewWide = 128;
 bool wide_wanted(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_t cols,
                  bool vec) {

@@ -19,7 +19,8 @@ pytestmark = pytest.mark.gpu
 # rows, cols, elements past a 16-byte address
 SHAPES = [(1, 16385, 0), (3, 20001, 1), (128, 16391, 0), (129, 33001, 0), (1, 262143, 0),
           (2, 262144, 3), (2, 262145, 0), (5, 98309, 2), (300, 66001, 0), (32, 24580, 0),
-          (16, 131072, 0), (17, 262144, 0), (1, 262144, 0), (33, 32768, 0)]
+          (16, 131072, 0), (17, 262144, 0), (1, 262144, 0), (33, 32768, 0),
+          (7, 65540, 0)]
 
 
 @pytest.mark.parametrize("rows,cols,shift", SHAPES)

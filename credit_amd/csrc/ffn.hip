@@ -686,8 +686,9 @@ __device__ __forceinline__ void store_quad(const f32x16& acc, int q, const float
 // tiles, and K cut into `slices` pieces whose fp32 sums are added in slice
 // order.
 //  - One operand ring for A and B: ST stages of (BM + 128) rows x 64 K, filled
-//    by the LDS-direct loads of the 256-tile kernel (the same row swizzle; KN: the stage's B part is 64 K-rows of 256 bytes, chunk c of
-//    K-row r at position c ^ 4 (r & 3)).
+//    by the LDS-direct loads of the 256-tile kernel (the same row swizzle; KN:
+//    the stage's B part is 64 K-rows of 256 bytes, chunk c of K-row r at
+//    position c ^ 4 (r & 3)).
 //  - K-step k reads stage k % ST.  Iteration it runs four sub-steps of k = 16,
 //    each reading the next one's fragments while its MFMAs issue.  Before the
 //    last sub-step: own loads of step it+1 landed (vmcnt leaves the ST - 2

@@ -38,6 +38,7 @@
 
 #include "api_internal.hpp"
 #include "common.hpp"
+#include "ffn_plan.hpp"
 #include "workspace_cache.hpp"
 
 namespace credit {
@@ -45,6 +46,8 @@ namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+using namespace ffn;
 
 constexpr int kFfnMultiple = 128;  // rows, d and f
 
@@ -225,8 +228,6 @@ __global__ __launch_bounds__(256) void ffn_rstd_kernel(const uint16_t* __restric
 //   kEpiGelu:     C = bf16(GELU(acc * scale[m]))   (RMSNorm folded in: the
 //                 row scale commutes with the GEMM)
 //   kEpiResidual: C = bf16(acc + R[m, n])
-constexpr int kBig = 256;
-constexpr int kBigK = 64;
 constexpr int kBigTile = kBig * kBigK * 2;   // one operand tile of a stage, bytes (32 KiB)
 constexpr int kBigBRing = 3;                 // B stages (A has two)
 constexpr int kBigBBase = 2 * kBigTile;      // B ring after the two A stages
@@ -716,7 +717,6 @@ __device__ __forceinline__ void store_quad(const f32x16& acc, int q, const float
 //    fragments are used.  Twice as slow as reading an A that
 //    ffn_rstd_kernel scaled (176 against 87 us for 128 x 28672 x 8192), so it
 //    serves calls with no room for that copy.
-constexpr int kTileN = 128;
 template <int BM>
 constexpr int kTileStageBytes = (BM + kTileN) * kBigK * 2;
 
@@ -1202,110 +1202,6 @@ int allow_lds(Kernel kernel, int bytes) {
                                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   return e == hipSuccess ? CREDIT_OK
                          : hip_failure(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
-}
-
-// How a product C[M, N] over K runs.  The slices follow from the sizes alone and
-// are the same for (M, N) and (N, M), so that every entry point that forms a product (either
-// weight layout, recomputed or saved) adds its terms in the same order.
-//  - slices: K pieces.  Time of the units on 256 CUs (flat_us), plus, when
-//    split, kReduceUs and the fp32 sums written and read at kReduceGBs.  1024 x
-//    2048 x 8192 (128 tiles): 131 us on 32 256-tiles, 47 + 5 us in 2 slices;
-//    128 x 8192 x 28672 (64 tiles): 472 us, 103 + 5 us in 4.
-//  - bm: 256 where its rounds take less by the same count; a tall step costs
-//    less than two flat ones (fewer LDS bytes per MFMA), but 256 x 6144 x
-//    18944 gains (245 -> 196 us) where 512 x 28672 x 8192 would leave half the
-//    CUs idle (490 -> 540 us).
-//  - held: more tiles than CUs, unsplit, of a [N, K] B; not with one M-tile,
-//    whose tile columns start skewed.
-//  - big: likewise (the FFN of 1024 rows x 8192 x 28672: 783 us with it
-//    against 846 on tall tiles; 512 rows, 224 tiles: 487 against 512).
-struct GemmPlan {
-  bool big;    // the 256-tile kernel
-  int bm;      // else rows per tile of ffn_gemm_tile_kernel
-  int slices;
-  int skew;    // its tile columns start their slices a step apart
-  bool held;   // ffn_gemm_held_kernel
-};
-constexpr int kGemmCus = 256;
-constexpr int kMaxSlices = 16;
-// Time of `units` tiles of `steps` 64-wide K-steps, from 1024-row products:
-// 0.45 us a step and 6 us beside them for a 128-row tile (0.6 us where two
-// share a CU), 0.85 and 8.4 us for a 256-row one, 1.55 and 10 us for the
-// 256-tile kernel's.
-double flat_us(int64_t units, int64_t steps) {
-  const int64_t rounds = (units + kGemmCus - 1) / kGemmCus;
-  return rounds * (steps * (rounds > 1 ? 0.6 : 0.45) + 6.0);
-}
-double tall_us(int64_t units, int64_t steps) {
-  return (units + kGemmCus - 1) / kGemmCus * (steps * 0.85 + 8.4);
-}
-double big_us(int64_t units, int64_t steps) {
-  return (units + kGemmCus - 1) / kGemmCus * (steps * 1.55 + 10.0);
-}
-// More units than CUs on ffn_gemm_held_kernel: 0.6 us a step for each of a
-// CU's tiles and the 6 us once (600 tiles of 28 steps 56, measured 55; 736 of 16
-// 35, 33; 1125 of 50 156, 158).
-double held_us(int64_t units, int64_t steps) {
-  return (units + kGemmCus - 1) / kGemmCus * (steps * 0.6) + 6.0;
-}
-constexpr int64_t kSlabBytes = int64_t{64} << 20;  // most fp32 partial sums of one product
-
-int gemm_slices(int64_t M, int64_t N, int64_t K) {
-  constexpr double kReduceUs = 4.0, kReduceGBs = 4000.0;
-  const int64_t tiles = (M / 128) * (N / 128), steps = K / kBigK;
-  int best = 1;
-  double best_us = 1e30;
-  for (int s = 1; s <= kMaxSlices && steps / s >= 8; ++s) {
-    if (s > 1 && s * M * N * 4 > kSlabBytes) break;
-    double us = flat_us(tiles * s, (steps + s - 1) / s);
-    if (s > 1) us += kReduceUs + s * M * N * 8.0 / (kReduceGBs * 1e3);
-    if (us < best_us * 0.95) {
-      best = s;
-      best_us = us;
-    }
-  }
-  return best;
-}
-
-// Shapes the 256-tile kernel can take: M and N multiples of 256, K of 128, a
-// tile count that is a multiple of the 8 XCDs, and operand tiles (256 * K * 2
-// bytes; a [K, N] B's (K - 1) * N * 2 + 512, which every accepted shape keeps
-// below 2^32) and the epilogue's R tile ((255 * N + 256) * 2 bytes) that fit
-// a buffer resource.  A GEMM that scales its A rows (RMSNorm) multiplies the
-// fp32 sums by rstd on these shapes and rounds x * rstd to bf16 first on every
-// other one, whichever kernel runs.
-bool big_shape(int64_t M, int64_t N, int64_t K) {
-  return M % kBig == 0 && N % kBig == 0 && K % (2 * kBigK) == 0 &&
-         ((M / kBig) * (N / kBig)) % 8 == 0 && K <= (1 << 22) && N <= (1 << 22);
-}
-
-GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, bool kn) {
-  GemmPlan p{false, 128, gemm_slices(M, N, K), 0, false};
-  const int64_t steps = K / kBigK / p.slices, tiles = (M / 128) * (N / 128) * p.slices;
-  p.held = !kn && p.slices == 1 && tiles > kGemmCus && M > 128;
-  double us = p.held ? held_us(tiles, steps) : flat_us(tiles, steps);
-  if (M % 256 == 0 && K <= (1 << 22) && tall_us(tiles / 2, steps) < us) {
-    p.bm = 256;
-    p.held = false;
-    us = tall_us(tiles / 2, steps);
-  }
-  p.big = p.slices == 1 && big_shape(M, N, K) && big_us(tiles / 4, steps) < us;
-  p.held = p.held && !p.big;
-  p.skew = M == p.bm;
-  return p;
-}
-
-// Scratch bytes: the partial sums of a product, and those of the scaled
-// product with its copy of a.
-size_t part_bytes(int64_t M, int64_t N, int64_t K) {
-  const int64_t slices = gemm_slices(M, N, K);
-  return slices > 1 ? static_cast<size_t>(slices * M * N) * sizeof(float) : 0;
-}
-size_t copy_bytes(int64_t M, int64_t F, int64_t D) {
-  return big_shape(M, F, D) ? 0 : align_up(static_cast<size_t>(M) * D * 2, 256);
-}
-size_t norm_bytes(int64_t M, int64_t F, int64_t D) {
-  return copy_bytes(M, F, D) + part_bytes(M, F, D);
 }
 
 // Device memory a call's products may use beside its own buffers: fp32

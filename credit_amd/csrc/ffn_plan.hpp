@@ -13,8 +13,9 @@ constexpr int kBig = 256;    // rows and columns of a tile of ffn_gemm256_kernel
 constexpr int kBigK = 64;    // K of a step, in every kernel
 constexpr int kTileN = 128;  // columns of a tile of the other two
 
-// How a product C[M, N] over K runs.  The slices follow from the sizes alone and
-// are the same for (M, N) and (N, M), so that every entry point that forms a product (either
+// How a product C[M, N] over K runs.  The slices and the skew follow from the
+// sizes alone, whatever B's layout and kernel, and the slices are the same for
+// (M, N) and (N, M), so that every entry point that forms a product (either
 // weight layout, recomputed or saved) adds its terms in the same order.
 //  - slices: K pieces.  Time of the units on 256 CUs (flat_us), plus, when
 //    split, kReduceUs and the fp32 sums written and read at kReduceGBs.  1024 x
@@ -24,9 +25,11 @@ constexpr int kTileN = 128;  // columns of a tile of the other two
 //    less than two flat ones (fewer LDS bytes per MFMA), but 256 x 6144 x
 //    18944 gains (245 -> 196 us) where 512 x 28672 x 8192 would leave half the
 //    CUs idle (490 -> 540 us).
-//  - held: more tiles than CUs, unsplit, of a [N, K] B; not with one M-tile,
-//    whose tile columns start skewed.
-//  - big: likewise (the FFN of 1024 rows x 8192 x 28672: 783 us with it
+//  - skew: one M-tile, but for the sizes that run held in the [N, K] layout,
+//    which has no skew (256 x 768 x 32896: the FFN takes 68 us there, 81 on
+//    skewed tall tiles; [K, N] 78 without the skew, 80 with it).
+//  - held: more tiles than CUs, unsplit, of a [N, K] B.
+//  - big: likewise by time (the FFN of 1024 rows x 8192 x 28672: 783 us with it
 //    against 846 on tall tiles; 512 rows, 224 tiles: 487 against 512).
 struct GemmPlan {
   bool big;    // the 256-tile kernel
@@ -91,16 +94,21 @@ inline bool big_shape(int64_t M, int64_t N, int64_t K) {
 inline GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, bool kn) {
   GemmPlan p{false, 128, gemm_slices(M, N, K), 0, false};
   const int64_t steps = K / kBigK / p.slices, tiles = (M / 128) * (N / 128) * p.slices;
-  p.held = !kn && p.slices == 1 && tiles > kGemmCus && M > 128;
-  double us = p.held ? held_us(tiles, steps) : flat_us(tiles, steps);
+  double us = flat_us(tiles, steps);
   if (M % 256 == 0 && K <= (1 << 22) && tall_us(tiles / 2, steps) < us) {
     p.bm = 256;
-    p.held = false;
     us = tall_us(tiles / 2, steps);
   }
-  p.big = p.slices == 1 && big_shape(M, N, K) && big_us(tiles / 4, steps) < us;
-  p.held = p.held && !p.big;
-  p.skew = M == p.bm;
+  const bool held = p.slices == 1 && tiles > kGemmCus && M > 128 && held_us(tiles, steps) < us;
+  p.skew = M == p.bm && !held;
+  if (held && !kn) {
+    p.held = true;
+    us = held_us(tiles, steps);
+  }
+  if (p.slices == 1 && big_shape(M, N, K) && big_us(tiles / 4, steps) < us) {
+    p.big = true;
+    p.held = false;
+  }
   return p;
 }
 

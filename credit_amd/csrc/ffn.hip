@@ -716,7 +716,7 @@ __device__ __forceinline__ void store_quad(const f32x16& acc, int q, const float
 //  - RA: the A rows are scaled by scale[m] and rounded to bf16 as their
 //    fragments are used.  Twice as slow as reading an A that
 //    ffn_rstd_kernel scaled (176 against 87 us for 128 x 28672 x 8192), so it
-//    serves calls with no room for that copy.
+//    serves calls whose output is in place of x, with no room for that copy.
 template <int BM>
 constexpr int kTileStageBytes = (BM + kTileN) * kBigK * 2;
 
@@ -1204,8 +1204,8 @@ int allow_lds(Kernel kernel, int bytes) {
                          : hip_failure(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
 }
 
-// Device memory a call's products may use beside its own buffers: fp32
-// partial sums, and the scaled copy of x where a product rounds it first.
+// Device memory a call's products may use beside its own buffers, for their
+// fp32 partial sums.
 struct Scratch {
   char* base = nullptr;
   size_t bytes = 0;
@@ -1297,25 +1297,33 @@ int launch_gemm(const uint16_t* A, const float* scale, const uint16_t* B, const 
                                                            plan, stream, name);
 }
 
+// Where a product that rounds a = bf16(x * rstd) first may leave that copy
+// until the call writes `out`, [rows, d] bf16 as well; nullptr: out shares
+// memory with what the product reads.
+uint16_t* copy_room(uint16_t* out, const uint16_t* x, const uint16_t* w1, int64_t rows, int64_t d,
+                    int64_t f) {
+  const auto apart = [&](const uint16_t* p, int64_t n) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(out), b = reinterpret_cast<uintptr_t>(p);
+    return a + static_cast<size_t>(rows * d) * 2 <= b || b + static_cast<size_t>(n) * 2 <= a;
+  };
+  return apart(x, rows * d) && apart(w1, d * f) ? out : nullptr;
+}
+
 // The scaled product u = rstd (x W1^T) with its RMSNorm statistics: rstd, then
 // the GEMM over x with rstd in the epilogue, or on the shapes that round
-// a = bf16(x * rstd) first over the copy of a that the scratch holds.
+// a = bf16(x * rstd) first over a copy of a at `a` (nullptr: none, the A rows
+// are scaled as the product runs).
 template <int EPI, bool KN>
 int launch_norm_gemm(const uint16_t* x, float* rstd, const uint16_t* w1, uint16_t* C, uint16_t* C2,
-                     int M, int F, int D, float eps, const Scratch& scratch, hipStream_t stream,
-                     const char* name) {
-  uint16_t* a = nullptr;
+                     uint16_t* a, int M, int F, int D, float eps, const Scratch& scratch,
+                     hipStream_t stream, const char* name) {
   const bool rounds = !big_shape(M, F, D);
-  const size_t a_bytes = copy_bytes(M, F, D);
-  Scratch rest = scratch;
-  if (rounds && scratch.bytes >= norm_bytes(M, F, D)) {
-    a = reinterpret_cast<uint16_t*>(scratch.base);
-    rest = Scratch{scratch.base + a_bytes, scratch.bytes - a_bytes};
-  }
+  if (!rounds) a = nullptr;
   ffn_rstd_kernel<<<dim3(M), dim3(256), 0, stream>>>(x, rstd, a, D, eps);
   CREDIT_TRY(check_launch("ffn_rstd_kernel"));
   return launch_gemm<EPI, KN>(a != nullptr ? a : x, a != nullptr ? nullptr : rstd, w1, nullptr, C,
-                              C2, nullptr, M, F, D, rest, stream, name, rounds && a == nullptr);
+                              C2, nullptr, M, F, D, scratch, stream, name,
+                              rounds && a == nullptr);
 }
 
 int launch_transpose(const uint16_t* src, uint16_t* dst, int64_t rows, int64_t cols,
@@ -1355,19 +1363,17 @@ BwdLayout bwd_layout(int64_t M, int64_t d, int64_t f) {
 
 // Scratch of the whole calls: the most any one of their products uses.
 size_t fwd_scratch(int64_t M, int64_t d, int64_t f) {
-  return std::max(norm_bytes(M, f, d), part_bytes(M, d, f));
+  return std::max(part_bytes(M, f, d), part_bytes(M, d, f));
 }
 size_t bwd_scratch(int64_t M, int64_t d, int64_t f) {
-  return std::max({norm_bytes(M, f, d), part_bytes(d, f, M), part_bytes(M, d, f)});
+  return std::max({part_bytes(M, f, d), part_bytes(d, f, M), part_bytes(M, d, f)});
 }
 
 // The training forward brings no workspace and shares none: its scratch is a
 // buffer per (device, stream) of its own, in use only between the launches of
 // one call, which train_mutex keeps together when threads share a stream; a
-// captured call goes without (keeps_scratch), with the same bits.  At most 2 *
-// kTrainScratch for each of the first kTrainStreams, kept while the process
-// runs.
-constexpr size_t kTrainScratch = size_t{256} << 20;
+// captured call goes without (keeps_scratch), with the same bits.  For the
+// first kTrainStreams, kept while the process runs.
 constexpr size_t kTrainStreams = 16;
 struct ScratchAlloc {
   int operator()(int, void*, size_t bytes, char** out) const {
@@ -1422,8 +1428,8 @@ size_t ffn_workspace(int64_t rows, int64_t ffn_dim) {
 }
 
 // What callers are told to bring: the calls' own use plus scratch for their
-// products (the forward's query does not know d, so what it names may not hold
-// a copy of a; a call runs with any scratch or none).
+// products' partial sums, the most there can be since the forward's query does
+// not know d (a call runs with any scratch or none).
 size_t ffn_workspace_advised(int64_t rows, int64_t ffn_dim) {
   return align_up(ffn_workspace(rows, ffn_dim), 256) + kSlabBytes;
 }
@@ -1474,15 +1480,24 @@ int ffn_forward(const uint16_t* x, const uint16_t* w1, const uint16_t* w2, uint1
   if (rows == 0) return CREDIT_OK;
   char* ws = nullptr;
   Scratch scratch;
-  CREDIT_TRY(acquire_workspace_with(cfg, ffn_workspace(rows, f), fwd_scratch(rows, d, f), &ws,
-                                    &scratch.base, &scratch.bytes));
+  uint16_t* a = copy_room(out, x, w1, rows, d, f);
+  // In place of x, the copy of a takes scratch too.
+  const size_t copy = a != nullptr || big_shape(rows, f, d)
+                          ? 0 : align_up(static_cast<size_t>(rows) * d * sizeof(uint16_t), 256);
+  const size_t want = copy + fwd_scratch(rows, d, f);
+  CREDIT_TRY(acquire_workspace_with(cfg, ffn_workspace(rows, f), want, &ws, &scratch.base,
+                                    &scratch.bytes));
+  if (copy != 0 && scratch.bytes >= want) {
+    a = reinterpret_cast<uint16_t*>(scratch.base);
+    scratch = Scratch{scratch.base + copy, scratch.bytes - copy};
+  }
   float* rstd = reinterpret_cast<float*>(ws_scratch(ws));
   uint16_t* h = reinterpret_cast<uint16_t*>(
       ws_scratch(ws) + align_up(static_cast<size_t>(rows) * sizeof(float), 256));
   hipStream_t stream = cfg_stream(cfg);
   const int M = static_cast<int>(rows), D = static_cast<int>(d), F = static_cast<int>(f);
-  CREDIT_TRY((launch_norm_gemm<kEpiGelu, KN>(x, rstd, w1, h, nullptr, M, F, D, eps, scratch, stream,
-                                             "ffn gemm1 (gelu)")));
+  CREDIT_TRY((launch_norm_gemm<kEpiGelu, KN>(x, rstd, w1, h, nullptr, a, M, F, D, eps, scratch,
+                                             stream, "ffn gemm1 (gelu)")));
   return launch_gemm<kEpiResidual, KN>(h, nullptr, w2, x, out, nullptr, nullptr, M, D, F, scratch,
                                        stream, "ffn gemm2 (residual)");
 }
@@ -1522,14 +1537,13 @@ int ffn_train_forward(const uint16_t* x, const uint16_t* w1, const uint16_t* w2,
                        "ffn training forward: x, w1, w2, out, u and h must be 16-byte aligned");
   if (rows == 0) return CREDIT_OK;
   hipStream_t stream = cfg_stream(cfg);
-  size_t want = fwd_scratch(rows, d, f);
-  if (want > kTrainScratch) want = std::max(part_bytes(rows, f, d), part_bytes(rows, d, f));
   std::lock_guard<std::mutex> lock(train_mutex());
   Scratch scratch;
-  CREDIT_TRY(train_scratch(stream, want, &scratch));
+  CREDIT_TRY(train_scratch(stream, fwd_scratch(rows, d, f), &scratch));
+  uint16_t* a = copy_room(out, x, w1, rows, d, f);
   const int M = static_cast<int>(rows), D = static_cast<int>(d), F = static_cast<int>(f);
-  CREDIT_TRY((launch_norm_gemm<kEpiGeluSave, KN>(x, rstd, w1, h, u, M, F, D, eps, scratch, stream,
-                                                 "ffn gemm1 (gelu, saving u and h)")));
+  CREDIT_TRY((launch_norm_gemm<kEpiGeluSave, KN>(x, rstd, w1, h, u, a, M, F, D, eps, scratch,
+                                                 stream, "ffn gemm1 (gelu, saving u and h)")));
   return launch_gemm<kEpiResidual, KN>(h, nullptr, w2, x, out, nullptr, nullptr, M, D, F, scratch,
                                        stream, "ffn gemm2 (residual)");
 }
@@ -1635,11 +1649,13 @@ int ffn_backward(const uint16_t* x, const uint16_t* w1, const uint16_t* w2,
   uint16_t* at = reinterpret_cast<uint16_t*>(b + L.at);
   float* da = reinterpret_cast<float*>(b + L.da);
   const int M = static_cast<int>(rows), D = static_cast<int>(d), F = static_cast<int>(f);
-  // u = (x W1^T) rstd (x W1 for [in, out]), h^T = GELU(u)^T, unless saved.
+  // u = (x W1^T) rstd (x W1 for [in, out]), h^T = GELU(u)^T, unless saved; a
+  // copy of a passes through da, which the last product writes.
   if (saved == nullptr)
     CREDIT_TRY((launch_norm_gemm<kEpiUH, KN>(x, reinterpret_cast<float*>(b + L.rstd), w1,
-                                             reinterpret_cast<uint16_t*>(b + L.u), ht, M, F, D,
-                                             eps, scratch, stream, "ffn bwd gemm u")));
+                                             reinterpret_cast<uint16_t*>(b + L.u), ht,
+                                             reinterpret_cast<uint16_t*>(da), M, F, D, eps,
+                                             scratch, stream, "ffn bwd gemm u")));
   // The A operands of the weight gradients in the K-contiguous layout A
   // takes: a^T = bf16(x rstd)^T always, dout^T where no other form reads it.
   if (!KN || saved != nullptr) CREDIT_TRY(launch_transpose(dout, doutt, M, D, nullptr, stream));

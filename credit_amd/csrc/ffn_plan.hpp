@@ -112,17 +112,10 @@ inline GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, bool kn) {
   return p;
 }
 
-// Scratch bytes: the partial sums of a product, and those of the scaled
-// product with its copy of a.
+// Bytes of a product's partial sums.
 inline size_t part_bytes(int64_t M, int64_t N, int64_t K) {
   const int64_t slices = gemm_slices(M, N, K);
   return slices > 1 ? static_cast<size_t>(slices * M * N) * sizeof(float) : 0;
-}
-inline size_t copy_bytes(int64_t M, int64_t F, int64_t D) {
-  return big_shape(M, F, D) ? 0 : (static_cast<size_t>(M) * D * 2 + 255) / 256 * 256;
-}
-inline size_t norm_bytes(int64_t M, int64_t F, int64_t D) {
-  return copy_bytes(M, F, D) + part_bytes(M, F, D);
 }
 
 }  // namespace ffn

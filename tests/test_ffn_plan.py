@@ -3,7 +3,7 @@ import shutil
 
 import pytest
 
-from ffn_plan import gemm_plan
+from ffn_plan import gemm_plan, products
 
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 
@@ -27,3 +27,14 @@ def test_order_of_additions_does_not_depend_on_the_layout():
                 a, b = gemm_plan(m, n, k, False), gemm_plan(m, n, k, True)
                 assert order(a) == order(b), (m, n, k, a, b)
                 assert a.slices == gemm_plan(n, m, k, False).slices, (m, n, k)
+
+
+@pytest.mark.parametrize("rows,d,f", [(2176, 2304, 6912), (4224, 2176, 8576)])
+def test_backward_workspace_holds_no_copy_of_the_input(lib, rows, d, f):
+    """Where no product is split the backward's workspace is its own regions
+    (rstd; u, du, h^T, du^T; dout^T, a^T; da): the rounded copy of x that these
+    shapes read passes through da, so that no workspace is too small for it."""
+    assert all(p.slices == 1 for p in products(rows, d, f, False, train=True).values())
+    own = [4 * rows] + 4 * [2 * rows * f] + 2 * [2 * rows * d] + [4 * rows * d]
+    fixed = 256 + (1 << 20) + (4 << 20)
+    assert lib.credit_ffn_bwd_workspace_bytes(rows, d, f) <= fixed + sum(own) + 256 * len(own)

@@ -60,6 +60,22 @@ def test_split_products(gpu, rows, d, f, layout):
     assert torch.equal(run(x, w1, w2, layout, full), out)
 
 
+@pytest.mark.parametrize("layout", ["linear", "in_out"])
+@pytest.mark.parametrize("rows,d,f", [(128, 256, 8192), (384, 640, 1152), (2048, 256, 256)])
+def test_output_in_place_of_x(gpu, rows, d, f, layout):
+    """The output holds the normalised copy of x until the last product writes
+    it, but not where it is x: the same bits, with room for a copy or none."""
+    print(f"ffn in place rows={rows} d={d} f={f} {layout}", flush=True)
+    x, w1, w2 = make(rows, d, f, layout, gpu)
+    out = run(x, w1, w2, layout)
+    least = torch.zeros(WS_FIXED + 4 * rows + 2 * rows * f, dtype=torch.uint8, device=gpu)
+    for workspace in (None, least):
+        y = x.clone()
+        hip_lib.ffn(y, w1, w2, y, EPS, hip_lib.make_cfg(workspace=workspace), layout=layout)
+        torch.cuda.synchronize()
+        assert torch.equal(y, out)
+
+
 @pytest.mark.parametrize("rows,d,f", [(128, 256, 8192), (1024, 2048, 3200)])
 def test_train_forward_captured_first(gpu, rows, d, f):
     """The training forward as a stream's first call, under capture (it can

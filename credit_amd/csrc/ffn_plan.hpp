@@ -17,10 +17,13 @@ constexpr int kTileN = 128;  // columns of a tile of the other two
 // sizes alone, whatever B's layout and kernel, and the slices are the same for
 // (M, N) and (N, M), so that every entry point that forms a product (either
 // weight layout, recomputed or saved) adds its terms in the same order.
-//  - slices: K pieces.  Time of the units on 256 CUs (flat_us), plus, when
-//    split, kReduceUs and the fp32 sums written and read at kReduceGBs.  1024 x
-//    2048 x 8192 (128 tiles): 131 us on 32 256-tiles, 47 + 5 us in 2 slices;
-//    128 x 8192 x 28672 (64 tiles): 472 us, 103 + 5 us in 4.
+//  - slices: K pieces.  Time of the units on 256 CUs (flat_us; unsplit, the
+//    held kernel's where it can run), plus, when split, kReduceUs and the fp32
+//    sums written and read at kReduceGBs.  1024 x 2048 x 8192 (128 tiles): 131
+//    us on 32 256-tiles, 47 + 5 us in 2 slices; 128 x 8192 x 28672 (64 tiles):
+//    472 us, 103 + 5 us in 4.  1920 x 3200 x 9600 (375 tiles) unsplit: the FFN
+//    takes 339 us, 358 in 2 slices ([K, N], without the held kernel, 342 and
+//    355).
 //  - bm: 256 where its rounds take less by the same count; a tall step costs
 //    less than two flat ones (fewer LDS bytes per MFMA), but 256 x 6144 x
 //    18944 gains (245 -> 196 us) where 512 x 28672 x 8192 would leave half the
@@ -62,6 +65,12 @@ inline double held_us(int64_t units, int64_t steps) {
 }
 constexpr int64_t kSlabBytes = int64_t{64} << 20;  // most fp32 partial sums of one product
 
+// Whether the held kernel can run an unsplit product of a [N, K] B, whichever
+// of its sides is called M.
+inline bool held_fits(int64_t M, int64_t N) {
+  return (M / 128) * (N / 128) > kGemmCus && M > 128 && N > 128;
+}
+
 inline int gemm_slices(int64_t M, int64_t N, int64_t K) {
   constexpr double kReduceUs = 4.0, kReduceGBs = 4000.0;
   const int64_t tiles = (M / 128) * (N / 128), steps = K / kBigK;
@@ -70,6 +79,7 @@ inline int gemm_slices(int64_t M, int64_t N, int64_t K) {
   for (int s = 1; s <= kMaxSlices && steps / s >= 8; ++s) {
     if (s > 1 && s * M * N * 4 > kSlabBytes) break;
     double us = flat_us(tiles * s, (steps + s - 1) / s);
+    if (s == 1 && held_fits(M, N) && held_us(tiles, steps) < us) us = held_us(tiles, steps);
     if (s > 1) us += kReduceUs + s * M * N * 8.0 / (kReduceGBs * 1e3);
     if (us < best_us * 0.95) {
       best = s;
@@ -99,7 +109,7 @@ inline GemmPlan gemm_plan(int64_t M, int64_t N, int64_t K, bool kn) {
     p.bm = 256;
     us = tall_us(tiles / 2, steps);
   }
-  const bool held = p.slices == 1 && tiles > kGemmCus && M > 128 && held_us(tiles, steps) < us;
+  const bool held = p.slices == 1 && held_fits(M, N) && held_us(tiles, steps) < us;
   p.skew = M == p.bm && !held;
   if (held && !kn) {
     p.held = true;

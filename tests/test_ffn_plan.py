@@ -3,7 +3,7 @@ import shutil
 
 import pytest
 
-from ffn_plan import gemm_plan, products
+from ffn_plan import gemm_plan, kernel, products
 
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 
@@ -27,6 +27,14 @@ def test_order_of_additions_does_not_depend_on_the_layout():
                 a, b = gemm_plan(m, n, k, False), gemm_plan(m, n, k, True)
                 assert order(a) == order(b), (m, n, k, a, b)
                 assert a.slices == gemm_plan(n, m, k, False).slices, (m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(1920, 3200, 9600), (2176, 9600, 2432), (1408, 3584, 9600)])
+def test_an_unsplit_product_is_priced_on_the_kernel_that_runs_it(m, n, k):
+    """Products that the ring kernel would run faster in two K slices and the
+    held kernel faster whole."""
+    assert kernel(gemm_plan(m, n, k, False)) == "held"
+    assert gemm_plan(m, n, k, True).slices == 1
 
 
 @pytest.mark.parametrize("rows,d,f", [(2176, 2304, 6912), (4224, 2176, 8576)])

@@ -163,6 +163,19 @@ bool keeps_scratch(hipStream_t stream) {
   return stream != hipStreamPerThread && !stream_capturing(stream);
 }
 
+int ScratchAlloc::operator()(int, void*, size_t bytes, char** out) const {
+  // Relaxed: another thread's stream may be under capture meanwhile.
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  void* p = nullptr;
+  const hipError_t err = hipMalloc(&p, bytes);
+  if (err != hipSuccess) (void)hipGetLastError();
+  CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  if (err != hipSuccess) return CREDIT_ERR_HIP;
+  *out = static_cast<char*>(p);
+  return CREDIT_OK;
+}
+
 int acquire_workspace_with(const credit_cfg* cfg, size_t own, size_t extra, char** base,
                            char** spare, size_t* spare_bytes) {
   const size_t at = align_up(own, 256);

@@ -135,6 +135,11 @@ bool stream_capturing(hipStream_t stream);
 // stream, beside the eager calls of the one it was captured on) and not on the
 // per-thread default stream, one handle for as many streams as threads.
 bool keeps_scratch(hipStream_t stream);
+// Allocates such scratch (StreamScratch): 0, or negative where there is no
+// memory to spare.
+struct ScratchAlloc {
+  int operator()(int device, void* stream, size_t bytes, char** out) const;
+};
 // A workspace of `own` scratch bytes and, where they can be had, `extra` more
 // behind them (*spare, *spare_bytes) that the call can do without: the rest of
 // a caller's workspace, or the library's buffer unless it would have to grow

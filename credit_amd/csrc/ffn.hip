@@ -32,7 +32,6 @@
 #include <algorithm>
 #include <atomic>
 #include <initializer_list>
-#include <mutex>
 #include <type_traits>
 #include <utility>
 
@@ -1369,39 +1368,18 @@ size_t bwd_scratch(int64_t M, int64_t d, int64_t f) {
   return std::max({part_bytes(M, f, d), part_bytes(d, f, M), part_bytes(M, d, f)});
 }
 
-// The training forward brings no workspace and shares none: its scratch is a
-// buffer per (device, stream) of its own, in use only between the launches of
-// one call, which train_mutex keeps together when threads share a stream; a
-// captured call goes without (keeps_scratch), with the same bits.  For the
-// first kTrainStreams, kept while the process runs.
-constexpr size_t kTrainStreams = 16;
-struct ScratchAlloc {
-  int operator()(int, void*, size_t bytes, char** out) const {
-    // Relaxed: another thread's stream may be under capture meanwhile.
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-    void* p = nullptr;
-    const hipError_t err = hipMalloc(&p, bytes);
-    if (err != hipSuccess) (void)hipGetLastError();  // no memory to spare: the call does without
-    CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-    if (err != hipSuccess) return CREDIT_ERR_HIP;
-    *out = static_cast<char*>(p);
-    return CREDIT_OK;
-  }
-};
-std::mutex& train_mutex() {
-  static std::mutex* m = new std::mutex();
-  return *m;
-}
-int train_scratch(hipStream_t stream, size_t want, Scratch* out) {
-  static WorkspaceCache<ScratchAlloc>* cache = new WorkspaceCache<ScratchAlloc>();
-  *out = Scratch{};
-  if (want == 0) return CREDIT_OK;
+// The training forward brings no workspace and shares none: the partial sums of
+// its products, of at most kSlabBytes, live in a buffer per (device, stream) of
+// its own, for the first 16 of them; a captured call goes without
+// (keeps_scratch), with the same bits.
+using TrainScratch = StreamScratch<ScratchAlloc>;
+int train_scratch(hipStream_t stream, size_t want, TrainScratch::Use* use, Scratch* out) {
+  static TrainScratch* scratch = new TrainScratch(kSlabBytes, 16);
+  if (want == 0 || !keeps_scratch(stream)) return CREDIT_OK;
   int dev = 0;
   CREDIT_HIP(hipGetDevice(&dev));
-  if (!keeps_scratch(stream) || !cache->room(dev, stream, kTrainStreams)) return CREDIT_OK;
-  char* p = nullptr;
-  if (cache->get(dev, stream, want, &p) == CREDIT_OK) *out = Scratch{p, want};
+  *use = scratch->use(dev, stream);
+  if (use->base != nullptr) *out = Scratch{use->base, want};
   return CREDIT_OK;
 }
 
@@ -1537,9 +1515,9 @@ int ffn_train_forward(const uint16_t* x, const uint16_t* w1, const uint16_t* w2,
                        "ffn training forward: x, w1, w2, out, u and h must be 16-byte aligned");
   if (rows == 0) return CREDIT_OK;
   hipStream_t stream = cfg_stream(cfg);
-  std::lock_guard<std::mutex> lock(train_mutex());
+  TrainScratch::Use use;
   Scratch scratch;
-  CREDIT_TRY(train_scratch(stream, fwd_scratch(rows, d, f), &scratch));
+  CREDIT_TRY(train_scratch(stream, fwd_scratch(rows, d, f), &use, &scratch));
   uint16_t* a = copy_room(out, x, w1, rows, d, f);
   const int M = static_cast<int>(rows), D = static_cast<int>(d), F = static_cast<int>(f);
   CREDIT_TRY((launch_norm_gemm<kEpiGeluSave, KN>(x, rstd, w1, h, u, a, M, F, D, eps, scratch,

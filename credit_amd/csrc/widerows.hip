@@ -18,7 +18,6 @@
 //   LayerNorm fwd   84 -> 7.8   20 -> 11.7   245 -> 105      9.4 -> 7.7
 //   LayerNorm bwd  101 -> 7.3   28 -> 15.5   324 -> 173     12.5 -> 9.2
 #include <algorithm>
-#include <mutex>
 #include <type_traits>
 
 #include "api_internal.hpp"
@@ -412,35 +411,16 @@ __global__ __launch_bounds__(kThreads) void layernorm_bwd_outputs_kernel(
 
 // ---------------------------------------------------------------- host ----
 // The partials live in a buffer per (device, stream) of their own (5 MiB, for
-// the first kMaxStreams of them, kept while the process runs): calls that
-// brought no workspace before bring none now and share none with the other
-// operations.  One call's two launches stay together under pair_mutex when
-// threads share a stream.
-constexpr size_t kMaxStreams = 64;
+// the first 64 of them): calls that brought no workspace before bring none now
+// and share none with the other operations.
+using Partials = StreamScratch<ScratchAlloc>;
 constexpr size_t kPartialBytes = size_t{kMaxRows} * kMaxParts * kValues * sizeof(double);
-struct PartialAlloc {
-  int operator()(int, void*, size_t bytes, char** out) const {
-    // Relaxed: another thread's stream may be under capture meanwhile.
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-    void* p = nullptr;
-    const hipError_t err = hipMalloc(&p, bytes);
-    if (err != hipSuccess) (void)hipGetLastError();
-    CREDIT_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-    if (err != hipSuccess) return CREDIT_ERR_HIP;
-    *out = static_cast<char*>(p);
-    return CREDIT_OK;
-  }
-};
-std::mutex& pair_mutex() {
-  static std::mutex* m = new std::mutex();
-  return *m;
-}
 
 struct WidePlan {
   dim3 grid;
   int chunk = 0, parts = 0;
   double* partials = nullptr;
+  Partials::Use use;  // held until both launches are made
 };
 
 // Where AUTO takes this path.  Ragged rows of up to kFewWide rows leave most of
@@ -481,10 +461,9 @@ bool wide_wanted(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int6
 }
 
 // Chunks per row: enough workgroups for three to a CU, at least 1024 columns
-// and at most kChunk each.  Holds the pair's lock from then on.  False: the
-// call's other kernels take it.
+// and at most kChunk each.  False: the call's other kernels take it.
 bool wide_plan(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_t cols, bool vec,
-               WidePlan* plan, std::unique_lock<std::mutex>* lock) {
+               WidePlan* plan) {
   if (!wide_wanted(rule, cfg, rows, cols, vec)) return false;
   const int64_t least = (cols + kChunk - 1) / kChunk;
   const int64_t most = std::min<int64_t>(kMaxParts, std::max<int64_t>(least, cols / 1024));
@@ -492,7 +471,7 @@ bool wide_plan(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_
   plan->chunk = static_cast<int>(((cols + want - 1) / want + 7) / 8 * 8);
   plan->parts = static_cast<int>((cols + plan->chunk - 1) / plan->chunk);
   plan->grid = dim3(static_cast<unsigned>(plan->parts), static_cast<unsigned>(rows));
-  static WorkspaceCache<PartialAlloc>* cache = new WorkspaceCache<PartialAlloc>();
+  static Partials* partials = new Partials(kPartialBytes, 64);
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) {
     (void)hipGetLastError();
@@ -505,13 +484,9 @@ bool wide_plan(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_
     (void)hipGetLastError();
     return false;
   }
-  *lock = std::unique_lock<std::mutex>(pair_mutex());
-  char* base = nullptr;
-  if (!cache->room(dev, stream, kMaxStreams) ||
-      cache->get(dev, stream, kPartialBytes, &base) != CREDIT_OK)
-    return false;
-  plan->partials = reinterpret_cast<double*>(base);
-  return true;
+  plan->use = partials->use(dev, stream);
+  plan->partials = reinterpret_cast<double*>(plan->use.base);
+  return plan->partials != nullptr;
 }
 
 template <WideSoftmax OP>
@@ -531,9 +506,8 @@ int wide_softmax(WideSoftmax op, const float* a, const float* dy, float* out, fl
                  float* lse, int64_t rows, int64_t cols, bool vec, const credit_cfg* cfg,
                  bool* taken) {
   const WideRule& rule = op == WideSoftmax::kForward ? kSoftmaxFwdRule : kSoftmaxBwdRule;
-  std::unique_lock<std::mutex> lock;
   WidePlan w;
-  if (!(*taken = wide_plan(rule, cfg, rows, cols, vec, &w, &lock))) return CREDIT_OK;
+  if (!(*taken = wide_plan(rule, cfg, rows, cols, vec, &w))) return CREDIT_OK;
   hipStream_t s = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
   switch (op) {
@@ -548,9 +522,8 @@ int wide_softmax(WideSoftmax op, const float* a, const float* dy, float* out, fl
 
 int wide_quant(const float* x, int8_t* q, float* scale, int64_t rows, int64_t cols, bool vec,
                const credit_cfg* cfg, bool* taken) {
-  std::unique_lock<std::mutex> lock;
   WidePlan w;
-  if (!(*taken = wide_plan(kQuantRule, cfg, rows, cols, vec, &w, &lock))) return CREDIT_OK;
+  if (!(*taken = wide_plan(kQuantRule, cfg, rows, cols, vec, &w))) return CREDIT_OK;
   hipStream_t s = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
   quant_chunks_kernel<<<w.grid, kThreads, 0, s>>>(x, w.partials, c, w.chunk, w.parts);
@@ -562,10 +535,9 @@ int wide_quant(const float* x, int8_t* q, float* scale, int64_t rows, int64_t co
 template <class T>
 int wide_layernorm_bwd(const T* x, const T* dy, const T* gamma, T* dx, int64_t rows, int64_t cols,
                        float eps, bool vec, const credit_cfg* cfg, bool* taken) {
-  std::unique_lock<std::mutex> lock;
   WidePlan w;
   const WideRule& rule = std::is_same_v<T, float> ? kLnBwdRule : kLnBwdHalfRule;
-  if (!(*taken = wide_plan(rule, cfg, rows, cols, vec, &w, &lock))) return CREDIT_OK;
+  if (!(*taken = wide_plan(rule, cfg, rows, cols, vec, &w))) return CREDIT_OK;
   hipStream_t s = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
   const auto launch = [&](auto odd) {
@@ -591,9 +563,8 @@ template int wide_layernorm_bwd<uint16_t>(const uint16_t*, const uint16_t*, cons
 int wide_layernorm_fwd(const uint16_t* x, const uint16_t* gamma, const uint16_t* beta,
                        uint16_t* y, float* mean, float* rstd, int64_t rows, int64_t cols,
                        float eps, bool vec, const credit_cfg* cfg, bool* taken) {
-  std::unique_lock<std::mutex> lock;
   WidePlan w;
-  if (!(*taken = wide_plan(kLnFwdRule, cfg, rows, cols, vec, &w, &lock))) return CREDIT_OK;
+  if (!(*taken = wide_plan(kLnFwdRule, cfg, rows, cols, vec, &w))) return CREDIT_OK;
   hipStream_t s = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
   const auto launch = [&](auto odd) {

@@ -68,12 +68,6 @@ class WorkspaceCache {
     return e == nullptr ? 0 : e->buf.bytes;
   }
 
-  // Whether (device, stream) has an entry, or may have one of at most `most`.
-  bool room(int device, void* stream, size_t most) {
-    std::lock_guard<std::mutex> lock(mu_);
-    return find(device, stream) != nullptr || entries_.size() < most;
-  }
-
   // Every live buffer (for maintenance that must reach all of them).
   std::vector<WsBuffer> live() {
     std::lock_guard<std::mutex> lock(mu_);
@@ -106,6 +100,45 @@ class WorkspaceCache {
   std::mutex mu_;
   std::vector<Entry> entries_;
   std::vector<WsBuffer> retired_;
+  Alloc alloc_;
+};
+
+// Scratch that a call uses between its launches and can do without: a buffer of
+// `bytes` for each of the first `most` (device, stream) pairs that ask, kept
+// while the process runs and never more than bytes * most.
+template <class Alloc>
+class StreamScratch {
+ public:
+  StreamScratch(size_t bytes, size_t most, Alloc alloc = Alloc())
+      : bytes_(bytes), most_(most), alloc_(alloc) {}
+
+  // The buffer, and the lock that keeps the launches of one call together when
+  // threads share a stream: held from here on.  base nullptr (no room for
+  // another pair, or no memory): the call does without, unlocked.
+  struct Use {
+    std::unique_lock<std::mutex> lock;
+    char* base = nullptr;
+  };
+  Use use(int device, void* stream) {
+    Use u{std::unique_lock<std::mutex>(mu_)};
+    for (const Entry& e : entries_)
+      if (e.device == device && e.stream == stream) u.base = e.base;
+    if (u.base == nullptr && entries_.size() < most_ &&
+        alloc_(device, stream, bytes_, &u.base) == 0)
+      entries_.push_back(Entry{device, stream, u.base});
+    if (u.base == nullptr) u.lock.unlock();
+    return u;
+  }
+
+ private:
+  struct Entry {
+    int device;
+    void* stream;
+    char* base;
+  };
+  const size_t bytes_, most_;
+  std::mutex mu_;
+  std::vector<Entry> entries_;
   Alloc alloc_;
 };
 

@@ -700,7 +700,7 @@ extern "C" int credit_layernorm_fwd_bf16(const uint16_t* x, const uint16_t* gamm
     if (vec_ok)
       layernorm_fwd_read_kernel<256, true><<<row_grid, dim3(256), 0, stream>>>(
           x, gamma, beta, y, mean, rstd, c, eps);
-    else if (rows::stream_threads(rows) == 1024)
+    else if (rows::stream_threads(rows::kStream, rows, cols) == 1024)
       layernorm_fwd_read_kernel<1024, false><<<row_grid, dim3(1024), 0, stream>>>(
           x, gamma, beta, y, mean, rstd, c, eps);
     else

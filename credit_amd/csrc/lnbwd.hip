@@ -786,7 +786,7 @@ int layernorm_bwd(const T* x, const T* dy, const T* gamma, T* dx, int64_t rows, 
   CREDIT_TRY(resolve(cfg, cols / E, vec, Slices<T>::capacity, &plan));
   if (plan.variant == CREDIT_VARIANT_READ) {
     const dim3 grid(static_cast<unsigned>(rows));
-    if (rows::stream_threads(rows) == 1024)
+    if (rows::stream_threads(rows::kStream, rows, cols) == 1024)
       layernorm_bwd_read_kernel<T, 1024><<<grid, 1024, 0, stream>>>(x, dy, gamma, dx, c, eps);
     else
       layernorm_bwd_read_kernel<T, 256><<<grid, 256, 0, stream>>>(x, dy, gamma, dx, c, eps);

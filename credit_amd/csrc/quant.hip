@@ -217,7 +217,7 @@ extern "C" int credit_rowwise_quant_f32(const float* x, int8_t* q, float* scale,
   Plan plan;
   CREDIT_TRY(resolve(cfg, cols, vec, kQuantCapacity, "rowwise_quant", &plan));
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (rows::stream_threads(rows) == 1024)
+    if (rows::stream_threads(rows::kStream, rows, cols) == 1024)
       rowwise_quant_read_kernel<1024><<<r, 1024, 0, stream>>>(x, q, scale, c);
     else
       rowwise_quant_read_kernel<256><<<r, 256, 0, stream>>>(x, q, scale, c);

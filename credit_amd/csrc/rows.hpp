@@ -17,6 +17,7 @@
 
 #include "api_internal.hpp"
 #include "common.hpp"
+#include "row_rules.hpp"
 
 namespace credit {
 namespace rows {
@@ -167,9 +168,6 @@ __device__ __forceinline__ f32x4 stream_load(const float* row, int vec) {
 __device__ __forceinline__ void stream_store(float* row, int vec, f32x4 v) {
   __builtin_nontemporal_store(static_cast<f32x4_a4>(v), reinterpret_cast<f32x4_a4*>(row) + vec);
 }
-// Few rows: one workgroup streams a whole row, so a wide one.
-inline unsigned stream_threads(int64_t rows) { return rows < 1024 ? 1024 : 256; }
-
 template <class Fn>
 struct RowsPick {
   Fn fn;

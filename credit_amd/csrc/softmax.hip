@@ -1227,7 +1227,7 @@ extern "C" int credit_softmax_fwd_f32(const float* x, float* p, float* rowmax, f
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (rows::stream_threads(rows) == 1024)
+    if (rows::stream_threads(rows::kSoftmaxFwdStream, rows, cols) == 1024)
       softmax_fwd_read_kernel<1024><<<r, 1024, 0, stream>>>(x, p, rowmax, lse, c);
     else
       softmax_fwd_read_kernel<256><<<r, 256, 0, stream>>>(x, p, rowmax, lse, c);
@@ -1284,7 +1284,7 @@ extern "C" int credit_softmax_bwd_f32(const float* p, const float* dy, float* dx
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (rows::stream_threads(rows) == 1024)
+    if (rows::stream_threads(rows::kSoftmaxBwdStream, rows, cols) == 1024)
       softmax_bwd_read_kernel<1024><<<r, 1024, 0, stream>>>(p, dy, dx, c);
     else
       softmax_bwd_read_kernel<256><<<r, 256, 0, stream>>>(p, dy, dx, c);
@@ -1342,7 +1342,7 @@ extern "C" int credit_softmax_logits_bwd_f32(const float* logits, const float* d
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (rows::stream_threads(rows) == 1024)
+    if (rows::stream_threads(rows::kLogitsStream, rows, cols) == 1024)
       softmax_logits_bwd_read_kernel<1024><<<r, 1024, 0, stream>>>(logits, dy, dx, c);
     else
       softmax_logits_bwd_read_kernel<256><<<r, 256, 0, stream>>>(logits, dy, dx, c);

@@ -1,0 +1,40 @@
+"""The dispatch rules of the any-width row kernels on the host
+(credit_amd/csrc/row_rules.hpp).  No GPU."""
+import ctypes
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+
+OPS = ("row", "softmax_fwd", "softmax_bwd", "softmax_logits_backward")
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    source = Path(__file__).resolve().parent / "cpp" / "row_rules_query.cpp"
+    out = tmp_path_factory.mktemp("rules") / "row_rules.so"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", str(source), "-o",
+                    str(out)], check=True)
+    return ctypes.CDLL(str(out))
+
+
+@pytest.mark.parametrize("op", range(len(OPS)), ids=OPS)
+def test_wide_workgroups_stream_wide_rows_only(rules, op):
+    """1024 lanes to a row measured slower than 256 at these shapes, up to
+    2.5 times, and faster at the wide ones."""
+    def threads(rows, cols):
+        return rules.row_rules_stream_threads(op, ctypes.c_int64(rows), ctypes.c_int64(cols))
+    for rows in (1, 32, 256, 400, 512, 700, 1023, 1024, 4096):
+        for cols in (1, 64, 1000, 1024):
+            assert threads(rows, cols) == 256
+    for rows in (400, 512, 700, 1023):
+        assert threads(rows, 2048) == 256
+    for rows in (1024, 100000):
+        assert threads(rows, 262144) == 256
+    for rows in (1, 128, 256):
+        for cols in (8192, 65536):
+            assert threads(rows, cols) == 1024
+    assert threads(700, 32768) == (256 if OPS[op] == "softmax_bwd" else 1024)

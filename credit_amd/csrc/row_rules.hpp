@@ -31,5 +31,31 @@ inline int stream_threads(const StreamRule& rule, int64_t rows, int64_t cols) {
   return cols >= from ? 1024 : 256;
 }
 
+// A kernel that holds a ragged row in one workgroup's registers (rows.hpp).
+template <class Fn>
+struct RowsPick {
+  Fn fn;
+  int threads;
+  int64_t capacity;  // elements
+  bool few = false;  // for at most kFewRows rows, unless it is one wave
+};
+
+// The first entry that holds `cols`; nullptr: none.  A lone row's time is its
+// lanes' serial work, so the tables open with narrow rows spread over many
+// lanes, taken up to kFewRows rows (softmax logits backward 1 x 1134: 4.5 ->
+// 3.4 us a call); with more, fewer lanes of more vectors keep more rows in
+// flight (softmax forward 16384 x 770: 20.6 us on 64 lanes, 25.2 on 256).  One
+// wave of one vector a lane is the least there is: rows that fit it take it at
+// any number (20000 x 62, us a call, against four vectors a lane: softmax
+// forward 17.8 -> 11.1, backward 12.9 -> 6.4, LayerNorm forward 23.3 -> 11.3).
+constexpr int64_t kFewRows = 2048;
+constexpr int kWaveLanes = 64;
+template <class Fn, int N>
+const RowsPick<Fn>* rows_pick(const RowsPick<Fn> (&table)[N], int64_t rows, int64_t cols) {
+  for (const RowsPick<Fn>& p : table)
+    if (cols <= p.capacity && (rows <= kFewRows || !p.few || p.threads == kWaveLanes)) return &p;
+  return nullptr;
+}
+
 }  // namespace rows
 }  // namespace credit

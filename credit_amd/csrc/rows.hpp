@@ -168,27 +168,6 @@ __device__ __forceinline__ f32x4 stream_load(const float* row, int vec) {
 __device__ __forceinline__ void stream_store(float* row, int vec, f32x4 v) {
   __builtin_nontemporal_store(static_cast<f32x4_a4>(v), reinterpret_cast<f32x4_a4*>(row) + vec);
 }
-template <class Fn>
-struct RowsPick {
-  Fn fn;
-  int threads;
-  int64_t capacity;  // elements
-  bool few = false;  // for at most kFewRows rows
-};
-
-// The first entry that holds `cols`; nullptr: none.  A lone row's time is its
-// lanes' serial work, so the tables open with narrow rows spread over many
-// lanes, taken up to kFewRows rows (softmax logits backward 1 x 1134: 4.5 ->
-// 3.4 us a call); with more, fewer lanes of more vectors keep more rows in
-// flight (softmax forward 16384 x 770: 20.6 us on 64 lanes, 25.2 on 256).
-constexpr int64_t kFewRows = 2048;
-template <class Fn, int N>
-const RowsPick<Fn>* rows_pick(const RowsPick<Fn> (&table)[N], int64_t rows, int64_t cols) {
-  for (const RowsPick<Fn>& p : table)
-    if (cols <= p.capacity && (rows <= kFewRows || !p.few)) return &p;
-  return nullptr;
-}
-
 // The persistent grid of a pick over `rows` rows.
 template <class Fn>
 int rows_grid(const RowsPick<Fn>& pick, int64_t rows, unsigned* grid) {

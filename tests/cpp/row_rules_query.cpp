@@ -10,3 +10,14 @@ extern "C" int row_rules_stream_threads(int op, int64_t rows, int64_t cols) {
   const StreamRule* rules[] = {&kStream, &kSoftmaxFwdStream, &kSoftmaxBwdStream, &kLogitsStream};
   return stream_threads(*rules[op], rows, cols);
 }
+
+// The entry that rows_pick takes from the softmax tables' ladder: lanes * 100 +
+// vectors a lane.
+extern "C" int row_rules_pick(int64_t rows, int64_t cols) {
+  static const RowsPick<int> ladder[] = {
+      {6401, 64, 256, true},    {12801, 128, 512, true}, {25601, 256, 1024, true},
+      {25602, 256, 2048, true}, {6404, 64, 1024},        {12804, 128, 2048},
+      {25604, 256, 4096}};
+  const RowsPick<int>* p = rows_pick(ladder, rows, cols);
+  return p == nullptr ? 0 : p->fn;
+}

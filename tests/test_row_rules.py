@@ -38,3 +38,14 @@ def test_wide_workgroups_stream_wide_rows_only(rules, op):
         for cols in (8192, 65536):
             assert threads(rows, cols) == 1024
     assert threads(700, 32768) == (256 if OPS[op] == "softmax_bwd" else 1024)
+
+
+def test_narrow_rows_take_the_least_work_at_any_number(rules):
+    """Rows that one wave holds with a vector a lane are not given four."""
+    def pick(rows, cols):
+        return rules.row_rules_pick(ctypes.c_int64(rows), ctypes.c_int64(cols))
+    for rows in (1, 2048, 2049, 3000, 20000, 1 << 24):
+        for cols in (1, 3, 62, 256):
+            assert pick(rows, cols) == 6401, (rows, cols)
+    assert pick(100, 770) == 25601 and pick(16384, 770) == 6404
+    assert pick(100, 4097) == 0

@@ -682,7 +682,9 @@ extern "C" int credit_layernorm_fwd_bf16(const uint16_t* x, const uint16_t* gamm
     CREDIT_TRY(wide_layernorm_fwd(x, gamma, beta, y, mean, rstd, rows, cols, eps, vec_ok, cfg,
                                   &taken));
   if (taken) return CREDIT_OK;
-  if (!vec_ok && dwords && cfg_variant(cfg) == CREDIT_VARIANT_AUTO) {
+  const rows::NarrowRule& few = cols % 2 != 0 ? rows::kLnHalfOddNarrow : rows::kLnHalfNarrow;
+  if (!vec_ok && dwords && cfg_variant(cfg) == CREDIT_VARIANT_AUTO &&
+      !rows::narrow(few, rows, cols)) {
     const auto* rp = cols % 2 != 0 ? rows::rows_pick(RowsTable<true>::table, rows, cols)
                                    : rows::rows_pick(RowsTable<false>::table, rows, cols);
     if (rp != nullptr) {

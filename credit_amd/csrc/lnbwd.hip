@@ -769,7 +769,10 @@ int layernorm_bwd(const T* x, const T* dy, const T* gamma, T* dx, int64_t rows, 
   }
   hipStream_t stream = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
-  if (!vec && dwords && cfg_variant(cfg) == CREDIT_VARIANT_AUTO) {
+  const rows::NarrowRule& few = std::is_same_v<T, float> ? rows::kLnBwdNarrow
+                                : cols % 2 != 0 ? rows::kLnHalfOddNarrow : rows::kLnHalfNarrow;
+  if (!vec && dwords && cfg_variant(cfg) == CREDIT_VARIANT_AUTO &&
+      !rows::narrow(few, rows, cols)) {
     const rows::RowsPick<RowsFn<T>>* pick = rows::rows_pick(RowsTable<T, false>::table, rows, cols);
     if constexpr (std::is_same_v<T, uint16_t>) {
       if (cols % 2 != 0) pick = rows::rows_pick(RowsTable<T, true>::table, rows, cols);

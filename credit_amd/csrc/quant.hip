@@ -119,8 +119,9 @@ __global__ __launch_bounds__(THREADS) void rowwise_quant_rows_kernel(
   }
 }
 
-// Two passes over the row, at any width and address.
-template <int THREADS>
+// Two passes over the row, at any width and address.  VEC: in vectors with a
+// tail of single elements; else single elements.
+template <int THREADS, bool VEC>
 __global__ __launch_bounds__(THREADS) void rowwise_quant_read_kernel(
     const float* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scale, int cols) {
   constexpr int NW = THREADS / kWave;
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(THREADS) void rowwise_quant_read_kernel(
   const size_t off = static_cast<size_t>(blockIdx.x) * cols;
   const float* xr = x + off;
   float lm = 0.0f;
-  const int nvec = cols >> 2;
+  const int nvec = VEC ? cols >> 2 : 0;
   int i = tid;
   for (; i + THREADS < nvec; i += 2 * THREADS)
     lm = fmax_nan(lm, fmax_nan(absmax4(rows::stream_load(xr, i)),
@@ -217,10 +218,11 @@ extern "C" int credit_rowwise_quant_f32(const float* x, int8_t* q, float* scale,
   Plan plan;
   CREDIT_TRY(resolve(cfg, cols, vec, kQuantCapacity, "rowwise_quant", &plan));
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (rows::stream_threads(rows::kStream, rows, cols) == 1024)
-      rowwise_quant_read_kernel<1024><<<r, 1024, 0, stream>>>(x, q, scale, c);
-    else
-      rowwise_quant_read_kernel<256><<<r, 256, 0, stream>>>(x, q, scale, c);
+    rows::launch_read(rows::kStream, rows, cols, vec, [&](auto threads, auto vectors) {
+      constexpr int kT = decltype(threads)::value;
+      rowwise_quant_read_kernel<kT, decltype(vectors)::value>
+          <<<r, kT, 0, stream>>>(x, q, scale, c);
+    });
     return check_launch("rowwise_quant_read_kernel");
   }
   const Pick<QuantFn>* pk = pick_for(kQuant, plan.chunk);

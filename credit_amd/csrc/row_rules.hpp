@@ -17,18 +17,43 @@ namespace rows {
 // 17).  The softmaxes, whose passes are longer, gain later (forward 700 x
 // 12288: 17.8 and 18.7; backward 400 x 16384: 19.1 and 20.4, so never above 256
 // rows).
+//
+// A row without the 16-byte layout moves in vectors (at 4-byte addresses, its
+// last elements by themselves) from `vectors` columns on, below that in single
+// elements: a vector leaves three lanes of four idle there and the last
+// elements take a step of their own (softmax forward 3000 x 257: 6.9 us in
+// elements, 7.4 in vectors; backward 3000 x 1002: 7.6, 9.6).
 struct StreamRule {
-  int64_t one, two, three;
+  int64_t one, two, three, vectors;
 };
 constexpr int64_t kNever = INT64_MAX;
-constexpr StreamRule kStream{2048, 6144, 6144};
-constexpr StreamRule kSoftmaxFwdStream{6144, 6144, 16384};
-constexpr StreamRule kSoftmaxBwdStream{6144, kNever, kNever};
-constexpr StreamRule kLogitsStream{2048, 4096, 6144};
+constexpr StreamRule kStream{2048, 6144, 6144, 512};
+constexpr StreamRule kSoftmaxFwdStream{6144, 6144, 16384, 512};
+constexpr StreamRule kSoftmaxBwdStream{6144, kNever, kNever, 3072};
+constexpr StreamRule kLogitsStream{2048, 4096, 6144, 512};
 inline int stream_threads(const StreamRule& rule, int64_t rows, int64_t cols) {
   const int64_t from = rows <= 256 ? rule.one : rows <= 512 ? rule.two
                                    : rows < 1024 ? rule.three : kNever;
   return cols >= from ? 1024 : 256;
+}
+
+// Rows narrow enough, and few enough, that AUTO runs READ where it could hold
+// them in registers: both corners' columns are exclusive, rows inclusive.  A
+// row of a few elements shares its cache lines with other workgroups' rows, to
+// which READ's plain stores do less harm than nontemporal ones, and 256 lanes
+// take one element each without a loop (softmax backward 3000 x 3: 2.7 us, 3.6
+// held; 1500 x 257: 2.7, 2.9; 8000 x 62: 4.7, 4.1; LayerNorm forward 300 x 7:
+// 2.6, 3.3; 300 x 201: 2.7, 2.9; 3000 x 7: 5.2, 4.6).
+struct NarrowRule {
+  int64_t cols1, rows1, cols2, rows2;
+};
+constexpr NarrowRule kSoftmaxNarrow{8, 2048, 0, 0};  // forward and logits backward
+constexpr NarrowRule kSoftmaxBwdNarrow{16, 12288, 512, 4096};
+constexpr NarrowRule kLnBwdNarrow{8, 1024, 0, 0};       // fp32
+constexpr NarrowRule kLnHalfNarrow{16, 2048, 64, 512};  // bf16, both directions
+constexpr NarrowRule kLnHalfOddNarrow{16, 2048, 256, 512};
+inline bool narrow(const NarrowRule& rule, int64_t rows, int64_t cols) {
+  return (cols < rule.cols1 && rows <= rule.rows1) || (cols < rule.cols2 && rows <= rule.rows2);
 }
 
 // A kernel that holds a ragged row in one workgroup's registers (rows.hpp).

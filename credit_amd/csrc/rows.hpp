@@ -15,6 +15,8 @@
 // overlap without a second set of registers.
 #pragma once
 
+#include <type_traits>
+
 #include "api_internal.hpp"
 #include "common.hpp"
 #include "row_rules.hpp"
@@ -168,6 +170,18 @@ __device__ __forceinline__ f32x4 stream_load(const float* row, int vec) {
 __device__ __forceinline__ void stream_store(float* row, int vec, f32x4 v) {
   __builtin_nontemporal_store(static_cast<f32x4_a4>(v), reinterpret_cast<f32x4_a4*>(row) + vec);
 }
+// Launches READ with the lanes and the loads its rules give a row:
+// launch(integral_constant threads, bool_constant vectors).
+template <class Launch>
+void launch_read(const StreamRule& rule, int64_t rows, int64_t cols, bool vec, Launch&& launch) {
+  if (stream_threads(rule, rows, cols) == 1024)  // wide rows
+    launch(std::integral_constant<int, 1024>{}, std::true_type{});
+  else if (vec || cols >= rule.vectors)
+    launch(std::integral_constant<int, 256>{}, std::true_type{});
+  else
+    launch(std::integral_constant<int, 256>{}, std::false_type{});
+}
+
 // The persistent grid of a pick over `rows` rows.
 template <class Fn>
 int rows_grid(const RowsPick<Fn>& pick, int64_t rows, unsigned* grid) {

@@ -722,10 +722,10 @@ __global__ __launch_bounds__(THREADS) void softmax_rows_kernel(
   }
 }
 
-// Streaming forward: online (max, sum) pass, then the output pass, in vectors
-// at any 4-byte address with a tail of single elements (4-byte loads
-// throughout ran 1 x 250001 at 12 GB/s).
-template <int THREADS>
+// Streaming forward: online (max, sum) pass, then the output pass.  VEC: in
+// vectors at any 4-byte address with a tail of single elements (4-byte loads
+// throughout ran 1 x 250001 at 12 GB/s); else single elements.
+template <int THREADS, bool VEC>
 __global__ __launch_bounds__(THREADS) void softmax_fwd_read_kernel(
     const float* __restrict__ x, float* __restrict__ p, float* __restrict__ rowmax,
     float* __restrict__ lse, int cols) {
@@ -738,7 +738,7 @@ __global__ __launch_bounds__(THREADS) void softmax_fwd_read_kernel(
   float* pr = p + static_cast<size_t>(row) * cols;
   float m = kNegInf;  // running max of the finite path
   double s = 0.0;     // sum of e^(x - m)
-  const int nvec = cols >> 2;
+  const int nvec = VEC ? cols >> 2 : 0;
   int i = tid;
   for (; i + THREADS < nvec; i += 2 * THREADS) {
     const f32x4 a = rows::stream_load(xr, i), b = rows::stream_load(xr, i + THREADS);
@@ -826,7 +826,7 @@ __global__ __launch_bounds__(THREADS) void softmax_bwd_slice_kernel(
   split_leave(sa);
 }
 
-template <int THREADS>
+template <int THREADS, bool VEC>
 __global__ __launch_bounds__(THREADS) void softmax_bwd_read_kernel(
     const float* __restrict__ p, const float* __restrict__ dy, float* __restrict__ dx, int cols) {
   constexpr int NW = THREADS / kWave;
@@ -836,7 +836,7 @@ __global__ __launch_bounds__(THREADS) void softmax_bwd_read_kernel(
   const float* pr = p + off;
   const float* dr = dy + off;
   double acc = 0.0;
-  const int nvec = cols >> 2;
+  const int nvec = VEC ? cols >> 2 : 0;
   int i = tid;
   for (; i + THREADS < nvec; i += 2 * THREADS) {
     const f32x4 a = rows::stream_load(pr, i), b = rows::stream_load(pr, i + THREADS);
@@ -957,7 +957,7 @@ __global__ __launch_bounds__(THREADS) void softmax_logits_bwd_slice_kernel(
 
 // Streaming logits backward: online (max, sum) over the logits; sum p*dy
 // (re-reading logits and dy); output pass (re-reading both again).
-template <int THREADS>
+template <int THREADS, bool VEC>
 __global__ __launch_bounds__(THREADS) void softmax_logits_bwd_read_kernel(
     const float* __restrict__ logits, const float* __restrict__ dy, float* __restrict__ dx,
     int cols) {
@@ -970,7 +970,7 @@ __global__ __launch_bounds__(THREADS) void softmax_logits_bwd_read_kernel(
   const float* dr = dy + off;
   float m = kNegInf;
   double s = 0.0;
-  const int nvec = cols >> 2;
+  const int nvec = VEC ? cols >> 2 : 0;
   for (int i = tid; i < nvec; i += THREADS) {
     const f32x4 a = rows::stream_load(lr, i);
     online_update(max4(a), m, s);
@@ -1047,11 +1047,12 @@ const rows::RowsPick<RowsFn> kLogitsRows[] = CREDIT_ROWS_TABLE(kOpLogits, 26);
 #undef CREDIT_ROWS_TABLE
 
 // AUTO on a shape without the 16-byte layout: the rows kernel that holds the
-// row.  nullptr: READ (explicit, or wider rows).
+// row.  nullptr: READ (explicit, wider or narrow rows).
 template <int N>
 const rows::RowsPick<RowsFn>* ragged_pick(const rows::RowsPick<RowsFn> (&table)[N],
-                                          const credit_cfg* cfg, int64_t rows, int64_t cols,
-                                          bool vec) {
+                                          const rows::NarrowRule& narrow, const credit_cfg* cfg,
+                                          int64_t rows, int64_t cols, bool vec) {
+  if (rows::narrow(narrow, rows, cols)) return nullptr;
   if (vec || cfg_variant(cfg) != CREDIT_VARIANT_AUTO || rows > (int64_t{1} << 30)) return nullptr;
   return rows::rows_pick(table, rows, cols);
 }
@@ -1220,17 +1221,17 @@ extern "C" int credit_softmax_fwd_f32(const float* x, float* p, float* rowmax, f
   CREDIT_TRY(wide_softmax(WideSoftmax::kForward, x, nullptr, p, rowmax, lse, rows, cols, vec, cfg,
                           &taken));
   if (taken) return CREDIT_OK;
-  if (const auto* pick = ragged_pick(kFwdRows, cfg, rows, cols, vec))
+  if (const auto* pick = ragged_pick(kFwdRows, rows::kSoftmaxNarrow, cfg, rows, cols, vec))
     return launch_rows(*pick, x, nullptr, p, rowmax, lse, rows, cols, stream);
   Plan plan;
   CREDIT_TRY(resolve_fwd(cfg, cols, vec, &plan));
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (rows::stream_threads(rows::kSoftmaxFwdStream, rows, cols) == 1024)
-      softmax_fwd_read_kernel<1024><<<r, 1024, 0, stream>>>(x, p, rowmax, lse, c);
-    else
-      softmax_fwd_read_kernel<256><<<r, 256, 0, stream>>>(x, p, rowmax, lse, c);
+    rows::launch_read(rows::kSoftmaxFwdStream, rows, cols, vec, [&](auto threads, auto vectors) {
+      constexpr int kT = decltype(threads)::value;
+      softmax_fwd_read_kernel<kT, decltype(vectors)::value><<<r, kT, 0, stream>>>(x, p, rowmax, lse, c);
+    });
     return check_launch("softmax_fwd_read_kernel");
   }
   if (fwd_group_ok(plan)) {
@@ -1277,17 +1278,17 @@ extern "C" int credit_softmax_bwd_f32(const float* p, const float* dy, float* dx
   CREDIT_TRY(wide_softmax(WideSoftmax::kBackward, p, dy, dx, nullptr, nullptr, rows, cols, vec, cfg,
                           &taken));
   if (taken) return CREDIT_OK;
-  if (const auto* pick = ragged_pick(kBwdRows, cfg, rows, cols, vec))
+  if (const auto* pick = ragged_pick(kBwdRows, rows::kSoftmaxBwdNarrow, cfg, rows, cols, vec))
     return launch_rows(*pick, p, dy, dx, nullptr, nullptr, rows, cols, stream);
   Plan plan;
   CREDIT_TRY(resolve_bwd(cfg, cols, vec, &plan));
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (rows::stream_threads(rows::kSoftmaxBwdStream, rows, cols) == 1024)
-      softmax_bwd_read_kernel<1024><<<r, 1024, 0, stream>>>(p, dy, dx, c);
-    else
-      softmax_bwd_read_kernel<256><<<r, 256, 0, stream>>>(p, dy, dx, c);
+    rows::launch_read(rows::kSoftmaxBwdStream, rows, cols, vec, [&](auto threads, auto vectors) {
+      constexpr int kT = decltype(threads)::value;
+      softmax_bwd_read_kernel<kT, decltype(vectors)::value><<<r, kT, 0, stream>>>(p, dy, dx, c);
+    });
     return check_launch("softmax_bwd_read_kernel");
   }
   if (bwd_group_ok(plan)) {
@@ -1335,17 +1336,17 @@ extern "C" int credit_softmax_logits_bwd_f32(const float* logits, const float* d
   CREDIT_TRY(wide_softmax(WideSoftmax::kLogits, logits, dy, dx, nullptr, nullptr, rows, cols, vec, cfg,
                           &taken));
   if (taken) return CREDIT_OK;
-  if (const auto* pick = ragged_pick(kLogitsRows, cfg, rows, cols, vec))
+  if (const auto* pick = ragged_pick(kLogitsRows, rows::kSoftmaxNarrow, cfg, rows, cols, vec))
     return launch_rows(*pick, logits, dy, dx, nullptr, nullptr, rows, cols, stream);
   Plan plan;
   CREDIT_TRY(resolve(cfg, cols, vec, kBwdCapacity, "softmax_logits_bwd", &plan));
   const int c = static_cast<int>(cols);
   const unsigned r = static_cast<unsigned>(rows);
   if (plan.variant == CREDIT_VARIANT_READ) {
-    if (rows::stream_threads(rows::kLogitsStream, rows, cols) == 1024)
-      softmax_logits_bwd_read_kernel<1024><<<r, 1024, 0, stream>>>(logits, dy, dx, c);
-    else
-      softmax_logits_bwd_read_kernel<256><<<r, 256, 0, stream>>>(logits, dy, dx, c);
+    rows::launch_read(rows::kLogitsStream, rows, cols, vec, [&](auto threads, auto vectors) {
+      constexpr int kT = decltype(threads)::value;
+      softmax_logits_bwd_read_kernel<kT, decltype(vectors)::value><<<r, kT, 0, stream>>>(logits, dy, dx, c);
+    });
     return check_launch("softmax_logits_bwd_read_kernel");
   }
   const Pick<BwdFn>* pk = pick_for(kLogits, plan.chunk);

@@ -21,3 +21,11 @@ extern "C" int row_rules_pick(int64_t rows, int64_t cols) {
   const RowsPick<int>* p = rows_pick(ladder, rows, cols);
   return p == nullptr ? 0 : p->fn;
 }
+
+// op: 0 softmax forward and logits backward, 1 softmax backward, 2 LayerNorm
+// backward fp32, 3 and 4 bf16 LayerNorm of even and odd width.
+extern "C" int row_rules_narrow(int op, int64_t rows, int64_t cols) {
+  const NarrowRule* rules[] = {&kSoftmaxNarrow, &kSoftmaxBwdNarrow, &kLnBwdNarrow, &kLnHalfNarrow,
+                               &kLnHalfOddNarrow};
+  return narrow(*rules[op], rows, cols);
+}

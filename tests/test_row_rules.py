@@ -49,3 +49,17 @@ def test_narrow_rows_take_the_least_work_at_any_number(rules):
             assert pick(rows, cols) == 6401, (rows, cols)
     assert pick(100, 770) == 25601 and pick(16384, 770) == 6404
     assert pick(100, 4097) == 0
+
+
+@pytest.mark.parametrize("op,read,held", [
+    (0, [(100, 3), (2048, 7)], [(100, 8), (3000, 3), (20000, 62)]),
+    (1, [(100, 3), (3000, 3), (8000, 15), (700, 62), (4096, 257)],
+     [(20000, 3), (8000, 62), (100, 601), (20000, 257)]),
+    (2, [(100, 3), (700, 7)], [(1500, 3), (100, 15), (700, 62)]),
+    (3, [(100, 6), (1500, 14), (300, 62)], [(3000, 6), (700, 62), (100, 130)]),
+    (4, [(100, 7), (1500, 15), (300, 201)], [(3000, 7), (700, 201), (100, 257)])])
+def test_few_narrow_rows_run_read(rules, op, read, held):
+    """Shapes that measured faster on READ, and on the kernels that hold a row."""
+    for shapes, want in ((read, 1), (held, 0)):
+        for rows, cols in shapes:
+            assert rules.row_rules_narrow(op, ctypes.c_int64(rows), ctypes.c_int64(cols)) == want

@@ -556,6 +556,9 @@ __global__ __launch_bounds__(THREADS) void layernorm_bwd_rows_kernel(
 
 template <class T>
 using RowsFn = void (*)(const T*, const T*, const T*, T*, int, int, float);
+// Five and six vectors a lane beside eight: a lane's empty vectors cost an odd
+// row their shifts all the same (bf16 2048 x 16385: 96 us with eight, 67 with
+// five; READ 73).
 template <class T, bool ODD>
 struct RowsTable {
   static constexpr int kE = Vec<T>::kN;
@@ -567,7 +570,10 @@ struct RowsTable {
       {layernorm_bwd_rows_kernel<T, ODD, 64, 4>, 64, 256 * kE},
       {layernorm_bwd_rows_kernel<T, ODD, 128, 4>, 128, 512 * kE},
       {layernorm_bwd_rows_kernel<T, ODD, 256, 4>, 256, 1024 * kE},
+      {layernorm_bwd_rows_kernel<T, ODD, 256, 5>, 256, 1280 * kE},
       {layernorm_bwd_rows_kernel<T, ODD, 256, 8>, 256, 2048 * kE},
+      {layernorm_bwd_rows_kernel<T, ODD, 512, 5>, 512, 2560 * kE},
+      {layernorm_bwd_rows_kernel<T, ODD, 512, 6>, 512, 3072 * kE},
       {layernorm_bwd_rows_kernel<T, ODD, 512, 8>, 512, 4096 * kE},
       {layernorm_bwd_rows_kernel<T, ODD, 512, 16>, 512, 8192 * kE},
   };

@@ -37,3 +37,15 @@ def test_narrow_layernorm_backward(gpu, rows, cols, shift, dtype):
 @pytest.mark.parametrize("rows,cols,shift", SHAPES)
 def test_narrow_layernorm_forward(gpu, rows, cols, shift):
     ragged.test_ragged_layernorm_forward(gpu, rows, cols, shift)
+
+
+# LayerNorm backward: the last and the first width of the tables' entries of five
+# and six vectors a lane (fp32 5120, 10240 and 12288 columns, bf16 twice that).
+@pytest.mark.parametrize("cols,shift,dtype", [
+    (5119, 0, torch.float32), (5121, 0, torch.float32), (10239, 1, torch.float32),
+    (10241, 0, torch.float32), (12287, 0, torch.float32), (12289, 0, torch.float32),
+    (10239, 0, torch.bfloat16), (10242, 0, torch.bfloat16), (20479, 2, torch.bfloat16),
+    (20478, 0, torch.bfloat16), (20481, 0, torch.bfloat16), (24574, 0, torch.bfloat16),
+    (24577, 0, torch.bfloat16)])
+def test_layernorm_backward_table_edges(gpu, cols, shift, dtype):
+    ragged.test_ragged_layernorm_backward(gpu, 270, cols, shift, dtype)

@@ -56,6 +56,47 @@ inline bool narrow(const NarrowRule& rule, int64_t rows, int64_t cols) {
   return (cols < rule.cols1 && rows <= rule.rows1) || (cols < rule.cols2 && rows <= rule.rows2);
 }
 
+// Few wide rows in two launches of chunks (widerows.hip), columns exclusive:
+// ragged rows past `few` columns with up to kFewWide rows and past `many` with
+// more, rows of whole 16-byte vectors past `vec`.
+//
+// Ragged rows of up to kFewWide rows leave most of the chip idle on a workgroup
+// each: from 16384 columns on (8195: the same or 0.4 us slower; quantisation,
+// one pass of a narrow output, from 32768; bf16 LayerNorm forward 16 x 16386 7.1
+// us, 7.6 in chunks, 64 x 16387 9.6, 8.5).  More rows fill it, and the kernels
+// that hold a row in registers read it once (softmax logits backward 256 x
+// 40003: 30 us, 33.5 in chunks); past `many` columns they stream it more than
+// once, or so few rows fit that latency shows (LayerNorm backward 384 x 40003:
+// 76 us, 49).
+//
+// Rows of whole vectors have faster kernels, SPLIT among them: at most 32 rows,
+// wide ones and little data (64 x 131072: 22, 27).  One workgroup that holds the
+// row is sooner done than two launches: softmax forward and logits backward up
+// to 24576 columns (8 x 24584: 7.5 and 7.8 us, 6.1 and 6.2 in chunks; 32 x 24584
+// 7.9 and 8.3, 7.4 and 8.8), softmax backward up to 32768 (8 x 24584: 4.9, 6.0;
+// 8 x 36864, SPLIT: 8.1, 6.0), quantisation up to 65536 (16 x 65536: 6.4, 7.0;
+// 16 x 65544, SPLIT: 7.8, 5.9), LayerNorm forward up to 57344 (24 x 49160: 6.6,
+// 7.2; 16 x 65536: 7.2, 7.1), its bf16 backward up to 49152.  16 x 262144 would
+// gain too (softmax forward 13.4, 9.9) but AUTO is known to run SPLIT there
+// (credit_last_split_shape).
+struct WideRule {
+  int64_t few, many, vec;
+};
+constexpr int64_t kWideMaxRows = 2048;
+constexpr int64_t kFewWide = 128;
+constexpr WideRule kSoftmaxFwdWide{16384, 32768, 24576};
+constexpr WideRule kSoftmaxBwdWide{16384, 53248, 32768};
+constexpr WideRule kLogitsWide{16384, 53248, 24576};
+constexpr WideRule kLnBwdWide{16384, 32768, 24576};
+constexpr WideRule kLnBwdHalfWide{16384, 32768, 49152};
+constexpr WideRule kLnFwdWide{20480, 32768, 57344};
+constexpr WideRule kQuantWide{32768, 65536, 65536};
+inline bool wide(const WideRule& rule, int64_t rows, int64_t cols, bool vec) {
+  if (rows > kWideMaxRows) return false;
+  if (vec) return rows <= 32 && cols > rule.vec && rows * cols <= int64_t{1} << 21;
+  return cols > (rows <= kFewWide ? rule.few : rule.many);
+}
+
 // A kernel that holds a ragged row in one workgroup's registers (rows.hpp).
 template <class Fn>
 struct RowsPick {

@@ -35,7 +35,7 @@ constexpr int kVpt = 4;
 constexpr int kChunk = kThreads * kVpt * 4;  // columns a workgroup holds
 constexpr int kMaxParts = kWave;             // one wave merges a row's chunks
 constexpr int kValues = 5;                   // fp64 values per chunk
-constexpr int kMaxRows = 2048;
+constexpr int kMaxRows = rows::kWideMaxRows;
 constexpr float kNegInf = -__builtin_inff();
 
 // Where a workgroup is: its row and its chunk's columns.
@@ -423,47 +423,18 @@ struct WidePlan {
   Partials::Use use;  // held until both launches are made
 };
 
-// Where AUTO takes this path.  Ragged rows of up to kFewWide rows leave most of
-// the chip idle on a workgroup each: from 16384 columns on (8195: the same or
-// 0.4 us slower; quantisation, one pass of a narrow output, from 32768).  More
-// rows fill it, and the kernels that hold a row in registers read it once
-// (softmax logits backward 256 x 40003: 30 us, 33.5 here); past `many` columns
-// they stream it more than once, or so few rows fit that latency shows
-// (LayerNorm backward 384 x 40003: 76 us, 49 here).  Rows of whole 16-byte
-// vectors have faster kernels, SPLIT among them: at most 32 rows, wide ones and
-// little data (softmax forward 16 x 16384: 6.0 us, 6.9 here; 16 x 65536: 16,
-// 7.4; logits backward 64 x 32768: 9.4, 10.1; 64 x 131072: 22, 27).
-// Quantisation holds rows of up to 65536 columns in one workgroup (16 x 65536:
-// 6.7, 7.0); wider ones ran in SPLIT groups (16 x 70952: 8.0, 7.0).  16 x
-// 262144 would gain too (forward 13.4, 9.9 here) but AUTO is known to run SPLIT
-// there (credit_last_split_shape).  A caller's workspace is SPLIT's.  bf16 rows
-// are half the bytes: LayerNorm forward 16 x 16386 7.1 us, 7.6 here, 64 x 16387
-// 9.6, 8.5; aligned 16 x 32768 5.5, 7.2, 32 x 65536 8.5, 7.0.
-struct WideRule {
-  int64_t few, many, vec;  // columns, exclusive
-};
-constexpr WideRule kSoftmaxFwdRule{16384, 32768, 24576};
-constexpr WideRule kSoftmaxBwdRule{16384, 53248, 24576};
-constexpr WideRule kLnBwdRule{16384, 32768, 24576};
-constexpr WideRule kLnBwdHalfRule{16384, 32768, 49152};
-constexpr WideRule kLnFwdRule{20480, 32768, 49152};
-constexpr WideRule kQuantRule{32768, 65536, 65536};
-constexpr int64_t kFewWide = 128;
-bool wide_wanted(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_t cols,
+// Where AUTO takes this path (row_rules.hpp).  A caller's workspace is SPLIT's.
+bool wide_wanted(const rows::WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_t cols,
                  bool vec) {
-  if (cfg_variant(cfg) != CREDIT_VARIANT_AUTO || rows > kMaxRows ||
-      cols > int64_t{kMaxParts} * kChunk)
-    return false;
-  if (vec)
-    return (cfg == nullptr || cfg->workspace == nullptr) && rows <= 32 && cols > rule.vec &&
-           rows * cols <= int64_t{1} << 21;
-  return cols > (rows <= kFewWide ? rule.few : rule.many);
+  return cfg_variant(cfg) == CREDIT_VARIANT_AUTO && cols <= int64_t{kMaxParts} * kChunk &&
+         !(vec && cfg != nullptr && cfg->workspace != nullptr) &&
+         rows::wide(rule, rows, cols, vec);
 }
 
 // Chunks per row: enough workgroups for three to a CU, at least 1024 columns
 // and at most kChunk each.  False: the call's other kernels take it.
-bool wide_plan(const WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_t cols, bool vec,
-               WidePlan* plan) {
+bool wide_plan(const rows::WideRule& rule, const credit_cfg* cfg, int64_t rows, int64_t cols,
+               bool vec, WidePlan* plan) {
   if (!wide_wanted(rule, cfg, rows, cols, vec)) return false;
   const int64_t least = (cols + kChunk - 1) / kChunk;
   const int64_t most = std::min<int64_t>(kMaxParts, std::max<int64_t>(least, cols / 1024));
@@ -505,7 +476,9 @@ int launch_softmax(const WidePlan& w, const float* a, const float* dy, float* ou
 int wide_softmax(WideSoftmax op, const float* a, const float* dy, float* out, float* rowmax,
                  float* lse, int64_t rows, int64_t cols, bool vec, const credit_cfg* cfg,
                  bool* taken) {
-  const WideRule& rule = op == WideSoftmax::kForward ? kSoftmaxFwdRule : kSoftmaxBwdRule;
+  const rows::WideRule& rule = op == WideSoftmax::kForward    ? rows::kSoftmaxFwdWide
+                               : op == WideSoftmax::kBackward ? rows::kSoftmaxBwdWide
+                                                              : rows::kLogitsWide;
   WidePlan w;
   if (!(*taken = wide_plan(rule, cfg, rows, cols, vec, &w))) return CREDIT_OK;
   hipStream_t s = cfg_stream(cfg);
@@ -523,7 +496,7 @@ int wide_softmax(WideSoftmax op, const float* a, const float* dy, float* out, fl
 int wide_quant(const float* x, int8_t* q, float* scale, int64_t rows, int64_t cols, bool vec,
                const credit_cfg* cfg, bool* taken) {
   WidePlan w;
-  if (!(*taken = wide_plan(kQuantRule, cfg, rows, cols, vec, &w))) return CREDIT_OK;
+  if (!(*taken = wide_plan(rows::kQuantWide, cfg, rows, cols, vec, &w))) return CREDIT_OK;
   hipStream_t s = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
   quant_chunks_kernel<<<w.grid, kThreads, 0, s>>>(x, w.partials, c, w.chunk, w.parts);
@@ -536,7 +509,7 @@ template <class T>
 int wide_layernorm_bwd(const T* x, const T* dy, const T* gamma, T* dx, int64_t rows, int64_t cols,
                        float eps, bool vec, const credit_cfg* cfg, bool* taken) {
   WidePlan w;
-  const WideRule& rule = std::is_same_v<T, float> ? kLnBwdRule : kLnBwdHalfRule;
+  const rows::WideRule& rule = std::is_same_v<T, float> ? rows::kLnBwdWide : rows::kLnBwdHalfWide;
   if (!(*taken = wide_plan(rule, cfg, rows, cols, vec, &w))) return CREDIT_OK;
   hipStream_t s = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
@@ -564,7 +537,7 @@ int wide_layernorm_fwd(const uint16_t* x, const uint16_t* gamma, const uint16_t*
                        uint16_t* y, float* mean, float* rstd, int64_t rows, int64_t cols,
                        float eps, bool vec, const credit_cfg* cfg, bool* taken) {
   WidePlan w;
-  if (!(*taken = wide_plan(kLnFwdRule, cfg, rows, cols, vec, &w))) return CREDIT_OK;
+  if (!(*taken = wide_plan(rows::kLnFwdWide, cfg, rows, cols, vec, &w))) return CREDIT_OK;
   hipStream_t s = cfg_stream(cfg);
   const int c = static_cast<int>(cols);
   const auto launch = [&](auto odd) {

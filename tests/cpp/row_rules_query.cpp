@@ -29,3 +29,11 @@ extern "C" int row_rules_narrow(int op, int64_t rows, int64_t cols) {
                                &kLnHalfOddNarrow};
   return narrow(*rules[op], rows, cols);
 }
+
+// op: 0 softmax forward, 1 its backward, 2 the logits backward, 3 quantisation,
+// 4 LayerNorm forward, 5 and 6 its backward in fp32 and bf16.
+extern "C" int row_rules_wide(int op, int64_t rows, int64_t cols, int vec) {
+  const WideRule* rules[] = {&kSoftmaxFwdWide, &kSoftmaxBwdWide, &kLogitsWide, &kQuantWide,
+                             &kLnFwdWide,      &kLnBwdWide,      &kLnBwdHalfWide};
+  return wide(*rules[op], rows, cols, vec != 0);
+}

@@ -63,3 +63,20 @@ def test_few_narrow_rows_run_read(rules, op, read, held):
     for shapes, want in ((read, 1), (held, 0)):
         for rows, cols in shapes:
             assert rules.row_rules_narrow(op, ctypes.c_int64(rows), ctypes.c_int64(cols)) == want
+
+
+@pytest.mark.parametrize("op,whole,chunks", [
+    (0, [(8, 16384), (33, 65536), (16, 262144)], [(8, 28672), (16, 131072), (32, 65536)]),
+    (1, [(1, 24580), (8, 24580), (8, 32768), (16, 28672)], [(1, 36864), (16, 131072)]),
+    (2, [(8, 16384), (64, 32768)], [(8, 28672), (16, 131072)]),
+    (3, [(16, 65536), (1, 32768)], [(7, 65544), (16, 131072)]),
+    (4, [(16, 49160), (32, 49160), (32, 57344)], [(1, 65536), (16, 131072)]),
+    (5, [(8, 16384)], [(8, 28672), (32, 65536)]),
+    (6, [(16, 40960), (32, 49152)], [(8, 65536), (32, 57344)])])
+def test_aligned_rows_in_chunks_where_they_gain(rules, op, whole, chunks):
+    """Rows of whole vectors, by which of the two measured sooner."""
+    for shapes, want in ((whole, 0), (chunks, 1)):
+        for rows, cols in shapes:
+            assert rules.row_rules_wide(op, ctypes.c_int64(rows), ctypes.c_int64(cols), 1) == want
+    assert not rules.row_rules_wide(op, ctypes.c_int64(2049), ctypes.c_int64(200003), 0)
+    assert rules.row_rules_wide(op, ctypes.c_int64(1), ctypes.c_int64(200003), 0)

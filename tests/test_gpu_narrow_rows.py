@@ -49,3 +49,9 @@ def test_narrow_layernorm_forward(gpu, rows, cols, shift):
     (24577, 0, torch.bfloat16)])
 def test_layernorm_backward_table_edges(gpu, cols, shift, dtype):
     ragged.test_ragged_layernorm_backward(gpu, 270, cols, shift, dtype)
+
+
+# Softmax: the same of the entry of three vectors a lane.
+@pytest.mark.parametrize("rows,cols", [(900, 2049), (1000, 2051), (2100, 3071), (700, 3073)])
+def test_softmax_table_edges(gpu, rows, cols):
+    ragged.test_ragged_softmax(gpu, rows, cols, 0)

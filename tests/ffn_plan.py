@@ -29,17 +29,17 @@ def gemm_plan(m, n, k, kn):
 
 
 def kernel(plan):
+    """The kernel of a plan and its K slices, for people and assertions."""
     return ("256-tile" if plan.big else "held" if plan.held else f"ring {plan.bm}") + (
         f" split {plan.slices}" if plan.slices > 1 else "")
 
 
-def products(rows, d, f, kn, train=False):
-    """{product: plan} of one call: GEMM1 and GEMM2 (train: also the backward's
-    du, da, dW1 and dW2, whose skew is not used)."""
-    out = {"gemm1": gemm_plan(rows, f, d, kn), "gemm2": gemm_plan(rows, d, f, kn)}
-    if train:
-        out["du"] = gemm_plan(rows, f, d, not kn)
-        out["da"] = gemm_plan(rows, d, f, not kn)
-        # nn.Linear: dW1 [f, d] of a [N, K] B; [in, out]: dW1 [d, f] of a [K, N] one.
-        out["dw1"] = gemm_plan(d, f, rows, True) if kn else gemm_plan(f, d, rows, False)
-    return out
+def products(rows, d, f, kn):
+    """{product: plan} of a training step: the forward's two and the recomputing
+    backward's four."""
+    # nn.Linear: dW1 [f, d] and dW2 [d, f] of [N, K] Bs; [in, out]: the other way
+    # round, of [K, N] ones.
+    dw = (((d, f), (f, d)) if kn else ((f, d), (d, f)))
+    return {"gemm1": gemm_plan(rows, f, d, kn), "gemm2": gemm_plan(rows, d, f, kn),
+            "du": gemm_plan(rows, f, d, not kn), "da": gemm_plan(rows, d, f, not kn),
+            "dw1": gemm_plan(*dw[0], rows, kn), "dw2": gemm_plan(*dw[1], rows, kn)}

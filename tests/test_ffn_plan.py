@@ -42,7 +42,7 @@ def test_backward_workspace_holds_no_copy_of_the_input(lib, rows, d, f):
     """Where no product is split the backward's workspace is its own regions
     (rstd; u, du, h^T, du^T; dout^T, a^T; da): the rounded copy of x that these
     shapes read passes through da, so that no workspace is too small for it."""
-    assert all(p.slices == 1 for p in products(rows, d, f, False, train=True).values())
+    assert all(p.slices == 1 for p in products(rows, d, f, False).values())
     own = [4 * rows] + 4 * [2 * rows * f] + 2 * [2 * rows * d] + [4 * rows * d]
     fixed = 256 + (1 << 20) + (4 << 20)
     assert lib.credit_ffn_bwd_workspace_bytes(rows, d, f) <= fixed + sum(own) + 256 * len(own)

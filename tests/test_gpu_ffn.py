@@ -66,12 +66,12 @@ def test_transpose_is_exact(gpu, shape):
     assert torch.equal(dst.cpu(), src.t().contiguous())
 
 
-# The first four take the 128-tile kernels; the rest run GEMM1 (and where
-# d allows, GEMM2) on the 256-tile direct-to-LDS kernel (M and N multiples
-# of 256, K of 128, tile count a multiple of 8).  (512, 128, 1024) gives it
-# the shortest K (two 64-wide steps), (2048, 384, 256) an odd number of
-# step pairs (six steps), (4096, 256, 4608) GEMM1 288 tiles: more than one
-# workgroup per CU, so a second, partial wave of tiles.
+# All on the 128 x 128 ring tiles, K split in (256, 2048, 2048) and in GEMM2 of
+# (1024, 512, 4096) and (4096, 256, 4608), but GEMM1 of the last: the held
+# kernel, and for [in, out] weights 288 of the 256-tile kernel's tiles (a second,
+# partial wave).  From (512, 1024, 1024) on rows and f are whole 256-tiles, a
+# multiple of 8 of them: rstd scales the fp32 sum, a is not rounded.
+# Shapes by kernel: test_gpu_ffn_kernels.py.
 @pytest.mark.parametrize("rows,d,f", [(128, 128, 128), (128, 256, 384), (256, 128, 512),
                                       (384, 512, 256), (512, 1024, 1024), (256, 2048, 2048),
                                       (1024, 512, 4096), (512, 128, 1024), (2048, 384, 256),
@@ -89,9 +89,8 @@ def test_ffn_in_out_layout_is_bit_identical(gpu, rows, d, f):
     """The [in, out] weight path feeds every MFMA the same operand values in
     the same lanes as the nn.Linear path (its B fragments come from
     transposing LDS reads of [K, N] tiles), so the outputs agree bit for
-    bit; the first three shapes take the 128-tile kernels (B staged through
-    registers), the rest the 256-tile ones, (2048, 384, 256) with GEMM2 on
-    the 128-tile kernel (d = 384)."""
+    bit; on the 128 x 128 ring tiles, GEMM1 of (4096, 256, 4608) on the held
+    and the 256-tile kernel."""
     print(f"ffn in_out rows={rows} d={d} f={f}", flush=True)
     x, w1, w2 = make(rows, d, f, seed=rows + d + f + 1)
     got = run_ffn_in_out(x, w1, w2, gpu)
@@ -106,9 +105,8 @@ def test_ffn_in_out_structured_inputs(gpu, rows, d):
     position (swizzle, transposing-read lane order, stage pitch) moves
     values to the wrong output column.  Each output carries one a value
     straight through GELU, so the oracle follows the kernel's arithmetic
-    for a: rounded to bf16 on the 128-tile path (rows 128), unrounded on the
-    256-tile path (rows 2048, both GEMMs), where the fp32 sum is scaled by
-    rstd."""
+    for a: rounded to bf16 at rows 128, unrounded at rows 2048 (whole
+    256-tiles), where the fp32 sum is scaled by rstd."""
     g = torch.Generator().manual_seed(5)
     p = torch.randperm(d, generator=g)
     q = torch.randperm(d, generator=g)
@@ -126,8 +124,8 @@ def test_ffn_in_out_structured_inputs(gpu, rows, d):
 def test_ffn_structured_inputs_pin_layout(gpu, rows, d):
     """Identity-like weights make each output element depend on one input
     element, so any transposed or shifted fragment mapping (or a wrong LDS
-    swizzle / direct-to-LDS lane placement) fails.  (2048, 256) takes the
-    256-tile kernels."""
+    swizzle / direct-to-LDS lane placement) fails.  Both on the ring tiles, a
+    rounded at rows 128 and not at 2048."""
     f = d
     x = (torch.arange(rows * d, dtype=torch.float32).reshape(rows, d) % 7 - 3).to(torch.bfloat16)
     w1 = torch.eye(d, dtype=torch.bfloat16) * 2
@@ -142,8 +140,8 @@ def test_ffn_gelu_negative_tail(gpu, rows):
     sigmoid and 1 - r would cancel: x = 1 (a = x rstd = 1), W1 = -diag(c)
     with c from 3 to 9 (h = GELU(-c) from -4e-3 down to -1e-28) and W2 =
     diag(2 / |GELU(-c)|), so out = 1 + h * 2 / |h| = -1 where h keeps its
-    relative accuracy and 1 where it was flushed to zero.  rows 128 takes the
-    128-tile kernels, 2048 the 256-tile ones."""
+    relative accuracy and 1 where it was flushed to zero.  a is rounded at
+    rows 128 and not at 2048."""
     d = 256
     c = np.linspace(3.0, 9.0, d)
     w1 = torch.from_numpy(-np.diag(c)).to(torch.bfloat16)

@@ -7,11 +7,11 @@ Tolerance: bf16 outputs within rtol 1e-2 of each element plus 1e-2 of the
 tensor's largest magnitude (dW entries are sums over the rows and span a wide
 range; a flat atol of 1e-2 would not scale with them).  A wrong operand
 layout or transpose scrambles every output by O(1) of that scale.  Shapes
-cover the 128-tile GEMMs, the 256-tile GEMMs and mixtures of both; at the
-full C5 shape sampled rows of dx and sampled columns of dW1 / dW2 are checked
-(each depends only on its own rows / columns of the intermediates), and every
-element against a float32 restatement on the GPU (torch_fp32_backward), itself
-held to float64 on sampled rows and columns."""
+cover the ring tiles with and without a K split (the other kernels:
+test_gpu_ffn_kernels.py); at the full C5 shape sampled rows of dx and sampled
+columns of dW1 / dW2 are checked (each depends only on its own rows / columns of
+the intermediates), and every element against a float32 restatement on the GPU
+(torch_fp32_backward), itself held to float64 on sampled rows and columns."""
 import ctypes
 
 import numpy as np
@@ -63,9 +63,8 @@ def oracle(x, w1, w2, dout):
                                          w2.float().numpy(), dout.float().numpy(), EPS)
 
 
-# (128, 128, 128) .. (384, 512, 256): 128-tile GEMMs throughout;
-# (512, 512, 1024): the f-wide GEMMs on 256 tiles, da on 128 tiles;
-# (1024, 512, 2048): every GEMM on 256 tiles; (128, 12288, 256) and
+# Every GEMM on the 128 x 128 ring tiles, u and da of some with K split; from
+# (512, 512, 1024) on rstd scales the fp32 sums of u; (128, 12288, 256) and
 # (128, 20480, 128): rows wider than C5's for the dx row kernel.
 @pytest.mark.parametrize("rows,d,f", [(128, 128, 128), (128, 256, 384), (256, 128, 512),
                                       (384, 512, 256), (512, 512, 1024), (1024, 512, 2048),

@@ -26,12 +26,11 @@ import collections
 import csv
 import hashlib
 import json
+import re
 import subprocess
 from pathlib import Path
 
 CSRC = Path(__file__).resolve().parent / "csrc"
-# Headers every kernel source includes: a change there can change any kernel.
-SHARED_SOURCES = ("common.hpp", "api_internal.hpp", "slices.hpp")
 
 
 def source_fingerprints(csrc: Path = CSRC) -> dict[str, str]:
@@ -43,12 +42,23 @@ def source_fingerprints(csrc: Path = CSRC) -> dict[str, str]:
     return out
 
 
+def built_from(source: str, csrc: Path = CSRC) -> set[str]:
+    """`source` and the headers of its folder that it includes, directly or not."""
+    names, todo = set(), [source]
+    while todo:
+        name = todo.pop()
+        if name not in names and (csrc / name).is_file():
+            names.add(name)
+            todo += re.findall(r'^\s*#include "([^"/]+)"', (csrc / name).read_text(), re.M)
+    return names
+
+
 def sources_unchanged(stamped: dict[str, str], source: str, csrc: Path = CSRC) -> bool:
-    """True when `source` and the shared headers hash as they did when the
-    counters were collected (`stamped` = the summary's "sources")."""
+    """True when `source` and every header it is built from hash as they did
+    when the counters were collected (`stamped` = the summary's "sources")."""
     now = source_fingerprints(csrc)
     return all(name in stamped and stamped[name] == now.get(name)
-               for name in (source, *SHARED_SOURCES))
+               for name in built_from(source, csrc) | {source})
 
 
 def current_commit() -> str | None:

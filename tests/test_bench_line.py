@@ -15,7 +15,7 @@ sys.path.insert(0, str(ROOT))
 
 import bench  # noqa: E402
 from credit_amd import hip_lib  # noqa: E402
-from credit_amd.traffic import source_fingerprints  # noqa: E402
+from credit_amd.traffic import source_fingerprints, sources_unchanged  # noqa: E402
 
 C1_C5 = ("row_sum_max", "layernorm_fwd", "rmsnorm_fwd", "rmsnorm_bwd", "rmsnorm_fwd_bwd",
          "softmax_fwd", "softmax_bwd", "ffn")
@@ -113,3 +113,17 @@ def test_call_kernels_name_the_group_pipelines_auto_launches(name):
     assert group, kernels
     for k in group:
         assert "{" + k + "," in text or "fn = " + k + ";" in text, f"{k} is not in {source}"
+
+
+@pytest.mark.parametrize("source,header", [
+    ("softmax.hip", "rows.hpp"), ("quant.hip", "quant_codes.hpp"), ("lnbwd.hip", "row_rules.hpp"),
+    ("rmsnorm.hip", "split_plan.hpp"), ("ffn.hip", "ffn_plan.hpp")])
+def test_traffic_is_stale_when_a_header_of_the_source_changed(source, header):
+    """Headers that the source includes, also through another one."""
+    now = source_fingerprints()
+    assert sources_unchanged(now, source)
+    for value in ("0" * 16, None):
+        stamped = {k: v for k, v in now.items() if k != header}
+        if value is not None:
+            stamped[header] = value
+        assert not sources_unchanged(stamped, source)

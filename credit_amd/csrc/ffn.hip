@@ -941,9 +941,9 @@ __global__ __launch_bounds__(256) void ffn_gemm_tile_kernel(
 
 // ------------------------------------------- 128 x 128 tiles, many to a CU --
 // More 128-tiles than CUs, unsplit, B [N, K]: one LDS buffer of 36 KiB and the
-// next K-step in registers, so that three workgroups share a CU and cover each
-// other's barriers and epilogues, where the ring of ffn_gemm_tile_kernel lets
-// two: 600 tiles of 28 K-steps 55 us against 67 there, 624 of 24 46 against
+// next K-step in registers, so that three workgroups share a CU (152 to 165
+// registers; kEpiResidual's 175 let two) and cover each other's barriers and
+// epilogues, where the ring of ffn_gemm_tile_kernel lets two: 600 tiles of 28 K-steps 55 us against 67 there, 624 of 24 46 against
 // 60, 275 of 66 67 against 84, 621 of 18 35 against 48, 1125 of 50 158 against
 // 166, 847 of 46 118 against 120 (688 TFLOP/s).  Bound by the LDS reads of 64 x 64 a wave
 // and the two barriers of a step.  The same MFMAs in the same order as the

@@ -368,14 +368,18 @@ int credit_pearson_bwd_f32(const float* x, const float* y, const float* grad, fl
 /* ------------------------------------------ C5: norm-fused FFN ----------
  * out = bf16(x + h @ W2^T), h = bf16(GELU_tanh(rstd * (x @ W1^T))) with
  * rstd = 1/sqrt(mean_j x^2 + eps) per row (RMSNorm with unit weight), fp32
- * accumulation on bf16 MFMA.  (Shapes that are not whole 256 x 256
- * tiles, a multiple of 8 of them -- d or f not a multiple of 256, few rows -- form h = bf16(GELU_tanh(bf16(x * rstd) @
- * W1^T)): the normalised input rounded to bf16 before the product.)  Weights in the nn.Linear layout:
- * w1 [f, d] and w2 [d, f] (K contiguous).  x, out [rows, d].  rows, d and
- * f must be multiples of 128; buffers 16-byte aligned.  The hidden
- * activation h [rows, f] lives in the workspace (query with
- * credit_workspace_bytes(CREDIT_OP_FFN, rows, f, ...)).  No FFN exists in
- * the reference. */
+ * accumulation on bf16 MFMA.  (Unless rows x f is whole 256 x 256 tiles, a
+ * multiple of 8 of them, h = bf16(GELU_tanh(bf16(x * rstd) @ W1^T)): the
+ * normalised input is rounded to bf16 before the product, and waits in out
+ * until the call writes its result there.)  Weights in the nn.Linear layout:
+ * w1 [f, d] and w2 [d, f] (K contiguous).  x, out [rows, d].
+ * rows, d and f must be multiples of 128; buffers 16-byte aligned.  The hidden
+ * activation h [rows, f] lives in the workspace, which needs 5 MiB + 256 bytes
+ * + 4 rows + 2 rows f bytes (both terms rounded up to 256);
+ * credit_workspace_bytes(CREDIT_OP_FFN, rows, f, ...) names 64 MiB more, for
+ * the partial sums of products that run in several K slices (fewer bytes: the
+ * same slices one after another, the same outputs).  No FFN exists in the
+ * reference. */
 int credit_ffn_rmsnorm_gelu_bf16(const uint16_t* x, const uint16_t* w1, const uint16_t* w2,
                                  uint16_t* out, int64_t rows, int64_t d, int64_t f, float eps,
                                  const credit_cfg* cfg);
@@ -394,8 +398,11 @@ int credit_ffn_rmsnorm_gelu_kn_bf16(const uint16_t* x, const uint16_t* w1, const
  * [rows] fp32, u [rows, f] = bf16(rstd * (x @ W1^T)) and h [rows, f] =
  * bf16(GELU_tanh(rstd * (x @ W1^T))), both bf16 row-major (h is the hidden
  * activation GEMM2 reads).  out is bit-identical to
- * credit_ffn_rmsnorm_gelu_bf16.  No workspace.  Same shape and alignment
- * rules (u and h 16-byte aligned too).  No counterpart in the reference. */
+ * credit_ffn_rmsnorm_gelu_bf16.  Takes no workspace; on each of the first 16
+ * (device, stream) pairs that call it the library keeps 64 MiB for partial
+ * sums, except under capture and on hipStreamPerThread, where it runs without
+ * them (the same outputs).  Same shape and alignment rules (u and h 16-byte
+ * aligned too).  No counterpart in the reference. */
 int credit_ffn_rmsnorm_gelu_fwd_train_bf16(const uint16_t* x, const uint16_t* w1,
                                            const uint16_t* w2, uint16_t* out, float* rstd,
                                            uint16_t* u, uint16_t* h, int64_t rows, int64_t d,

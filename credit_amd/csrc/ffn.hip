@@ -695,13 +695,16 @@ __device__ __forceinline__ void store_quad(const f32x16& acc, int q, const float
 //    steps behind it in flight), then an LDS-only barrier, after which stage
 //    it % ST is free: step it+ST's loads go there, a quarter of them in each
 //    of that sub-step and the next iteration's first three (two stages: all in
-//    that sub-step).  Tail steps
-//    re-load the last K-step into stages nobody reads again.
+//    that sub-step).  Steps behind a slice's end are the next slice's first;
+//    behind the last slice they re-load its last step into stages nobody reads
+//    again.
 //  - With few tiles a CU would sit idle or run one long K chain (128 rows x
 //    8192 x 28672: 64 tiles on 256 CUs), so gemm_plan cuts K until the units
 //    (tiles x slices) fill the chip.  kEpiPartial launches one workgroup per
 //    unit, which stores its sums to Cf[slice] for ffn_reduce_kernel; every
-//    other EPI covers all slices of its tile in order with the same additions,
+//    other EPI covers all slices of its tile in order with the same additions
+//    (the loads run on from one slice to the next: 384 x 384 x 7808, 13 slices
+//    without scratch, 108 us for the FFN with a prologue each, 95 without),
 //    so both forms give the same bits.
 //  - B loads carry the nontemporal hint, which leaves the L2 to the A rows
 //    that every workgroup of an XCD reads (128 rows x 8192 x 28672: 206 ->
@@ -754,10 +757,21 @@ __global__ __launch_bounds__(256) void ffn_gemm_tile_kernel(
   const int m0 = (group * kGroupM + within % gm) * BM;
   const int n0 = within / gm * kTileN;
   const int steps = K / kBigK;
-  auto slice_begin = [&](int s) { return s * steps / slices; };
   const int s0 = EPI == kEpiPartial ? slice : 0;
   const int s1 = EPI == kEpiPartial ? slice + 1 : slices;
-  int first = 0, steps_here = 0, turn = 0;  // the slice being summed: its steps and first load
+  struct Slice {
+    int first, steps, turn;  // K-steps, and the first of them to load
+  };
+  auto slice_at = [&](int s) {
+    Slice r;
+    r.first = s * steps / slices;
+    r.steps = (s + 1) * steps / slices - r.first;
+    r.turn = static_cast<int>(static_cast<uint32_t>(skew * (n0 / kTileN)) %
+                              static_cast<uint32_t>(r.steps));
+    return r;
+  };
+  Slice here = slice_at(s0), then = here;  // the slice being summed, and the one behind it
+  bool more = false;                       // there is one behind it
 
   const buffer_rsrc_t rsrc_a =
       make_rsrc(A + static_cast<size_t>(m0) * K, static_cast<uint32_t>(BM) * K * 2u);
@@ -772,15 +786,19 @@ __global__ __launch_bounds__(256) void ffn_gemm_tile_kernel(
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
   const uint32_t m0_wave = static_cast<uint32_t>(
       __builtin_amdgcn_readfirstlane(static_cast<int>(lds0 + wave * 1024)));
-  // Load q of the slice's k-th K-step into `stage`: A rows 8 (4 q + w) .. + 7 (q < AL), else B
-  // rows likewise (KN: K-rows 16 (q - AL) + 4 w .. + 3).
+  // Load q of the slice's k-th K-step, or past its end the next slice's, into
+  // `stage`: A rows 8 (4 q + w) .. + 7 (q < AL), else B rows likewise (KN: K-rows
+  // 16 (q - AL) + 4 w .. + 3).
   auto load = [&](int k, int stage, auto qc) {
     constexpr int q = decltype(qc)::value;
     constexpr int qb = q < AL ? q : q - AL;
     constexpr uint32_t qoff = static_cast<uint32_t>(qb * 4096 + (q < AL ? 0 : kBOff));
-    int kk = (k < steps_here ? k : steps_here - 1) + turn;  // tail: a re-load
-    if (kk >= steps_here) kk -= steps_here;
-    const uint32_t kc = static_cast<uint32_t>(first + kk);
+    const bool behind = EPI != kEpiPartial && more && k >= here.steps;
+    const int n = behind ? then.steps : here.steps;
+    int kk = behind ? k - here.steps + then.turn
+                    : (k < n ? k : n - 1) + here.turn;  // tail: a re-load
+    if (kk >= n) kk -= n;
+    const uint32_t kc = static_cast<uint32_t>((behind ? then.first : here.first) + kk);
     const uint32_t soff =
         KN && q >= AL ? (kc * kBigK + qb * 16) * static_cast<uint32_t>(N) * 2u
                       : kc * (kBigK * 2) + static_cast<uint32_t>(qb * 64) * static_cast<uint32_t>(K);
@@ -866,28 +884,26 @@ __global__ __launch_bounds__(256) void ffn_gemm_tile_kernel(
   };
   static_assert(NF <= 2 * MI, "a sub-step's reads fit its regions");
 
-  for (int s = s0; s < s1; ++s) {
-    first = slice_begin(s);
-    steps_here = slice_begin(s + 1) - first;
-    turn = static_cast<int>(static_cast<uint32_t>(skew * (n0 / kTileN)) %
-                            static_cast<uint32_t>(steps_here));
-    // Prologue: the first ST - 1 steps whole and the next one's L3 loads; the
-    // first step landed before its fragments are read.
+  // Prologue: the first ST - 1 steps whole and the next one's L3 loads; the
+  // first step landed before its fragments are read.
 #pragma unroll
-    for (int k = 0; k < ST - 1; ++k)
-      [&]<int... Qs>(std::integer_sequence<int, Qs...>) {
-        (load(k, k, std::integral_constant<int, Qs>{}), ...);
-      }(std::make_integer_sequence<int, L>{});
+  for (int k = 0; k < ST - 1; ++k)
     [&]<int... Qs>(std::integer_sequence<int, Qs...>) {
-      (load(ST - 1, ST - 1, std::integral_constant<int, Qs>{}), ...);
-    }(std::make_integer_sequence<int, L3>{});
-    wait_vmcnt<(ST - 2) * L + L3>();
-    lds_barrier();
-    Frags f0, f1;
+      (load(k, k, std::integral_constant<int, Qs>{}), ...);
+    }(std::make_integer_sequence<int, L>{});
+  [&]<int... Qs>(std::integer_sequence<int, Qs...>) {
+    (load(ST - 1, ST - 1, std::integral_constant<int, Qs>{}), ...);
+  }(std::make_integer_sequence<int, L3>{});
+  wait_vmcnt<(ST - 2) * L + L3>();
+  lds_barrier();
+  Frags f0, f1;
 #pragma unroll
-    for (int m = 0; m < NF; ++m) f0.v[m] = frag(0, 0, m);
-    int cur = 0, prev = ST - 1;  // cur = stage of step it, prev of it - 1 and it + ST - 1
-    for (int it = 0; it < steps_here; ++it) {
+  for (int m = 0; m < NF; ++m) f0.v[m] = frag(0, 0, m);
+  int cur = 0, prev = ST - 1;  // cur = stage of step it, prev of it - 1 and it + ST - 1
+  for (int s = s0; s < s1; ++s) {
+    more = EPI != kEpiPartial && s + 1 < s1;
+    if (more) then = slice_at(s + 1);  // at least 8 steps (gemm_slices), more than the ring holds
+    for (int it = 0; it < here.steps; ++it) {
       const int next = cur + 1 == ST ? 0 : cur + 1;
       sub_step.template operator()<L3, LQ>(f0, f1, cur, 1, it + ST - 1, prev);
       sub_step.template operator()<L3 + LQ, LQ>(f1, f0, cur, 2, it + ST - 1, prev);
@@ -898,7 +914,7 @@ __global__ __launch_bounds__(256) void ffn_gemm_tile_kernel(
       prev = cur;
       cur = next;
     }
-    wait_vmcnt<0>();  // the tail re-loads
+    here = then;
     if constexpr (EPI != kEpiPartial) {
 #pragma unroll
       for (int i = 0; i < MI; ++i)
@@ -909,9 +925,9 @@ __global__ __launch_bounds__(256) void ffn_gemm_tile_kernel(
             total[i][j][r] = s == s0 ? acc[i][j][r] : total[i][j][r] + acc[i][j][r];
             acc[i][j][r] = 0.0f;
           }
-      if (s + 1 < s1) lds_barrier();  // every wave has read its last fragments
     }
   }
+  wait_vmcnt<0>();  // the tail re-loads
 
   // Epilogue.  Registers 4q .. 4q + 3 of tile (i, j) are rows mb .. mb + 3 of
   // column n.

@@ -1287,8 +1287,10 @@ int launch_gemm(const uint16_t* A, const float* scale, const uint16_t* B, const 
   }
   if constexpr (!KN) {
     if (plan.held) {
-      ffn_gemm_held_kernel<EPI><<<dim3(static_cast<unsigned>((M / kTileN) * (N / kTileN))),
-                                  dim3(256), 0, stream>>>(A, scale, B, R, C, C2, Cf, M, N, K);
+      const int64_t tiles = int64_t{M / kTileN} * (N / kTileN);
+      ffn_gemm_held_kernel<EPI><<<dim3(static_cast<unsigned>(tiles)), dim3(256),
+                                  held_extra_lds(tiles, K / kBigK), stream>>>(
+          A, scale, B, R, C, C2, Cf, M, N, K);
       return check_launch(name);
     }
   }

@@ -63,6 +63,16 @@ inline double big_us(int64_t units, int64_t steps) {
 inline double held_us(int64_t units, int64_t steps) {
   return (units + kGemmCus - 1) / kGemmCus * (steps * 0.6) + 6.0;
 }
+// LDS that a launch of the held kernel asks for beside its own 36 KiB, to keep a
+// third workgroup off each CU: 769 to 1024 tiles are two rounds of three to a
+// CU, the second nearly empty, and two even rounds of two (962 tiles of 84 steps
+// 247 us at three, 215 at two).  Not where the third workgroup's cover of short
+// K loops is worth more, nor where rounds come out otherwise (the FFN with GEMM1
+// of 825 tiles of 56 steps 306 and 296, 918 of 36 217.5 and 216, 840 of 12 78.6
+// and 80.9; 736 of 16 76 and 80; 1650 of 28 249 and 253).
+inline int held_extra_lds(int64_t tiles, int64_t steps) {
+  return tiles > 3 * kGemmCus && tiles <= 4 * kGemmCus && steps >= 32 ? 24 << 10 : 0;
+}
 constexpr int64_t kSlabBytes = int64_t{64} << 20;  // most fp32 partial sums of one product
 
 // Whether the held kernel can run an unsplit product of a [N, K] B, whichever

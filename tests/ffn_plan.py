@@ -7,7 +7,7 @@ import tempfile
 from collections import namedtuple
 from pathlib import Path
 
-Plan = namedtuple("Plan", "big bm slices skew held")
+Plan = namedtuple("Plan", "big bm slices skew held extra_lds")
 
 
 @functools.cache
@@ -22,10 +22,10 @@ def _library():
 
 def gemm_plan(m, n, k, kn):
     """How C[m, n] over k runs with a [n, k] B (kn: [k, n])."""
-    out = (ctypes.c_int64 * 5)()
+    out = (ctypes.c_int64 * 6)()
     _library().ffn_plan_query(ctypes.c_int64(m), ctypes.c_int64(n), ctypes.c_int64(k), int(kn),
                               out)
-    return Plan(bool(out[0]), out[1], out[2], out[3], bool(out[4]))
+    return Plan(bool(out[0]), out[1], out[2], out[3], bool(out[4]), out[5])
 
 
 def kernel(plan):

@@ -37,6 +37,17 @@ def test_an_unsplit_product_is_priced_on_the_kernel_that_runs_it(m, n, k):
     assert gemm_plan(m, n, k, True).slices == 1
 
 
+@pytest.mark.parametrize("m,n,k,two", [(4736, 3328, 5376, True), (2176, 6912, 2304, True),
+                                       (4096, 2944, 1024, False), (2816, 9600, 1792, False), (1024, 13440, 768, False),
+                                       (4224, 8576, 2176, False)])
+def test_held_workgroups_to_a_cu(m, n, k, two):
+    """Two to a CU where the third would leave a round nearly empty."""
+    plan = gemm_plan(m, n, k, False)
+    assert plan.held
+    lds = 36864 + plan.extra_lds
+    assert lds <= 65536 and ((160 << 10) // lds == 2) == two
+
+
 @pytest.mark.parametrize("rows,d,f", [(2176, 2304, 6912), (4224, 2176, 8576)])
 def test_backward_workspace_holds_no_copy_of_the_input(lib, rows, d, f):
     """Where no product is split the backward's workspace is its own regions

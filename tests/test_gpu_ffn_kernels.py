@@ -110,6 +110,14 @@ def test_tall_tiles_split(gpu):
     check(gpu, *shape, sample=np.array([0, 1, 127, 128, 255, 256, 400, 511, 512, 700, 766, 767]))
 
 
+def test_held_two_to_a_cu(gpu):
+    """810 tiles of 32 steps: launched with LDS that keeps the third workgroup off."""
+    shape = (1152, 2048, 11520)
+    assert_kernels(shape, {"gemm1": ("held", "ring 128"), "du": ("ring 128", "held")})
+    assert products(*shape, False)["gemm1"].extra_lds > 0
+    check(gpu, *shape, sample=np.array([0, 1, 127, 128, 255, 500, 1023, 1024, 1151]))
+
+
 def test_one_tall_tile_of_rows_is_skewed():
     for kn in (False, True):
         plan = products(256, 512, 20480, kn)["gemm1"]

@@ -70,10 +70,10 @@ inline bool narrow(const NarrowRule& rule, int64_t rows, int64_t cols) {
 // 76 us, 49).
 //
 // Rows of whole vectors have faster kernels, SPLIT among them: at most 32 rows,
-// wide ones and little data (64 x 131072: 22, 27).  One workgroup that holds the
-// row is sooner done than two launches: softmax forward and logits backward up
-// to 24576 columns (8 x 24584: 7.5 and 7.8 us, 6.1 and 6.2 in chunks; 32 x 24584
-// 7.9 and 8.3, 7.4 and 8.8), softmax backward up to 32768 (8 x 24584: 4.9, 6.0;
+// wide ones and little data (softmax logits backward 64 x 131072: 22 us, 27 in
+// chunks).  One workgroup that holds the row is sooner done than two launches:
+// softmax forward and logits backward up to 24576 columns (8 x 24584: 7.5 and
+// 7.8 us, 6.1 and 6.2 in chunks), softmax backward up to 32768 (8 x 24584: 4.9, 6.0;
 // 8 x 36864, SPLIT: 8.1, 6.0), quantisation up to 65536 (16 x 65536: 6.4, 7.0;
 // 16 x 65544, SPLIT: 7.8, 5.9), LayerNorm forward up to 57344 (24 x 49160: 6.6,
 // 7.2; 16 x 65536: 7.2, 7.1), its bf16 backward up to 49152.  16 x 262144 would

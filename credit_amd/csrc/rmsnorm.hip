@@ -300,15 +300,19 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_slice_kernel(
 // teams it has.  Bound by HBM: at 4096 x 8192 the 512-lane workgroups before
 // it, two to a CU with the accumulators in LDS, left 512 partial rows
 // (33.5 MB) and ran 54.5 us, the partial reduction behind them 26 us.
+// ONE: a row to a workgroup (at most one per CU), so a workgroup of one team,
+// whose accumulators are the partial row: what 1024 lanes and their LDS take to
+// start and add is most of such a call (8 x 512 with the reduction: 5.9 us on
+// 1024 lanes, 4.3 on one team; 256 x 8192 27, 16.5).
 constexpr int kRowsThreads = 1024;
 constexpr size_t kRowsLds = size_t{kRowsThreads} * 8 * sizeof(double);  // 64 KiB
 
-template <int TEAM>
-__global__ __launch_bounds__(kRowsThreads) void rmsnorm_bwd_rows_kernel(
+template <int TEAM, bool ONE>
+__global__ __launch_bounds__(ONE ? TEAM : kRowsThreads) void rmsnorm_bwd_rows_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
     const uint16_t* __restrict__ dy, const float* __restrict__ rstd, uint16_t* __restrict__ dx,
     double* __restrict__ dw_part, int rows, int cols, int rows_per_group) {
-  constexpr int T = kRowsThreads / TEAM;  // teams
+  constexpr int T = ONE ? 1 : kRowsThreads / TEAM;  // teams
   constexpr int NW = TEAM / kWave;        // waves per team
   extern __shared__ double dw_lds[];      // [team][8 TEAM]
   __shared__ double red[2][T][NW];
@@ -371,6 +375,15 @@ __global__ __launch_bounds__(kRowsThreads) void rmsnorm_bwd_rows_kernel(
     step(c, b, base + team + 2 * T, 0);
     if (base + 3 * T >= r1) break;
     step(d, c, base + team + 3 * T, 1);
+  }
+  if constexpr (ONE) {
+    f64x2* mine = reinterpret_cast<f64x2*>(dw_part + static_cast<size_t>(blockIdx.x) * cols +
+                                           8 * lane);
+    if (8 * lane < cols) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mine[e] = f64x2{acc[2 * e], acc[2 * e + 1]};
+    }
+    return;
   }
   double* mine = dw_lds + 8 * (team * TEAM + lane);
 #pragma unroll
@@ -966,13 +979,15 @@ const BwdPick kBwd[] = {
 using BwdRowsFn = void (*)(const uint16_t*, const uint16_t*, const uint16_t*, const float*,
                            uint16_t*, double*, int, int, int);
 struct BwdRowsPick {
-  BwdRowsFn fn;
-  int capacity;
+  BwdRowsFn fn, one;
+  int capacity;  // vectors, and lanes of a team
 };
 const BwdRowsPick kBwdRows[] = {
-    {rmsnorm_bwd_rows_kernel<64>, 64},   {rmsnorm_bwd_rows_kernel<128>, 128},
-    {rmsnorm_bwd_rows_kernel<256>, 256}, {rmsnorm_bwd_rows_kernel<512>, 512},
-    {rmsnorm_bwd_rows_kernel<1024>, 1024},
+    {rmsnorm_bwd_rows_kernel<64, false>, rmsnorm_bwd_rows_kernel<64, true>, 64},
+    {rmsnorm_bwd_rows_kernel<128, false>, rmsnorm_bwd_rows_kernel<128, true>, 128},
+    {rmsnorm_bwd_rows_kernel<256, false>, rmsnorm_bwd_rows_kernel<256, true>, 256},
+    {rmsnorm_bwd_rows_kernel<512, false>, rmsnorm_bwd_rows_kernel<512, true>, 512},
+    {rmsnorm_bwd_rows_kernel<1024, false>, rmsnorm_bwd_rows_kernel<1024, true>, 1024},
 };
 // Group kernels: four row buffers per lane.  At one dwordx4 per lane
 // (~104 VGPRs: 4 waves per SIMD, 16 per CU; 64 bytes of LDS dw
@@ -1522,9 +1537,11 @@ extern "C" int credit_rmsnorm_bwd_bf16(const uint16_t* x, const uint16_t* w,
     }();
     if (attr != hipSuccess)
       return hip_failure(attr, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
-    hipLaunchKernelGGL(pick_for(kBwdRows, plan.chunk)->fn, dim3(total), dim3(kRowsThreads),
-                       kRowsLds, stream, x, w, dy, rstd, dx, dw_part, static_cast<int>(rows), c,
-                       plan.rows_per_group);
+    const BwdRowsPick* pick = pick_for(kBwdRows, plan.chunk);
+    const bool one = plan.rows_per_group == 1;
+    hipLaunchKernelGGL(one ? pick->one : pick->fn, dim3(total),
+                       dim3(one ? pick->capacity : kRowsThreads), one ? 0 : kRowsLds, stream, x, w,
+                       dy, rstd, dx, dw_part, static_cast<int>(rows), c, plan.rows_per_group);
     CREDIT_TRY(check_launch("rmsnorm_bwd_rows_kernel"));
   } else {
     const BwdPick* pick = pick_for(kBwd, plan.chunk);

@@ -27,7 +27,8 @@ def backward(x, w, dy, rstd, gpu):
 # cols: both edges of each team width; rows: one, one per CU and one more,
 # blocks shorter and longer than the row buffers of 1 to 16 teams.
 @pytest.mark.parametrize("rows,cols", [
-    (1, 8), (1, 8192), (256, 512), (257, 520), (513, 1024), (1025, 1032), (2300, 2048),
+    (1, 8), (1, 8192), (256, 512), (257, 520), (7, 520), (40, 1024), (200, 1032), (9, 2056),
+    (33, 4096), (5, 4104), (255, 8192), (513, 1024), (1025, 1032), (2300, 2048),
     (1300, 2056), (771, 4096), (3000, 4104), (1281, 8192), (9000, 256)])
 def test_staged_backward(gpu, rows, cols):
     print(f"rmsnorm_bwd rows {rows} x {cols}", flush=True)

@@ -920,7 +920,29 @@ __global__ __launch_bounds__(256) void rmsnorm_dw_reduce_kernel(
   reinterpret_cast<float2_t*>(dw)[q] = float2_t{static_cast<float>(a.x), static_cast<float>(a.y)};
 }
 
+// The same sums, in the same order, of at most 16 blocks: each lane adds its
+// column pair's, with no barrier to meet (the fused pass at 1 x 12288: 10.5 ->
+// 10.0 us).
+constexpr int kFewBlocks = 16;
+__global__ __launch_bounds__(256) void rmsnorm_dw_few_kernel(const double* __restrict__ part,
+                                                             float* __restrict__ dw, int blocks,
+                                                             int cols) {
+  const int q = blockIdx.x * 256 + threadIdx.x;  // column pair
+  const int nq = cols >> 1;
+  if (q >= nq) return;
+  const f64x2* p = reinterpret_cast<const f64x2*>(part) + q;
+  f64x2 a{0.0, 0.0};
+#pragma unroll 8
+  for (int b = 0; b < blocks; ++b) a += load_nt(p + static_cast<size_t>(b) * nq);
+  reinterpret_cast<float2_t*>(dw)[q] = float2_t{static_cast<float>(a.x), static_cast<float>(a.y)};
+}
+
 int launch_dw_reduce(const double* part, float* dw, int64_t blocks, int cols, hipStream_t stream) {
+  if (blocks <= kFewBlocks) {
+    rmsnorm_dw_few_kernel<<<dim3(static_cast<unsigned>((cols / 2 + 255) / 256)), dim3(256), 0,
+                            stream>>>(part, dw, static_cast<int>(blocks), cols);
+    return check_launch("rmsnorm_dw_few_kernel");
+  }
   rmsnorm_dw_reduce_kernel<<<dim3(static_cast<unsigned>((cols / 2 + 15) / 16)), dim3(256), 0,
                              stream>>>(part, dw, static_cast<int>(blocks), cols);
   return check_launch("rmsnorm_dw_reduce_kernel");

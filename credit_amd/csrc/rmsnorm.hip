@@ -920,10 +920,10 @@ __global__ __launch_bounds__(256) void rmsnorm_dw_reduce_kernel(
   reinterpret_cast<float2_t*>(dw)[q] = float2_t{static_cast<float>(a.x), static_cast<float>(a.y)};
 }
 
-// The same sums, in the same order, of at most 16 blocks: each lane adds its
-// column pair's, with no barrier to meet (the fused pass at 1 x 12288: 10.5 ->
-// 10.0 us).
-constexpr int kFewBlocks = 16;
+// The same sums, in the same order, of at most 8 blocks, the loads of one batch:
+// each lane adds its column pair's, with no barrier to meet (the fused pass at 1
+// x 12288: 10.5 -> 10.2 us).
+constexpr int kFewBlocks = 8;
 __global__ __launch_bounds__(256) void rmsnorm_dw_few_kernel(const double* __restrict__ part,
                                                              float* __restrict__ dw, int blocks,
                                                              int cols) {
